@@ -20,6 +20,7 @@
 
 #include "fmm3d_internal.hpp"
 #include "lap_kernels.hip"
+#include "form_mfma.hpp"
 #include "m2l_mfma.hpp"
 #include "hess_kernels.hpp"
 #include "qp_kernels.hpp"
@@ -309,7 +310,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   constexpr bool near32 = sizeof(TN) < sizeof(double);
   double* spos = (double*)ctx.arena.get("spos", sizeof(double) * 4 * (size_t)ns);
   double* str64 = (double*)ctx.arena.get("str64", sizeof(double) * 8 * (size_t)ns);
-  float* str32 = near32 ? (float*)ctx.arena.get("str32", sizeof(float) * 8 * (size_t)ns) : nullptr;
+  float* str32 = near32 || sizeof(T) == 4 ? (float*)ctx.arena.get("str32", sizeof(float) * 8 * (size_t)ns) : nullptr;
   double* tpos = (double*)ctx.arena.get("tpos", sizeof(double) * 4 * (size_t)std::max(nt, 1));
   T* mp = (T*)ctx.arena.get("mp", sizeof(T) * 2 * K * nb, 16);
   T* lo = (T*)ctx.arena.get("lo", sizeof(T) * 2 * K * nb, 16);
@@ -402,45 +403,56 @@ int lap_solve(Context& ctx, const LapCall& c) {
   FMM_HIP(hipEventRecord(ctx.aux_ev[0], s));  // inputs gathered, sums zeroed
   mark(1);
   const double* fac = Tb.fac;
+  // the strengths in the far field's type (FP32 far fields have no triangles)
+  const T* fstrT = sizeof(T) == 4 ? (const T*)(const void*)str32 : (const T*)(const void*)fstr;
   // ---- STEP 1: P2M, STEP 2: P2L (list 4)
-  // k_form2 (per-thread sums) when its half table fits I1 (or 2 I1) entries
-  // per thread, else k_form (per-coefficient contraction)
   auto form = [&](auto irreg_tag, int nbox_form, T* dst) {
     constexpr bool IR = decltype(irreg_tag)::value;
-    constexpr int NT = form2_threads<IR>(), I1 = 512 / NT;
     if (nbox_form == 0 || (!f.ifcharge && !f.ifdipole)) return;
     const int pt = IR ? p + 1 : p;
     const int H = (pt + 1) * (pt + 2) / 2;
-    const size_t P2 = (size_t)(pt + 1) * (pt + 1);
-    const int HS = form2_row_stride<T>(H);
     DevPlan PF = P;  // the current plan (P2L needs list 4), source ranges in points for triangles
     if (tri) {
       PF.isrc = tri_rng;
       PF.nsrc = tri_rng + nb;
     }
-    int ts = (int)(65536 / (2 * sizeof(T) * (size_t)HS));
-    ts = std::max(1, std::min(32, ts));
-    const size_t lds2 = form2_fac_bytes(p) + 2 * sizeof(T) * std::max((size_t)ts * HS, 4 * P2) + (kFormScStride + 8) * sizeof(T) * ts;
-#define FORM2(C, D, I)                                                                                 \
-  if (f.ifcharge == C && f.ifdipole == D)                                                              \
-    hipLaunchKernelGGL((k_form2<T, IR, C, D, I>), dim3(nbox_form), dim3(NT), lds2, s, PF, fac, fpos, fstr, ts, dst);
-    const bool lds2_fits = lds2 <= max_lds_bytes(ctx);
-    if (H <= I1 * NT && lds2_fits) {
-      FORM2(1, 0, I1) FORM2(0, 1, I1) FORM2(1, 1, I1)
-    } else if (H <= 2 * I1 * NT && lds2_fits) {
-      FORM2(1, 0, 2 * I1) FORM2(0, 1, 2 * I1) FORM2(1, 1, 2 * I1)
-    } else {
-#undef FORM2
-      // tile of ts sources: 2K accumulators + ts (2H + 11) table, positions
-      // and strengths, sized in signed arithmetic against the device limit
-      const long avail = (long)(max_lds_bytes(ctx) / sizeof(T)) - 2L * K;
-      const long ts1 = avail / (2L * H + 11);
-      if (ts1 < 1) throw AllocError("P2M/P2L tile does not fit LDS", 16);
-      const int ts = (int)std::min<long>(32, ts1);
-      const size_t lds = sizeof(T) * (2 * (size_t)K + (size_t)ts * (2 * H + 11));
-      hipLaunchKernelGGL((k_form<T, IR>), dim3(nbox_form), dim3(256), lds, s, PF, fac, fpos, fstr,
-                         f.ifcharge, f.ifdipole, ts, dst);
+    const bool dip = f.ifdipole != 0;
+    if constexpr (std::is_same<T, double>::value) {
+      // charges at orders 16 to 42: two or three blocks of columns, their
+      // accumulators within a wave's registers
+      if (!dip && pt >= 16 && pt < 44) {
+        const size_t lds = sizeof(double) * (size_t)form_mfma_lds(pt);
+        const FormWaves W = form_waves(pt);
+        if (pt < 28)
+          hipLaunchKernelGGL((k_form_mfma<IR, 28>), dim3(nbox_form), dim3(64 * kFormMfmaWaves), lds, s, PF, fac, fpos, fstr, W, dst);
+        else
+          hipLaunchKernelGGL((k_form_mfma<IR, 44>), dim3(nbox_form), dim3(64 * kFormMfmaWaves), lds, s, PF, fac, fpos, fstr, W, dst);
+        return;
+      }
     }
+    // entries per thread: two where one would need a third range or, for
+    // dipoles, two overlapping ones (dipoles at order 26: 250,000 Plummer
+    // points P2L 4.8 -> 4.2 ms, 82,000 triangles 6.9 -> 5.8 ms)
+    const int items = H > 256 ? 2 : 1;
+    const FormRanges R = form_ranges(pt, dip, 256 * items);
+    if (R.n == 0) throw AllocError("P2M/P2L: order beyond the ranges of k_form2", 16);
+    int row = 0;
+    for (int r = 0; r < R.n; r++) row = std::max(row, form_row(pt, R.from[r], R.to[r]));
+    const int region = std::max((int)(32768 / sizeof(T)), 4 * row);
+    const size_t lds = sizeof(T) * ((size_t)form_head(pt, row) + region);
+#define FORM2(C, D, GS, I)                                                                                 \
+  if (f.ifcharge == C && f.ifdipole == D)                                                                  \
+    hipLaunchKernelGGL((k_form2<T, IR, C, D, GS, I>), dim3(nbox_form, R.n), dim3(256), lds, s, PF, fac, fpos, fstrT, R, region, dst);
+    if (H <= 64) {
+      FORM2(1, 0, 64, 1) FORM2(0, 1, 64, 1) FORM2(1, 1, 64, 1)
+    } else if (H <= 128) {
+      FORM2(1, 0, 128, 1) FORM2(0, 1, 128, 1) FORM2(1, 1, 128, 1)
+    } else if (items == 1) {
+      FORM2(1, 0, 256, 1) FORM2(0, 1, 256, 1) FORM2(1, 1, 256, 1)
+    } else {
+      FORM2(1, 0, 256, 2) FORM2(0, 1, 256, 2) FORM2(1, 1, 256, 2)
+    }
+#undef FORM2
   };
   form(std::false_type{}, P.n_p2m, mp);
   // quadrupoles: their multipoles (degrees >= 2) and, below, their list-4
@@ -616,13 +628,14 @@ int lap_solve(Context& ctx, const LapCall& c) {
   mark(7);
   // ---- STEP 7: L2P (packed local + gradient expansions, wave-uniform reads)
   if (P.n_l2p) {
-    const size_t H = (size_t)(p + 1) * (p + 2) / 2;
-    T* pack = (T*)ctx.arena.get("l2p_pack", sizeof(T) * 16 * H * (size_t)P.n_l2p);
-    const size_t tot = H * (size_t)P.n_l2p;
+    const size_t E = (size_t)pack_entries(p);
+    // (one entry more than the packs hold: the walk loads one ahead)
+    T* pack = (T*)ctx.arena.get("l2p_pack", sizeof(T) * kPackEntry * (E * (size_t)P.n_l2p + 1));
+    const size_t tot = E * (size_t)P.n_l2p;
     hipLaunchKernelGGL((k_l2p_pack<T>), dim3((unsigned)std::min<size_t>(blocks(tot, 256), 65536)), dim3(256), 0, s,
                        P, fac, lo, pack);
     if (P.n_l2pi)
-      hipLaunchKernelGGL((k_l2p2<T>), dim3(item_groups(P.n_l2pi)), dim3(kP2PBlock * kItemWaves), 0, s, P, fac, pack, spos, tpos, f.ifpot, f.iffld,
+      hipLaunchKernelGGL((k_l2p2<T>), dim3(item_groups(P.n_l2pi)), dim3(kP2PBlock * kItemWaves), 0, s, P, pack, spos, tpos, f.ifpot, f.iffld,
                          f.ifpottarg, f.iffldtarg, pot_s, fld_s, pot_t, fld_t);
   }
   mark(8);
@@ -633,7 +646,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
     const int grad = (f.iffld || f.iffldtarg) ? 1 : 0;
     const bool want_src = f.ifpot || f.iffld, want_trg = f.ifpottarg || f.iffldtarg;
     const int pd = grad ? p + 1 : p;
-    const int Hd = (pd + 1) * (pd + 2) / 2;
+    const int Hd = pack_entries(pd);
     constexpr int kSlice = 1024;
     const int nbx = tree.nboxes;
     thread_local std::vector<int> slot, pk, off, it, red, hv;
@@ -677,13 +690,13 @@ int lap_solve(Context& ctx, const LapCall& c) {
       const size_t o_pk = nbx, o_off = o_pk + pk.size(), o_it = o_off + off.size(), o_red = o_it + it.size();
       for (auto* v : {&slot, &pk, &off, &it, &red}) hv.insert(hv.end(), v->begin(), v->end());
       const int* dh = upload_ints("m2p_i", hv, s);
-      T* pack = (T*)ctx.arena.get("m2p_pack", sizeof(T) * 16 * (size_t)tot);
+      T* pack = (T*)ctx.arena.get("m2p_pack", sizeof(T) * kPackEntry * ((size_t)tot + 1));
       const size_t nit = it.size() / 5;
       double* partial = (double*)ctx.arena.get("m2p_part", sizeof(double) * 8 * 64 * nit);
       const size_t tp = (size_t)pk.size() * Hd;
       hipLaunchKernelGGL((k_m2p_pack<T>), dim3((unsigned)std::min<size_t>(blocks(tp, 256), 65536)), dim3(256), 0, s,
                          P, fac, mp, dh + o_pk, dh + o_off, (int)pk.size(), grad, pack);
-      hipLaunchKernelGGL((k_m2p_eval<T>), dim3(item_groups((int)nit)), dim3(kP2PBlock * kItemWaves), 0, s, P, fac,
+      hipLaunchKernelGGL((k_m2p_eval<T>), dim3(item_groups((int)nit)), dim3(kP2PBlock * kItemWaves), 0, s, P,
                          pack, dh, dh + o_it, (int)nit, grad, spos, tpos, partial);
       hipLaunchKernelGGL(k_slice_reduce, dim3((unsigned)(red.size() / 5)), dim3(64), 0, s, dh + o_red, partial,
                          P.isrc, P.nsrc, P.itrg, P.ntrg, f.ifpot, f.iffld, f.ifpottarg, f.iffldtarg, pot_s, fld_s,

@@ -40,13 +40,21 @@ __device__ __forceinline__ void cadd(T* p, int k, C2<T> v) { p[2 * k] += v.re; p
 //   [F_RB + h(n,m)] 1/sqrt((n-m)(n+m))
 //   [F_AR + e(n,m)], [F_BR..], [F_CR..]  derivative factors of R (n<=p+1)
 //   [F_AS + e(n,m)], [F_BS..], [F_CS..]  derivative factors of S (n<=p+1)
+//   [F_BT + h(n,m)] ((n-1)^2-m^2)/((2n-1)(2n-3)), 0 at n = m      (n<=p+2)
+//   [F_GN + h(n,m)] R_n^m / Q_n^m                                  (n<=p+1)
+// Q is the harmonic scaled so that its recurrence in n has unit leading
+// coefficient and its diagonal is a plain power,
+//   Q_m^m = w^m,  Q_n = z Q_{n-1} - BT(n,m) rho Q_{n-2}   (Q_{m-1} = 0),
+// with w = -(x + iy), z = z, rho = r^2 for R and, each over r^2, w, z and
+// rho = 1/r^2 for S (times 1/r): one dependent FMA per degree.
 struct FacLayout {
-  int MM, M1, RA, RB, AR, BR, CR, AS, BS, CS, total;
+  int MM, M1, RA, RB, AR, BR, CR, AS, BS, CS, BT, GN, total;
   __host__ __device__ explicit FacLayout(int p) {
     int P = p + 2;                       // tables cover degrees up to p+1
     int H = P * (P + 1) / 2, E = P * P;
     MM = 0; M1 = MM + P + 1; RA = M1 + P + 1; RB = RA + H; AR = RB + H;
-    BR = AR + E; CR = BR + E; AS = CR + E; BS = AS + E; CS = BS + E; total = CS + E;
+    BR = AR + E; CR = BR + E; AS = CR + E; BS = AS + E; CS = BS + E;
+    BT = CS + E; GN = BT + H + P + 1; total = GN + H;
   }
 };
 

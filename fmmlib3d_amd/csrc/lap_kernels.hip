@@ -15,187 +15,88 @@
 namespace fmm3d {
 
 // ---------------------------------------------------------------------------
-// P2M (src/laprouts3d.f:3210, :3835) and P2L (src/laprouts3d.f:3550, :4207)
-// One workgroup per box.  Sources are processed in tiles of `ts`: phase A
-// fills an LDS table of harmonics (one thread per (source, m) column),
-// phase B contracts it against the strengths (one thread per coefficient).
-// IRREG selects P2L (irregular harmonics at the target box centre, sources
-// taken from the boxes of list 4) instead of P2M.
+// P2M (src/laprouts3d.f:3210, :3835) and P2L (src/laprouts3d.f:3550, :4207;
+// IRREG: irregular harmonics at the target box centre, sources taken from the
+// boxes of list 4).  One workgroup per (box, range of orders |m| it writes).
+//
+// Each thread owns up to ITEMS half-table entries (n, a >= 0) of the range and
+// accumulates, in registers over every source, for the weights
+// w = q, v_x, v_y, v_z the four real sums of w_re, w_im times h_re, h_im, from
+// which S^w(n, +-a) = sum_s w_s H_n^{+-a}(u_s) (H^{-a} = conj(H^a)) follow at
+// the end; the weights are scalar loads, four sources at a time.  With at most
+// 64 (128) entries in all the 256 threads form four (two) groups of GS that
+// take the sources in turn and are added in order at the end.
+// The harmonics are the scaled ones of FacLayout: a tile of sources is built in
+// LDS, one thread per (source, column a) walking n with one dependent FMA per
+// degree; columns are stored so that neighbouring lanes (neighbouring a) write
+// neighbouring 16-byte slots.  Per-source scalars are computed 64 sources at a
+// time.  The sums then go to LDS one weight at a time, and the owner of an
+// entry combines the coefficients (n, +-a): charge S^q(n, -m), dipole through
+// the derivative factors and degree n-1 (P2M) or n+1 (P2L) and the orders next
+// to m, with (v_x -+ i v_y)/2 formed by linearity; a range of a dipole call
+// therefore also builds the column on either side of it.
+//
+// What bounds it is the walk along a column, pt + 1 dependent steps of about ten
+// instructions by the lanes that the tile's LDS admits, then the sums' FMAs (16
+// per entry and source with dipoles).  So the recurrence has one dependent FMA
+// per step (the normalised form had three operations), a range takes only the
+// columns it writes, so that a tile holds more sources, and the tile stays near
+// 32 KB, for three or four workgroups per CU.  Against the normalised harmonics
+// with eight FMAs per weight and the weights read from LDS: dipoles at order 26,
+// 200,000 + 180,000 points, P2L 8.5 -> 5.6 ms; 250,000 Plummer points 6.8 -> 4.2
+// ms; 1M + 1M uniform, P2M 1.41 -> 1.19 ms (FP32 1.00 -> 0.86 ms).  Measured and
+// not kept: two tiles, one built while the other is summed, in 512-thread
+// workgroups (5.6 -> 7.6 ms).
 // ---------------------------------------------------------------------------
-template <typename T, bool IRREG>
-__global__ void k_form(DevPlan P, const double* __restrict__ fac, const double* __restrict__ spos,
-                       const double* __restrict__ str, int ifcharge, int ifdipole, int ts,
-                       T* __restrict__ expn) {
-  extern __shared__ unsigned char smem_raw[];
-  T* smem = reinterpret_cast<T*>(smem_raw);
-  const int p = P.p, K = P.K;
-  const int pt = IRREG ? p + 1 : p;  // table degree (dipoles need one more for S)
-  const int H = (pt + 1) * (pt + 2) / 2;
-  FacLayout L(p);
-  T* acc = smem;                    // 2*K
-  T* tab = acc + 2 * K;             // ts * H complex
-  T* sst = tab + 2 * (size_t)ts * H; // ts * 8 : q, dz, du, dd (complex)
-  T* pos = sst + 8 * ts;            // ts * 3 scaled offsets
+constexpr int kFormBatch = 64;  // sources whose scalars are computed at a time
+constexpr int kFormSc = 5;      // scalars per source
+constexpr int kFormRanges = 32; // most ranges of orders
 
-  const int b = IRREG ? P.p2l_boxes[blockIdx.x] : P.p2m_boxes[blockIdx.x];
-  const double ihd = P.inv_side[P.level[b]];
-  const T ih = (T)ihd;
-  const double cx = P.center[3 * b], cy = P.center[3 * b + 1], cz = P.center[3 * b + 2];
-  for (int k = threadIdx.x; k < 2 * K; k += blockDim.x) acc[k] = T(0);
+// The ranges of orders of one launch: range r writes orders lo[r]..hi[r] and
+// builds the columns from[r]..to[r].
+struct FormRanges {
+  int n = 0;
+  short lo[kFormRanges], hi[kFormRanges], from[kFormRanges], to[kFormRanges];
+};
 
-  int jbeg, jend;
-  if (IRREG) { jbeg = P.l4_off[b]; jend = P.l4_off[b + 1]; }
-  else { jbeg = 0; jend = 1; }
-  for (int jj = jbeg; jj < jend; jj++) {
-    const int j = IRREG ? P.l4_idx[jj] : b;
-    const int s0 = P.isrc[j], sn = P.nsrc[j];
-    for (int t0 = 0; t0 < sn; t0 += ts) {
-      const int tn = min(ts, sn - t0);
-      __syncthreads();
-      for (int s = threadIdx.x; s < tn; s += blockDim.x) {
-        const double* x = spos + 4 * (size_t)(s0 + t0 + s);
-        const double* r = str + 8 * (size_t)(s0 + t0 + s);
-        pos[3 * s] = (T)((x[0] - cx) * ihd);
-        pos[3 * s + 1] = (T)((x[1] - cy) * ihd);
-        pos[3 * s + 2] = (T)((x[2] - cz) * ihd);
-        // charge, and dipole components dz = v_z, du = (v_x - i v_y)/2, dd = (v_x + i v_y)/2
-        sst[8 * s] = (T)r[0]; sst[8 * s + 1] = (T)r[1];
-        sst[8 * s + 2] = (T)r[6]; sst[8 * s + 3] = (T)r[7];
-        sst[8 * s + 4] = (T)(0.5 * (r[2] + r[5])); sst[8 * s + 5] = (T)(0.5 * (r[3] - r[4]));
-        sst[8 * s + 6] = (T)(0.5 * (r[2] - r[5])); sst[8 * s + 7] = (T)(0.5 * (r[3] + r[4]));
-      }
-      __syncthreads();
-      // phase A: harmonic columns
-      for (int task = threadIdx.x; task < tn * (pt + 1); task += blockDim.x) {
-        int s = task / (pt + 1), m = task - s * (pt + 1);
-        T ux = pos[3 * s], uy = pos[3 * s + 1], uz = pos[3 * s + 2];
-        T r2 = ux * ux + uy * uy + uz * uz;
-        if (IRREG) {
-          T ir2 = T(1) / r2, ir = sqrt(ir2);
-          irregular_column<T>(fac, L, pt, m, ux, uy, uz, ir2, ir, tab + 2 * (size_t)s * H, 1);
-        } else {
-          regular_column<T>(fac, L, pt, m, ux, uy, uz, r2, tab + 2 * (size_t)s * H, 1);
-        }
-      }
-      __syncthreads();
-      // phase B: contraction, one thread per coefficient (n,m)
-      for (int k = threadIdx.x; k < K; k += blockDim.x) {
-        int n = (int)sqrtf((float)k);
-        while (n * n > k) n--;
-        while ((n + 1) * (n + 1) <= k) n++;
-        int m = k - n * n - n;
-        C2<T> a = {T(0), T(0)};
-        // derivative factors of the harmonic with order -m (grad of conj(H_n^m) = grad H_n^{-m})
-        int km = -m;
-        T fa = 0, fb = 0, fcf = 0;
-        if (IRREG) {
-          fa = (T)fac[L.AS + eidx(n, km)]; fb = (T)fac[L.BS + eidx(n, km)]; fcf = (T)fac[L.CS + eidx(n, km)];
-        } else if (n >= 1) {
-          fa = (T)fac[L.AR + eidx(n, km)]; fb = (T)fac[L.BR + eidx(n, km)]; fcf = (T)fac[L.CR + eidx(n, km)];
-        }
-        for (int s = 0; s < tn; s++) {
-          const T* tb = tab + 2 * (size_t)s * H;
-          if (ifcharge) {
-            C2<T> hv = half_get(tb, n, km, 1);  // conj(H_n^m) = H_n^{-m}
-            cfma(a, C2<T>{sst[8 * s], sst[8 * s + 1]}, hv);
-          }
-          if (ifdipole) {
-            C2<T> g = {T(0), T(0)};
-            int nn = IRREG ? n + 1 : n - 1;
-            if (IRREG || n >= 1) {
-              if (abs(km) <= nn) { C2<T> h = half_get(tb, nn, km, 1); cfma(g, C2<T>{fa * sst[8 * s + 2], fa * sst[8 * s + 3]}, h); }
-              if (abs(km + 1) <= nn) { C2<T> h = half_get(tb, nn, km + 1, 1); cfma(g, C2<T>{fb * sst[8 * s + 4], fb * sst[8 * s + 5]}, h); }
-              if (abs(km - 1) <= nn) { C2<T> h = half_get(tb, nn, km - 1, 1); cfma(g, C2<T>{fcf * sst[8 * s + 6], fcf * sst[8 * s + 7]}, h); }
-            }
-            // d/dy of H(u) with u = (y-c)/h gives a factor 1/h
-            a.re += g.re * ih;
-            a.im += g.im * ih;
-          }
-        }
-        acc[2 * k] += a.re;
-        acc[2 * k + 1] += a.im;
-      }
-    }
+// Start of the column after one at `base` of `len` entries, that column being
+// the k-th: at a multiple of 8 entries plus k (the 32 LDS banks hold 8 complex
+// FP64 values).
+__host__ __device__ inline int form_next_col(int base, int len, int k) {
+  int c = base + len;
+  while ((c & 7) != (k & 7)) c++;
+  return c;
+}
+// entries of one source's row of columns from..to, degrees up to pt
+__host__ __device__ inline int form_row(int pt, int from, int to) {
+  int c = 0;
+  for (int a = from; a <= to; a++) c = form_next_col(c, pt + 1 - a, a + 1 - from);
+  return c;
+}
+// the ranges for degrees up to pt: as many orders each as `cap` entries hold
+inline FormRanges form_ranges(int pt, bool dip, int cap) {
+  FormRanges R;
+  const int halo = dip ? 1 : 0;
+  for (int lo = 0; lo <= pt; R.n++) {
+    if (R.n == kFormRanges) { R.n = 0; break; }
+    const int from = lo - halo < 0 ? 0 : lo - halo;
+    int to = from, e = pt + 1 - from;
+    while (to < pt && (e + pt - to <= cap || to < lo + halo)) { to++; e += pt + 1 - to; }
+    const int hi = to == pt ? pt : to - halo;
+    if (e > cap) { R.n = 0; break; }
+    R.lo[R.n] = (short)lo; R.hi[R.n] = (short)hi; R.from[R.n] = (short)from; R.to[R.n] = (short)to;
+    lo = hi + 1;
   }
-  __syncthreads();
-  // P2L: L = sum q conj(S(u)) / h ; P2M: M = sum q conj(R(u))
-  const T sc = IRREG ? ih : T(1);
-  T* out = expn + 2 * (size_t)b * K;
-  for (int k = threadIdx.x; k < 2 * K; k += blockDim.x) out[k] += acc[k] * sc;
+  return R;
 }
-
-// ---------------------------------------------------------------------------
-// P2M / P2L with per-thread sums.  Each thread owns up to two half-table
-// entries (n', a >= 0) and accumulates, in registers over every source of the
-// box, S^w(n', +-a) = sum_s w_s H_{n'}^{+-a}(u_s) for the weights
-// w = q, v_x, v_y, v_z (H^{-a} = conj(H^a)); the weights are wave-uniform
-// loads.  The harmonic table of a tile of `ts` sources is built in LDS, one
-// thread per (column m, source), m-major so that a wave holds few orders and
-// its loop lengths are close; each source's scalars (form_scalars) are
-// computed once, during the previous tile's sums, from positions read while
-// the previous tile's table was built.  At the end the sums go to LDS
-// and one thread per coefficient combines them: charge S^q(n, -m), dipole
-// through the derivative factors and degree n-1 (P2M) or n+1 (P2L), with
-// (v_x -+ i v_y)/2 formed from S^{v_x}, S^{v_y} by linearity.
-// ---------------------------------------------------------------------------
-// Threads of k_form2.  P2L: 512, since the tile's LDS admits two workgroups per
-// CU and twice the waves of 256-thread groups hide the column recurrence.
-// P2M: 256, since it runs beside the near field, where a 512-thread workgroup
-// waits for two near-field workgroups to leave a CU.  Each thread owns
-// 512 / threads half-table entries, twice that for larger orders.
-template <bool IRREG>
-__host__ __device__ constexpr int form2_threads() {
-  return IRREG ? 512 : 256;
-}
-// LDS bytes k_form2 keeps ahead of the harmonic table, 16-aligned: the
-// recurrence factors (FacLayout MM..RB) and cm[m] = prod_{k<=m} MM[k],
-// m = 0..p+2
-// Tile row stride (entries) of k_form2: the half table of one source, padded
-// so that consecutive sources start one entry apart modulo the 32 LDS banks
-// (the harmonic columns of neighbouring sources are written by neighbouring
-// lanes)
-template <typename T>
-__host__ __device__ inline int form2_row_stride(int H) {
-  const int words = 2 * (int)sizeof(T) / 4;  // per complex entry
-  int hs = H;
-  while ((hs * words) % 32 != words) hs++;
-  return hs;
-}
-
-__host__ __device__ inline size_t form2_fac_bytes(int p) {
-  return ((size_t)(FacLayout(p).AR + p + 3) * sizeof(double) + 15) / 16 * 16;
-}
-
-// LDS stride (T) of the per-source scalars: 8 used, padded so that the rows
-// of neighbouring sources start in different banks
-constexpr int kFormScStride = 10;
-
-// Per-source scalars of the column tasks, 8 T per source: the power base
-// w = -(ux + i uy) (times 1/|u|^2 for S), uz, the scale of the recurrence's
-// second term (|u|^2 for R, 1 for S), the scale of each new entry (1 for R,
-// 1/|u|^2 for S) and of the diagonal (1 for R, 1/|u| for S).
-template <typename T, bool IRREG>
-__device__ __forceinline__ void form_scalars(double x, double y, double z, double cx, double cy, double cz,
-                                             double ihd, T* sc) {
-  const T ux = (T)((x - cx) * ihd), uy = (T)((y - cy) * ihd), uz = (T)((z - cz) * ihd);
-  const T r2 = ux * ux + uy * uy + uz * uz;
-  T ir2 = T(1), ir = T(1);
-  if (IRREG) {
-    ir2 = T(1) / r2;
-    ir = sqrt(ir2);
-  }
-  sc[0] = IRREG ? -ux * ir2 : -ux;
-  sc[1] = IRREG ? -uy * ir2 : -uy;
-  sc[2] = uz;
-  sc[3] = IRREG ? T(1) : r2;
-  sc[4] = ir2;
-  sc[5] = ir;
-  sc[6] = T(0);
-  sc[7] = T(0);
+// LDS of k_form2 in T ahead of the tile: recurrence factors of a row, column
+// starts, the batch's scalars
+__host__ __device__ inline int form_head(int pt, int row) {
+  return (row + 8 + 3) / 4 * 4 + (pt + 2 + 3) / 4 * 4 + kFormBatch * kFormSc;
 }
 
 // One complex table entry as a single LDS store (16 bytes for double, 8 for
-// float; the k_form2 tile rows keep entries at that alignment)
+// float; tile rows keep entries at that alignment)
 template <typename T>
 __device__ __forceinline__ void cst_vec(T* p, int k, C2<T> v) {
   using V2 = typename std::conditional<std::is_same<T, double>::value, double2, float2>::type;
@@ -205,274 +106,313 @@ __device__ __forceinline__ void cst_vec(T* p, int k, C2<T> v) {
   *reinterpret_cast<V2*>(p + 2 * k) = t;
 }
 
-// Column m of the regular (R) or irregular (S) harmonics of one source into
-// a half table, n = m..pt, from that source's scalars `sc` (form_scalars).
-// The diagonal entry R_m^m = cm w^m, S_m^m = ir cm (w ir2)^m is taken by
-// binary powers; then the three-term recurrences of regular_column and
-// irregular_column.  The entry index advances by n + 1 per step, and the
-// next step's two recurrence factors are read from LDS before this step's
-// arithmetic, so the LDS latency overlaps the dependent chain.
-template <typename T, bool IRREG>
-__device__ __forceinline__ void form_column(const double* facl, const FacLayout& L, int pt, int m, T cm,
-                                            const T* sc, T* out) {
-  C2<T> base = {sc[0], sc[1]};
-  const T uz = sc[2], bsc = sc[3], csc = sc[4];
-  C2<T> r = {IRREG ? cm * sc[5] : cm, T(0)};
-  for (int e = m; e; e >>= 1) {
-    if (e & 1) r = cmul(r, base);
-    base = cmul(base, base);
-  }
-  int k = hidx(m, m);
-  cst_vec(out, k, r);
-  if (m + 1 > pt) return;
-  const T g = (T)facl[L.M1 + m] * uz * csc;
-  C2<T> r1 = {g * r.re, g * r.im};
-  k += m + 1;  // hidx(m + 1, m)
-  cst_vec(out, k, r1);
-  if (m + 2 > pt) return;
-  C2<T> r0 = r;
-  k += m + 2;  // hidx(m + 2, m)
-  double fa = facl[L.RA + k], fb = facl[L.RB + k];
-  T cn = (T)(2 * m + 3);  // 2n - 1, exact
-#pragma unroll 2
-  for (int n = m + 2; n <= pt; n++) {
-    const T b = IRREG ? (T)fa : (T)fa * bsc;
-    const T c = IRREG ? (T)fb * csc : (T)fb;
-    const int kn = k + n + 1;  // hidx(n + 1, m)
-    // at n = pt this reads past the column (still inside the factor and cm
-    // tables in LDS); the values go unused
-    fa = facl[L.RA + kn];
-    fb = facl[L.RB + kn];
-    const T a = cn * uz;
-    cn += T(2);
-    const C2<T> rn = {(a * r1.re - b * r0.re) * c, (a * r1.im - b * r0.im) * c};
-    cst_vec(out, k, rn);
-    r0 = r1;
-    r1 = rn;
-    k = kn;
-  }
-}
-
-template <typename T, bool IRREG, bool CHG, bool DIP, int ITEMS>
-__global__ __launch_bounds__(form2_threads<IRREG>()) void k_form2(DevPlan P, const double* __restrict__ fac,
-                                               const double* __restrict__ spos, const double* __restrict__ str,
-                                               int ts, T* __restrict__ expn) {
-  extern __shared__ unsigned char smem_raw[];
+// `region`: the tile's size in T; it also holds one weight's sums at the end
+template <typename T, bool IRREG, bool CHG, bool DIP, int GS, int ITEMS>
+__global__ __launch_bounds__(256) void k_form2(DevPlan P, const double* __restrict__ fac,
+                                               const double* __restrict__ spos, const T* __restrict__ str,
+                                               FormRanges R, int region, T* __restrict__ expn) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  using V2 = typename std::conditional<std::is_same<T, double>::value, double2, float2>::type;
   const int p = P.p, K = P.K;
   const int pt = IRREG ? p + 1 : p;
-  const int H = (pt + 1) * (pt + 2) / 2;
-  const int HS = form2_row_stride<T>(H);
-  const int P2 = (pt + 1) * (pt + 1);
-  FacLayout L(p);
-  const int tid = threadIdx.x;
-  // the recurrence factors (MM, M1, RA, RB: the head of the factor table) in
-  // LDS, ahead of the harmonic table: each column task reads a different
-  // entry; then the diagonal constants cm
-  double* facl = reinterpret_cast<double*>(smem_raw);
-  double* cmt = facl + L.AR;
-  for (int k = tid; k < L.AR; k += blockDim.x) facl[k] = fac[k];
+  const FacLayout L(p);
+  const int tid = threadIdx.x, rg = blockIdx.y;
+  const int lo = R.lo[rg], hi = R.hi[rg], from = R.from[rg], ncol = R.to[rg] - from + 1;
+  T* smem = reinterpret_cast<T*>(smem_raw);
+  T* beta = smem;
+  const int row = form_row(pt, from, from + ncol - 1);
+  int* cb = reinterpret_cast<int*>(smem + (row + 8 + 3) / 4 * 4);
+  T* scs = smem + form_head(pt, row) - kFormBatch * kFormSc;
+  T* tab = smem + form_head(pt, row);
+  const int ts = min(kFormBatch, region / (2 * row));
   if (tid == 0) {
-    double c = 1.0;
-    cmt[0] = 1.0;
-    for (int k = 1; k <= pt; k++) { c *= fac[L.MM + k]; cmt[k] = c; }
+    int c = 0;
+    for (int k = 0; k < ncol; k++) {
+      cb[k] = c;
+      c = form_next_col(c, pt + 1 - from - k, k + 1);
+    }
   }
-  T* tab = reinterpret_cast<T*>(smem_raw + form2_fac_bytes(p));
+  __syncthreads();
+  constexpr int G = 256 / GS;
+  const int grp = __builtin_amdgcn_readfirstlane(tid / GS), lt = tid - grp * GS;
+  int ent[ITEMS], adr[ITEMS];  // owned entries: n << 8 | a (or -1), and their place in a row
+#pragma unroll
+  for (int q = 0; q < ITEMS; q++) {
+    int k = 0, r = lt + q * GS;
+    while (k < ncol && r >= pt + 1 - from - k) { r -= pt + 1 - from - k; k++; }
+    ent[q] = -1;
+    adr[q] = 0;
+    if (k < ncol) {
+      const int a = from + k, n = a + r;
+      ent[q] = n << 8 | a;
+      adr[q] = cb[k] + r;
+      if (grp == 0) beta[adr[q]] = (T)fac[L.BT + hidx(n, a)];
+    }
+  }
   const int b = IRREG ? P.p2l_boxes[blockIdx.x] : P.p2m_boxes[blockIdx.x];
   const double ihd = P.inv_side[P.level[b]];
   const T ih = (T)ihd;
   const double cx = P.center[3 * b], cy = P.center[3 * b + 1], cz = P.center[3 * b + 2];
-  T acc[ITEMS][16];
+  constexpr int NW = (CHG ? 1 : 0) + (DIP ? 3 : 0), W0 = CHG ? 0 : 1;  // weights, first of q, x, y, z
+  T acc[ITEMS][NW][4];
 #pragma unroll
   for (int q = 0; q < ITEMS; q++)
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[q][e] = T(0);
-  // per-source scalars of the current tile, after the tile region
-  T* scs = tab + 2 * (size_t)max(ts * HS, 4 * P2);
-  T* wsh = scs + kFormScStride * ts;  // the tile's source weights
-  int rot = blockIdx.x;
-  using V2 = typename std::conditional<std::is_same<T, double>::value, double2, float2>::type;
-  // tile cursor over the sources of the list-4 boxes (P2L) or of box b (P2M):
-  // (jj, t0) moves to the first tile holding sources, s0/sn of its box
-  const int jend = IRREG ? P.l4_off[b + 1] : 1;
-  auto settle = [&](int& jj, int& t0, int& s0, int& sn) {
-    for (; jj < jend; jj++, t0 = 0) {
-      const int j = IRREG ? P.l4_idx[jj] : b;
-      s0 = P.isrc[j];
-      sn = P.nsrc[j];
-      if (t0 < sn) return;
-    }
-  };
-  int jj = IRREG ? P.l4_off[b] : 0, t0 = 0, s0 = 0, sn = 0;
-  settle(jj, t0, s0, sn);
-  if (jj < jend && tid < min(ts, sn - t0)) {
-    const double* x = spos + 4 * (size_t)(s0 + t0 + tid);
-    form_scalars<T, IRREG>(x[0], x[1], x[2], cx, cy, cz, ihd, scs + kFormScStride * tid);
-  }
-  while (jj < jend) {
-    const int tn = min(ts, sn - t0), cs0 = s0 + t0;
-    int njj = jj, nt0 = t0 + tn, ns0 = s0, nsn = sn;
-    settle(njj, nt0, ns0, nsn);
-    const int ntn = njj < jend ? min(ts, nsn - nt0) : 0;
-    __syncthreads();  // this tile's scalars written; the last tile's sums done with the table
-    // the next tile's positions, read while this tile's table is built
-    double nx = 0, ny = 0, nz = 0;
-    if (tid < ntn) {
-      const double* x = spos + 4 * (size_t)(ns0 + nt0 + tid);
-      nx = x[0];
-      ny = x[1];
-      nz = x[2];
-    }
-    // this tile's weights, one value per thread (8 ts <= 256 <= blockDim.x),
-    // staged in LDS
-    // for the sums
-    T wreg = T(0);
-    if (tid < 8 * tn) wreg = (T)str[8 * (size_t)cs0 + tid];
-    // column tasks, m-major, in blocks of 64; block k of round r goes to wave
-    // (k - r - rot) mod nw: the wave with the shortest columns of one round
-    // takes the longest of the next, and the long low-m columns visit every
-    // wave (and SIMD) in turn from tile to tile
-    {
-      const int ntask = tn * (pt + 1), nw = (int)blockDim.x >> 6;
-      int vw = ((tid >> 6) + rot) % nw;
-      for (int r0 = 0; r0 < ntask; r0 += blockDim.x) {
-        const int task = r0 + 64 * vw + (tid & 63);
-        if (task < ntask) {
-          const int m = task / tn, s = task - m * tn;
-          form_column<T, IRREG>(facl, L, pt, m, (T)cmt[m], scs + kFormScStride * s, tab + 2 * (size_t)s * HS);
+    for (int w = 0; w < NW; w++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[q][w][e] = T(0);
+  const int jbeg = IRREG ? P.l4_off[b] : 0, jend = IRREG ? P.l4_off[b + 1] : 1;
+  for (int jj = jbeg; jj < jend; jj++) {
+    const int j = IRREG ? P.l4_idx[jj] : b;
+    const int s0 = P.isrc[j], sn = P.nsrc[j];
+    for (int t0 = 0; t0 < sn; t0 += kFormBatch) {
+      const int bn = min(kFormBatch, sn - t0);
+      // (the batch before is done with: a barrier ended its last tile)
+      if (tid < bn) {
+        const double* x = spos + 4 * (size_t)(s0 + t0 + tid);
+        const T ux = (T)((x[0] - cx) * ihd), uy = (T)((x[1] - cy) * ihd), uz = (T)((x[2] - cz) * ihd);
+        const T r2 = ux * ux + uy * uy + uz * uz;
+        T* sc = scs + kFormSc * tid;
+        if (IRREG) {
+          const T ir2 = T(1) / r2;
+          sc[0] = -ux * ir2; sc[1] = -uy * ir2; sc[2] = uz * ir2; sc[3] = ir2; sc[4] = sqrt(ir2);
+        } else {
+          sc[0] = -ux; sc[1] = -uy; sc[2] = uz; sc[3] = r2; sc[4] = T(1);
         }
-        vw = vw + 1 == nw ? 0 : vw + 1;
       }
-      rot++;
+      __syncthreads();
+      for (int u0 = 0; u0 < bn; u0 += ts) {
+        const int tn = min(ts, bn - u0);
+        // columns: task = source * ncol + (a - from)
+        for (int task = tid; task < tn * ncol; task += 256) {
+          const int s = task / ncol, k0 = task - s * ncol, a = from + k0;
+          const T* sc = scs + kFormSc * (u0 + s);
+          C2<T> w = {sc[0], sc[1]}, r = {sc[4], T(0)}, r0 = {T(0), T(0)};
+          const T zz = sc[2], rho = sc[3];
+          T* out = tab + 2 * (size_t)(s * row + cb[k0]);
+          const T* bt = beta + cb[k0] + 1;
+          const int len = pt + 1 - a;
+          // four recurrence factors at a time, read ahead of the four steps
+          // that use them (the last reads run past the column's, unused)
+          T bc[4], bn4[4];
+#pragma unroll
+          for (int u = 0; u < 4; u++) bc[u] = bt[u];
+          for (int e = a; e; e >>= 1) {
+            if (e & 1) r = cmul(r, w);
+            w = cmul(w, w);
+          }
+          auto step = [&](int k, T bk) {
+            cst_vec(out, k, r);
+            const T br = bk * rho;
+            C2<T> rn;
+            rn.re = fma(zz, r.re, -(br * r0.re));
+            rn.im = fma(zz, r.im, -(br * r0.im));
+            r0 = r;
+            r = rn;
+          };
+          int k = 0;
+          for (; k + 4 <= len; k += 4) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) bn4[u] = bt[k + 4 + u];
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int u = 0; u < 4; u++) step(k + u, bc[u]);
+#pragma unroll
+            for (int u = 0; u < 4; u++) bc[u] = bn4[u];
+          }
+#pragma unroll
+          for (int u = 0; u < 3; u++)
+            if (k + u < len) step(k + u, bc[u]);
+        }
+        __syncthreads();
+        // sums, four sources' weights at a time (sources past the tile's end
+        // read its last weights again, unused)
+        for (int s = grp; s < tn; s += 4 * G) {
+          T wr[4][NW], wi[4][NW];
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            const int sv = s0 + t0 + u0 + min(s + v * G, tn - 1);
+            const T* __restrict__ wv = str + 8 * (size_t)(unsigned)__builtin_amdgcn_readfirstlane(sv);
+#pragma unroll
+            for (int w = 0; w < NW; w++) { wr[v][w] = wv[2 * (W0 + w)]; wi[v][w] = wv[2 * (W0 + w) + 1]; }
+          }
+#pragma unroll
+          for (int v = 0; v < 4; v++) {
+            if (s + v * G >= tn) break;
+#pragma unroll
+            for (int q = 0; q < ITEMS; q++) {
+              const V2 hv = *reinterpret_cast<const V2*>(tab + 2 * (size_t)((s + v * G) * row + adr[q]));
+#pragma unroll
+              for (int w = 0; w < NW; w++) {
+                acc[q][w][0] = fma(wr[v][w], hv.x, acc[q][w][0]);
+                acc[q][w][1] = fma(wi[v][w], hv.y, acc[q][w][1]);
+                acc[q][w][2] = fma(wr[v][w], hv.y, acc[q][w][2]);
+                acc[q][w][3] = fma(wi[v][w], hv.x, acc[q][w][3]);
+              }
+            }
+          }
+        }
+        __syncthreads();
+      }
     }
-    if (tid < 8 * tn) wsh[tid] = wreg;
-    __syncthreads();
-    if (tid < ntn) form_scalars<T, IRREG>(nx, ny, nz, cx, cy, cz, ihd, scs + kFormScStride * tid);
-#pragma unroll 2
-    for (int s = 0; s < tn; s++) {
-      const T* wv = wsh + 8 * s;
+  }
+  // one weight at a time: its sums S(n, +a), S(n, -a) to LDS (four values at
+  // an entry's place), then into the owners' coefficients (n, a) and (n, -a)
+  T co[ITEMS][4], cg[ITEMS][4];
+#pragma unroll
+  for (int q = 0; q < ITEMS; q++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) co[q][e] = cg[q][e] = T(0);
+  auto sget = [&](int n, int m, T& re, T& im) {
+    const int a = m < 0 ? -m : m;
+    re = im = T(0);
+    if (a > n) return;
+    const T* o = tab + 4 * (cb[a - from] + n - a) + (m < 0 ? 2 : 0);
+    re = o[0];
+    im = o[1];
+  };
+#pragma unroll
+  for (int w = 0; w < NW; w++) {
+    for (int g = 0; g < G; g++) {
+      if (grp == g) {
+#pragma unroll
+        for (int q = 0; q < ITEMS; q++) {
+          if (ent[q] < 0) continue;
+          const T gn = (T)fac[L.GN + hidx(ent[q] >> 8, ent[q] & 255)];
+          const T* A = acc[q][w];
+          const T v[4] = {gn * (A[0] - A[1]), gn * (A[2] + A[3]), gn * (A[0] + A[1]), gn * (A[3] - A[2])};
+          T* o = tab + 4 * adr[q];
+#pragma unroll
+          for (int e = 0; e < 4; e++) o[e] = g == 0 ? v[e] : o[e] + v[e];
+        }
+      }
+      __syncthreads();
+    }
+    const int c = W0 + w;  // 0: q, 1..3: v_x, v_y, v_z
+    if (grp == 0) {
 #pragma unroll
       for (int q = 0; q < ITEMS; q++) {
-        const int h = tid + q * (int)blockDim.x;
-        if (h < H) {
-          const V2 hv = *reinterpret_cast<const V2*>(tab + 2 * ((size_t)s * HS + h));
-          const T hr = hv.x, hi = hv.y;
+        const int n = ent[q] >> 8, a = ent[q] & 255;
+        if (ent[q] < 0 || a < lo || a > hi || n > p) continue;
 #pragma unroll
-          for (int c = 0; c < 4; c++) {
-            if ((c == 0 && !CHG) || (c > 0 && !DIP)) continue;
-            const T wr = wv[2 * c], wi = wv[2 * c + 1];
-            T* A = &acc[q][4 * c];
-            A[0] = fma(wr, hr, fma(-wi, hi, A[0]));  // w H^{+a}
-            A[1] = fma(wr, hi, fma(wi, hr, A[1]));
-            A[2] = fma(wr, hr, fma(wi, hi, A[2]));   // w H^{-a} = w conj(H^{a})
-            A[3] = fma(wi, hr, fma(-wr, hi, A[3]));
+        for (int sg = 0; sg < 2; sg++) {
+          const int km = sg ? a : -a;  // coefficient m = -km
+          T re, im;
+          if (c == 0) {
+            sget(n, km, re, im);
+            co[q][2 * sg] = re;
+            co[q][2 * sg + 1] = im;
+          } else if (IRREG || n >= 1) {
+            const int nn = IRREG ? n + 1 : n - 1;
+            T &gr = cg[q][2 * sg], &gi = cg[q][2 * sg + 1];
+            if (c == 3) {
+              const T fa = (T)fac[(IRREG ? L.AS : L.AR) + eidx(n, km)];
+              sget(nn, km, re, im);
+              gr += fa * re;
+              gi += fa * im;
+            } else {
+              // (v_x - i v_y)/2 with the order one up, (v_x + i v_y)/2 one down
+              const T fb = (T)fac[(IRREG ? L.BS : L.BR) + eidx(n, km)] * T(0.5);
+              const T fc = (T)fac[(IRREG ? L.CS : L.CR) + eidx(n, km)] * T(0.5);
+              T dr, di;
+              sget(nn, km + 1, re, im);
+              sget(nn, km - 1, dr, di);
+              if (c == 1) {
+                gr += fb * re + fc * dr;
+                gi += fb * im + fc * di;
+              } else {
+                gr += fb * im - fc * di;
+                gi += fc * dr - fb * re;
+              }
+            }
           }
         }
       }
     }
-    jj = njj;
-    t0 = nt0;
-    s0 = ns0;
-    sn = nsn;
+    __syncthreads();
   }
-  __syncthreads();
-  // sums to LDS: S[c][eidx(n', m')] complex, c = q, v_x, v_y, v_z
-#pragma unroll
-  for (int q = 0; q < ITEMS; q++) {
-    const int h = tid + q * (int)blockDim.x;
-    if (h < H) {
-      int n = (int)((sqrtf(8.0f * h + 1.0f) - 1.0f) * 0.5f);
-      while (n * (n + 1) / 2 > h) n--;
-      while ((n + 1) * (n + 2) / 2 <= h) n++;
-      const int a = h - n * (n + 1) / 2;
-#pragma unroll
-      for (int c = 0; c < 4; c++) {
-        T* S = tab + 2 * (size_t)c * P2;
-        S[2 * eidx(n, a)] = acc[q][4 * c];
-        S[2 * eidx(n, a) + 1] = acc[q][4 * c + 1];
-        S[2 * eidx(n, -a)] = acc[q][4 * c + 2];
-        S[2 * eidx(n, -a) + 1] = acc[q][4 * c + 3];
-      }
-    }
-  }
-  __syncthreads();
+  if (grp != 0) return;
   const T sc = IRREG ? ih : T(1);
   T* out = expn + 2 * (size_t)b * K;
-  for (int k = tid; k < K; k += blockDim.x) {
-    int n = (int)sqrtf((float)k);
-    while (n * n > k) n--;
-    while ((n + 1) * (n + 1) <= k) n++;
-    const int m = k - n * n - n, km = -m;
-    T ar = 0, ai = 0;
-    if (CHG) {
-      ar = tab[2 * eidx(n, km)];
-      ai = tab[2 * eidx(n, km) + 1];
+#pragma unroll
+  for (int q = 0; q < ITEMS; q++) {
+    const int n = ent[q] >> 8, a = ent[q] & 255;
+    if (ent[q] < 0 || a < lo || a > hi || n > p) continue;
+#pragma unroll
+    for (int sg = 0; sg < 2; sg++) {
+      if (sg && a == 0) continue;
+      T* o = out + 2 * eidx(n, sg ? -a : a);
+      o[0] += (co[q][2 * sg] + cg[q][2 * sg] * ih) * sc;
+      o[1] += (co[q][2 * sg + 1] + cg[q][2 * sg + 1] * ih) * sc;
     }
-    if (DIP && (IRREG || n >= 1)) {
-      const int nn = IRREG ? n + 1 : n - 1;
-      const T fa = (T)fac[(IRREG ? L.AS : L.AR) + eidx(n, km)];
-      const T fb = (T)fac[(IRREG ? L.BS : L.BR) + eidx(n, km)] * T(0.5);
-      const T fc = (T)fac[(IRREG ? L.CS : L.CR) + eidx(n, km)] * T(0.5);
-      const T* SX = tab + 2 * (size_t)P2;
-      const T* SY = SX + 2 * (size_t)P2;
-      const T* SZ = SY + 2 * (size_t)P2;
-      T gr = 0, gi = 0;
-      if (km <= nn && km >= -nn) {
-        gr += fa * SZ[2 * eidx(nn, km)];
-        gi += fa * SZ[2 * eidx(nn, km) + 1];
-      }
-      if (km + 1 <= nn && km + 1 >= -nn) {  // (v_x - i v_y)/2
-        const int e = eidx(nn, km + 1);
-        gr += fb * (SX[2 * e] + SY[2 * e + 1]);
-        gi += fb * (SX[2 * e + 1] - SY[2 * e]);
-      }
-      if (km - 1 <= nn && km - 1 >= -nn) {  // (v_x + i v_y)/2
-        const int e = eidx(nn, km - 1);
-        gr += fc * (SX[2 * e] - SY[2 * e + 1]);
-        gi += fc * (SX[2 * e + 1] + SY[2 * e]);
-      }
-      ar += gr * ih;
-      ai += gi * ih;
-    }
-    out[2 * k] += ar * sc;
-    out[2 * k + 1] += ai * sc;
   }
 }
 
 // ---------------------------------------------------------------------------
-// L2P (src/laprouts3d.f:2772 l3dtaevalall_trunc) from a packed expansion.
-// For every box of the L2P list the local
-// expansion L and the three derived expansions of the gradient,
-//   Gz(n,m) = AR(n+1,m)   L(n+1,m),
-//   Gu(n,m) = BR(n+1,m-1) L(n+1,m-1),
-//   Gd(n,m) = CR(n+1,m+1) L(n+1,m+1)       (n <= p-1; zero at n = p),
-// are stored per half-table entry (n, a >= 0) in the order the evaluation
-// walks them (column a, then n = a..p): 8 complex values
-//   L(n,a) L(n,-a) Gz(n,a) Gz(n,-a) Gu(n,a) Gu(n,-a) Gd(n,a) Gd(n,-a)
-// (the -a slots are zero for a = 0).  The evaluation then reads them with
-// wave-uniform loads and pays four complex products per harmonic:
-//   pot = sum L R, d/dz = sum Gz R, (d/dx + i d/dy) = sum Gu R, (d/dx - i d/dy) = sum Gd R.
+// L2P (src/laprouts3d.f:2772 l3dtaevalall_trunc) and M2P (list 3,
+// src/laprouts3d.f:2432 l3dmpevalall_trunc) from packed expansions.  The
+// potential and the three gradient sums are
+//   pot = sum E H, d/dz = sum Gz H, (d/dx + i d/dy) = sum Gu H, (d/dx - i d/dy) = sum Gd H
+// over the harmonics H = R of degree n <= p with
+//   Gz(n,m) = AR(n+1,m) L(n+1,m), Gu = BR(n+1,m-1) L(n+1,m-1), Gd = CR(n+1,m+1) L(n+1,m+1)
+// for a local L, and H = S of degree n <= p+1 with
+//   Gz(n,m) = AS(n-1,m) M(n-1,m), Gu = BS(n-1,m-1) M(n-1,m-1), Gd = CS(n-1,m+1) M(n-1,m+1)
+// for a multipole M (zero where an index is outside).  An entry (n, a >= 0) of
+// the pack holds, for each X of E, Gz, Gu, Gd and c+- = X(n, +-a) (c- = 0 for
+// a = 0), the four reals that take the harmonic h = H_n^a to c+ h + c- conj(h),
+//   re: (c+ + c-)_re h_re - (c+ - c-)_im h_im,  im: (c+ + c-)_im h_re + (c+ - c-)_re h_im,
+// times the scale of FacLayout's recurrence, then that recurrence's factor for
+// degree n + 1: kPackEntry values.  Entries are in the order of the walk
+// (column a, then n = a..pd), columns padded to an even count by zero entries.
+// The walk reads them with scalar loads, one entry ahead, and pays 16 FMAs and
+// the recurrence's 5 operations per entry and point (32 and 9 before, the
+// harmonics normalised and c+ h, c- conj(h) taken apart).  VALU bound: 400,000
+// clustered points at order 39, M2P 11.4 -> 8.2 ms; 200,000 + 180,000 at order
+// 26 7.8 -> 5.7 ms; 1M + 1M uniform, L2P 1.59 -> 1.22 ms (FP32 1.22 -> 0.74 ms).
 // ---------------------------------------------------------------------------
-__host__ __device__ inline int walk_index(int p, int a, int n) { return a * (p + 1) - a * (a - 1) / 2 + (n - a); }
+constexpr int kPackEntry = 18;
+__host__ __device__ inline int pack_col(int pd, int a) { return (pd + 2 - a) & ~1; }  // entries of column a
+__host__ __device__ inline int pack_entries(int pd) {
+  int e = 0;
+  for (int a = 0; a <= pd; a++) e += pack_col(pd, a);
+  return e;
+}
+
+// coefficients c+- of E, Gz, Gu, Gd at (n, a), as (re, im) pairs, to an entry
+template <typename T>
+__device__ __forceinline__ void pack_store(T* __restrict__ o, const T (&v)[16], T g, T beta) {
+#pragma unroll
+  for (int x = 0; x < 4; x++) {
+    o[4 * x] = g * (v[4 * x] + v[4 * x + 2]);
+    o[4 * x + 1] = -g * (v[4 * x + 1] - v[4 * x + 3]);
+    o[4 * x + 2] = g * (v[4 * x + 1] + v[4 * x + 3]);
+    o[4 * x + 3] = g * (v[4 * x] - v[4 * x + 2]);
+  }
+  o[16] = beta;
+  o[17] = T(0);
+}
 
 template <typename T>
 __global__ void k_l2p_pack(DevPlan P, const double* __restrict__ fac, const T* __restrict__ lo,
                            T* __restrict__ pack) {
   const int p = P.p, K = P.K;
-  const int H = (p + 1) * (p + 2) / 2;
+  const int NE = pack_entries(p);
   FacLayout L(p);
-  const size_t total = (size_t)P.n_l2p * H;
+  const size_t total = (size_t)P.n_l2p * NE;
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(t / H), w = (int)(t - (size_t)i * H);
-    int a = 0;
-    while (a < p && walk_index(p, a + 1, a + 1) <= w) a++;
-    const int n = a + (w - walk_index(p, a, a));
+    const int i = (int)(t / NE);
+    int a = 0, r = (int)(t - (size_t)i * NE);
+    while (r >= pack_col(p, a)) { r -= pack_col(p, a); a++; }
+    const int n = a + r;
     const T* E = lo + 2 * (size_t)P.l2p_boxes[i] * K;
     T v[16];
 #pragma unroll
     for (int e = 0; e < 16; e++) v[e] = T(0);
-    v[0] = E[2 * eidx(n, a)];
-    v[1] = E[2 * eidx(n, a) + 1];
-    if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
+    if (n <= p) {
+      v[0] = E[2 * eidx(n, a)];
+      v[1] = E[2 * eidx(n, a) + 1];
+      if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
+    }
     if (n + 1 <= p) {
       const int n1 = n + 1;
       for (int sgn = 0; sgn < (a > 0 ? 2 : 1); sgn++) {
@@ -486,37 +426,83 @@ __global__ void k_l2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
         v[13 + 2 * sgn] = fd * E[2 * eidx(n1, m + 1) + 1];
       }
     }
-    T* o = pack + 16 * t;
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[e] = v[e];
+    pack_store(pack + kPackEntry * t, v, n <= p ? (T)fac[L.GN + hidx(n, a)] : T(0), n <= p ? (T)fac[L.BT + hidx(n + 1, a)] : T(0));
   }
 }
 
-// out += c+ h + c- conj(h)
-template <typename T>
-__device__ __forceinline__ void pack_fma(C2<T>& out, const T* c, const C2<T>& h) {
-  out.re = fma(c[0], h.re, fma(-c[1], h.im, fma(c[2], h.re, fma(c[3], h.im, out.re))));
-  out.im = fma(c[0], h.im, fma(c[1], h.re, fma(-c[2], h.im, fma(c[3], h.re, out.im))));
+// One pack entry in scalar registers
+template <typename T, bool GRAD>
+struct PackRec {
+  T c[GRAD ? 16 : 4], b;
+  __device__ __forceinline__ void load(const T* __restrict__ o) {
+#pragma unroll
+    for (int e = 0; e < (GRAD ? 16 : 4); e++) c[e] = o[e];
+    b = o[16];
+  }
+};
+
+// The walk over one pack at a point: w, zz, rho of the recurrence, h00 its
+// first value; out (pot, d/dz, U, D) is added to.  Reads one entry past the
+// pack's last.
+template <typename T, bool GRAD>
+__device__ __forceinline__ void pack_walk(const T* __restrict__ pk, int pd, C2<T> w, T zz, T rho, T h00,
+                                          C2<T> (&out)[4]) {
+  PackRec<T, GRAD> ra, rb;
+  auto arrived = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  C2<T> hmm = {h00, T(0)}, h, hp;
+  auto step = [&](const PackRec<T, GRAD>& r) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int x = 0; x < (GRAD ? 4 : 1); x++) {
+      out[x].re = fma(r.c[4 * x], h.re, fma(r.c[4 * x + 1], h.im, out[x].re));
+      out[x].im = fma(r.c[4 * x + 2], h.re, fma(r.c[4 * x + 3], h.im, out[x].im));
+    }
+    const T br = r.b * rho;
+    C2<T> hn;
+    hn.re = fma(zz, h.re, -(br * hp.re));
+    hn.im = fma(zz, h.im, -(br * hp.im));
+    hp = h;
+    h = hn;
+  };
+  ra.load(pk);
+  int e = 0;
+  for (int a = 0; a <= pd; a++) {
+    if (a > 0) hmm = cmul(w, hmm);
+    h = hmm;
+    hp = {T(0), T(0)};
+    for (const int end = e + pack_col(pd, a); e < end; e += 2) {
+      const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane(e);
+      const T* __restrict__ o = pk + (size_t)kPackEntry * u;
+      arrived();
+      rb.load(o + kPackEntry);
+      step(ra);
+      arrived();
+      ra.load(o + 2 * kPackEntry);
+      step(rb);
+    }
+  }
 }
 
-// One workgroup per L2P work item (box, kind, first point); the loops over
-// the packed entries are wave uniform, so the entries are scalar loads.
+// One wave per L2P work item (box, kind, first point); the walk over the pack
+// is wave uniform.
 template <typename T>
-__global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const double* __restrict__ fac, const T* __restrict__ pack,
+__global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const T* __restrict__ pack,
                                                const double* __restrict__ spos, const double* __restrict__ tpos,
                                                int wpot0, int wfld0, int wpot1, int wfld1,
                                                double* __restrict__ pot0, double* __restrict__ fld0,
                                                double* __restrict__ pot1, double* __restrict__ fld1) {
   const int p = P.p;
-  const int H = (p + 1) * (p + 2) / 2;
-  FacLayout L(p);
   // one work item (64 points) per wave
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
   if (w >= P.n_l2pi) return;
   const int ib = P.l2p_items[3 * w], kind = P.l2p_items[3 * w + 1], start = P.l2p_items[3 * w + 2];
   if (ib < 0) return;   // padding item
   const int b = P.l2p_boxes[ib];
-  const T* pk = pack + (size_t)ib * H * 16;
+  const T* pk = pack + (size_t)ib * pack_entries(p) * kPackEntry;
   const T ih = (T)P.inv_side[P.level[b]];
   const double cx = P.center[3 * b], cy = P.center[3 * b + 1], cz = P.center[3 * b + 2];
   const int wp = kind ? wpot1 : wpot0, wf = kind ? wfld1 : wfld0;
@@ -531,39 +517,13 @@ __global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const double* __restric
   }
   const T ux = (T)((x - cx) * (double)ih), uy = (T)((y - cy) * (double)ih), uz = (T)((z - cz) * (double)ih);
   const T r2 = ux * ux + uy * uy + uz * uz;
-  C2<T> pv = {0, 0}, gz = {0, 0}, gu = {0, 0}, gd = {0, 0};
-  C2<T> hmm = {T(1), T(0)};
-  const T* c = pk;
-  for (int a = 0; a <= p; a++) {
-    if (a > 0) {
-      const T f = (T)fac[L.MM + a];
-      const C2<T> v = {-ux * f, -uy * f};
-      hmm = cmul(v, hmm);
-    }
-    C2<T> h0 = hmm, h1 = hmm;
-    for (int n = a; n <= p; n++, c += 16) {
-      C2<T> h;
-      if (n == a) {
-        h = hmm;
-      } else if (n == a + 1) {
-        const T g = (T)fac[L.M1 + a] * uz;
-        h = {g * hmm.re, g * hmm.im};
-        h1 = h;
-      } else {
-        const T aa = (T)(2 * n - 1) * uz, bq = (T)fac[L.RA + hidx(n, a)] * r2, cc = (T)fac[L.RB + hidx(n, a)];
-        h = {(aa * h1.re - bq * h0.re) * cc, (aa * h1.im - bq * h0.im) * cc};
-        h0 = h1;
-        h1 = h;
-      }
-      pack_fma(pv, c, h);
-      if (wf) {
-        pack_fma(gz, c + 4, h);
-        pack_fma(gu, c + 8, h);
-        pack_fma(gd, c + 12, h);
-      }
-    }
-  }
+  C2<T> out[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+  if (wf)
+    pack_walk<T, true>(pk, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
+  else
+    pack_walk<T, false>(pk, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
   if (!active) return;
+  const C2<T> pv = out[0], gz = out[1], gu = out[2], gd = out[3];
   const size_t id = (size_t)(n0 + i);
   double* po = kind ? pot1 : pot0;
   double* fo = kind ? fld1 : fld0;
@@ -578,36 +538,20 @@ __global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const double* __restric
   }
 }
 
-// ---------------------------------------------------------------------------
-// M2P (list 3) from packed multipoles.  For every box whose multipole is
-// evaluated, the multipole M and the three derived expansions of the
-// gradient over the irregular harmonics of degree n <= p+1,
-//   Gz(n,m) = AS(n-1,m)   M(n-1,m),
-//   Gu(n,m) = BS(n-1,m-1) M(n-1,m-1),
-//   Gd(n,m) = CS(n-1,m+1) M(n-1,m+1)      (zero where (n-1, m') is outside),
-// are stored per half-table entry (n, a >= 0) in the order of the walk
-// (column a, then n = a..pd, pd = p+1 with the gradient, else p), 8 complex
-// values as for L2P.  One wave evaluates 64 points of a box against a slice
-// of its list 3 (src/laprouts3d.f:2432 l3dmpevalall_trunc): per source box
-// the irregular harmonics S_n^a(u) by the column recurrence of
-// irregular_column, four complex products per harmonic, scaled
-// by 1/h (potential) and 1/h^2 (gradient) of the source box; the slice's sums
-// go to `partial` and k_slice_reduce adds the slices in order.
-// ---------------------------------------------------------------------------
 template <typename T>
 __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* __restrict__ mp,
                            const int* __restrict__ boxes, const int* __restrict__ offs, int nbox, int grad,
                            T* __restrict__ pack) {
   const int p = P.p, K = P.K;
   const int pd = grad ? p + 1 : p;
-  const int Hd = (pd + 1) * (pd + 2) / 2;
+  const int NE = pack_entries(pd);
   FacLayout L(p);
-  const size_t total = (size_t)nbox * Hd;
+  const size_t total = (size_t)nbox * NE;
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(t / Hd), w = (int)(t - (size_t)i * Hd);
-    int a = 0;
-    while (a < pd && walk_index(pd, a + 1, a + 1) <= w) a++;
-    const int n = a + (w - walk_index(pd, a, a));
+    const int i = (int)(t / NE), w = (int)(t - (size_t)i * NE);
+    int a = 0, r = w;
+    while (r >= pack_col(pd, a)) { r -= pack_col(pd, a); a++; }
+    const int n = a + r;
     const T* E = mp + 2 * (size_t)boxes[i] * K;
     auto ef = [&](int off, int n1, int m1, int e) -> T {  // factor * E(n1, m1), zero outside
       if (n1 < 0 || m1 > n1 || m1 < -n1) return T(0);
@@ -621,7 +565,7 @@ __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
       v[1] = E[2 * eidx(n, a) + 1];
       if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
     }
-    if (grad && n >= 1) {
+    if (grad && n >= 1 && n <= pd) {
       const int n1 = n - 1;
       for (int sgn = 0; sgn < (a > 0 ? 2 : 1); sgn++) {
         const int m = sgn ? -a : a;
@@ -632,22 +576,22 @@ __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
         }
       }
     }
-    T* o = pack + 16 * ((size_t)offs[i] + w);
-#pragma unroll
-    for (int e = 0; e < 16; e++) o[e] = v[e];
+    pack_store(pack + kPackEntry * ((size_t)offs[i] + w), v, n <= pd ? (T)fac[L.GN + hidx(n, a)] : T(0),
+               n <= pd ? (T)fac[L.BT + hidx(n + 1, a)] : T(0));
   }
 }
 
+// M2P: one wave per 64 points of a box and slice of its list 3, the sums
+// scaled by 1/h (potential) and 1/h^2 (gradient) of each source box; the
+// slice's sums go to `partial` and k_slice_reduce adds the slices in order.
 // items: 5 ints per wave (box, kind, first point, first and end position in
 // list 3); slot[j]: the pack offset (in entries) of source box j
 template <typename T>
-__global__ __launch_bounds__(256) void k_m2p_eval(DevPlan P, const double* __restrict__ fac, const T* __restrict__ pack,
+__global__ __launch_bounds__(256) void k_m2p_eval(DevPlan P, const T* __restrict__ pack,
                                                   const int* __restrict__ slot, const int* __restrict__ items, int nitems,
                                                   int grad, const double* __restrict__ spos,
                                                   const double* __restrict__ tpos, double* __restrict__ partial) {
-  const int p = P.p;
-  const int pd = grad ? p + 1 : p;
-  FacLayout L(p);
+  const int pd = grad ? P.p + 1 : P.p;
   const int w = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
   if (w >= nitems) return;
   const int lane = (int)(threadIdx.x & 63);
@@ -674,44 +618,20 @@ __global__ __launch_bounds__(256) void k_m2p_eval(DevPlan P, const double* __res
     const T uz = active ? (T)((z - P.center[3 * j + 2]) * ihd) : T(1);
     const T r2 = ux * ux + uy * uy + uz * uz;
     const T ir2 = T(1) / r2, ir = sqrt(ir2);
-    C2<T> pv = {0, 0}, gz = {0, 0}, gu = {0, 0}, gd = {0, 0};
-    C2<T> hmm = {ir, T(0)};
-    const T* c = pack + 16 * (size_t)slot[j];
-    for (int a = 0; a <= pd; a++) {
-      if (a > 0) {
-        const T f = (T)fac[L.MM + a] * ir2;
-        const C2<T> v = {-ux * f, -uy * f};
-        hmm = cmul(v, hmm);
-      }
-      C2<T> h0 = hmm, h1 = hmm;
-      for (int n = a; n <= pd; n++, c += 16) {
-        C2<T> h;
-        if (n == a) {
-          h = hmm;
-        } else if (n == a + 1) {
-          const T g = (T)fac[L.M1 + a] * uz * ir2;
-          h = {g * hmm.re, g * hmm.im};
-          h1 = h;
-        } else {
-          const T aa = (T)(2 * n - 1) * uz, bq = (T)fac[L.RA + hidx(n, a)], cc = (T)fac[L.RB + hidx(n, a)] * ir2;
-          h = {(aa * h1.re - bq * h0.re) * cc, (aa * h1.im - bq * h0.im) * cc};
-          h0 = h1;
-          h1 = h;
-        }
-        pack_fma(pv, c, h);
-        if (grad) {
-          pack_fma(gz, c + 4, h);
-          pack_fma(gu, c + 8, h);
-          pack_fma(gd, c + 12, h);
-        }
-      }
-    }
+    C2<T> out[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
+    const T* c = pack + kPackEntry * (size_t)slot[j];
+    if (grad)
+      pack_walk<T, true>(c, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
+    else
+      pack_walk<T, false>(c, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
     // pot = sum M S(u)/h ; the gradient w.r.t. x adds another 1/h
     const T sg = ih * ih;
-    acc[0] += (double)(pv.re * ih); acc[1] += (double)(pv.im * ih);
-    acc[2] += (double)(gz.re * sg); acc[3] += (double)(gz.im * sg);
-    acc[4] += (double)(gu.re * sg); acc[5] += (double)(gu.im * sg);
-    acc[6] += (double)(gd.re * sg); acc[7] += (double)(gd.im * sg);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      const T sc = v == 0 ? ih : sg;
+      acc[2 * v] += (double)(out[v].re * sc);
+      acc[2 * v + 1] += (double)(out[v].im * sc);
+    }
   }
   double* o = partial + 8 * ((size_t)w * 64 + lane);
 #pragma unroll

@@ -4,6 +4,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <utility>
 #include <vector>
 
@@ -161,18 +162,21 @@ inline void build_plan_far(const Octree& t, const Flags& f, Flat& F, PlanOffsets
   }
   O.l3o = F.i(t.list[2].off); O.l3i = F.i(t.list[2].idx);
   O.l4o = F.i(t.list[3].off); O.l4i = F.i(t.list[3].idx);
-  std::vector<int> l2p, m2p, p2l;
+  std::vector<int> l2p, m2p, p2l, p2l_src(nb, 0);
   for (int b = 0; b < nb; b++) {
     const bool leaf = t.nchild[b] == 0;
     const bool has_pts = (want_src && t.nsrc[b] > 0) || (want_trg && t.ntrg[b] > 0);
     if (leaf && t.level[b] >= 2 && has_pts) l2p.push_back(b);
     if (t.list[2].count(b) > 0 && has_pts) m2p.push_back(b);
     if (t.list[3].count(b) > 0) {
-      bool any = false;
-      for (int k = t.list[3].off[b]; k < t.list[3].off[b + 1]; k++) any |= t.nsrc[t.list[3].idx[k]] > 0;
-      if (any) p2l.push_back(b);
+      for (int k = t.list[3].off[b]; k < t.list[3].off[b + 1]; k++) p2l_src[b] += t.nsrc[t.list[3].idx[k]];
+      if (p2l_src[b] > 0) p2l.push_back(b);
     }
   }
+  // P2L: one workgroup per box, the boxes with the most list-4 sources first
+  // (on clustered points the longest has four times the mean), so that no
+  // long one starts last
+  std::stable_sort(p2l.begin(), p2l.end(), [&](int a, int b) { return p2l_src[a] > p2l_src[b]; });
   O.l2p = F.i(l2p); O.n_l2p = (int)l2p.size();
   {
     // L2P work items (position in the L2P list, kind, first point): one

@@ -227,9 +227,10 @@ void build_tables(int p, double eps, HostTables& H) {
 // the kernel-independent half of the translation tables.
 void build_fac_table(int p, std::vector<double>& fac) {
   const int P = p + 2, Hh = P * (P + 1) / 2, E = P * P;
-  fac.assign((size_t)2 * (P + 1) + 2 * Hh + 6 * E, 0.0);
+  fac.assign((size_t)2 * (P + 1) + 2 * Hh + 6 * E + (Hh + P + 1) + Hh, 0.0);
   const int MM = 0, M1 = MM + P + 1, RA = M1 + P + 1, RB = RA + Hh, AR = RB + Hh, BR = AR + E,
-            CR = BR + E, AS = CR + E, BS = AS + E, CS = BS + E;
+            CR = BR + E, AS = CR + E, BS = AS + E, CS = BS + E, BT = CS + E,
+            GN = BT + Hh + P + 1;
   for (int m = 1; m <= P; m++) fac[MM + m] = std::sqrt((2.0 * m - 1.0) / (2.0 * m));
   for (int m = 0; m <= P; m++) fac[M1 + m] = std::sqrt(2.0 * m + 1.0);
   for (int n = 0; n < P; n++)
@@ -238,6 +239,18 @@ void build_fac_table(int p, std::vector<double>& fac) {
       fac[RA + h] = (n >= m + 2) ? std::sqrt((n + m - 1.0) * (n - m - 1.0)) : 0.0;
       fac[RB + h] = (n > m) ? 1.0 / std::sqrt((double)(n - m) * (n + m)) : 0.0;
     }
+  for (int n = 0; n <= P; n++)
+    for (int m = 0; m <= n; m++)
+      fac[BT + n * (n + 1) / 2 + m] =
+          (n > m) ? (double)((n - 1 - m) * (n - 1 + m)) / ((2.0 * n - 1.0) * (2.0 * n - 3.0)) : 0.0;
+  for (int m = 0; m < P; m++) {
+    double g = 1.0;
+    for (int k = 1; k <= m; k++) g *= fac[MM + k];
+    for (int n = m; n < P; n++) {
+      if (n > m) g *= (2.0 * n - 1.0) / std::sqrt((double)(n - m) * (n + m));
+      fac[GN + n * (n + 1) / 2 + m] = g;
+    }
+  }
   for (int n = 0; n < P; n++)
     for (int m = -n; m <= n; m++) {
       int e = n * n + n + m;
