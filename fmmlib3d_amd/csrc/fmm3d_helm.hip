@@ -27,126 +27,157 @@ namespace fmm3d {
 
 namespace {
 
-// Host tables and their device copies, cached for repeated calls with the
-// same wavenumber, root box, depth and tolerance.
+// The tables in this context's arena: the geometry (rotations, phases, factors)
+// of one order, the Gaunt integrals, and the orders and coaxial operators of
+// one wavenumber, root box, depth and tolerance.  Each part is replaced when a
+// call needs another.
 struct HelmCache {
   HelmHostTables H;
-  std::vector<int> I;
-  std::vector<double> D;
-  std::vector<long> Lg;
-  size_t o_offrot = 0, o_offdist = 0, o_octrot = 0, o_plev = 0, o_ptrunc = 0;
-  size_t o_fac = 0, o_offph = 0, o_octph = 0, o_rot = 0, o_sclev = 0, o_z = 0;
-  size_t o_rotoff = 0, o_coax = 0;
+  bool valid = false;                        // the operators on the device are H's
+  std::shared_ptr<const HostTables> geo;     // the geometry on the device
+  std::shared_ptr<const Gaunt> gaunt;        // the integrals on the device
+  size_t gI = 0, gD = 0, gL = 0;             // geometry sizes
+  size_t o_offrot = 0, o_offdist = 0, o_octrot = 0, o_gri = 0, o_grc = 0, o_gzi = 0, o_gzo = 0;
+  size_t o_fac = 0, o_offph = 0, o_octph = 0, o_rot = 0, o_rothalf = 0;
+  size_t o_rotoff = 0, o_rothalf_off = 0;
+  size_t cI = 0, cD = 0, cL = 0, cZ = 0;     // per-call sizes
+  size_t o_plev = 0, o_ptrunc = 0, o_sclev = 0, o_coax = 0, o_ztoff = 0, o_zt = 0;
   int m2m_base = 0, l2l_base = 0;
-  // grouped M2L: rotation tiles and items at pmax, complex coaxial tiles
-  size_t o_rothalf = 0, o_rothalf_off = 0, o_gri = 0, o_grc = 0, o_gzi = 0, o_gzo = 0, o_zt = 0, o_ztoff = 0;
   bool grouped_m2l = false;   // every list-2 order fits its table's tiles
 };
 
+template <typename V>
+size_t put_aligned(std::vector<V>& to, const std::vector<V>& v, size_t a) {
+  const size_t o = to.size();
+  to.insert(to.end(), v.begin(), v.end());
+  while (to.size() % a) to.push_back(V(0));
+  return o;
+}
+
+void helm_upload_geometry(Context& ctx, HelmCache& c, const std::shared_ptr<const HostTables>& g) {
+  c.geo.reset();
+  std::vector<int> I;
+  std::vector<double> D;
+  std::vector<long> L;
+  c.o_offrot = put_aligned(I, g->off_rot, 16);
+  c.o_offdist = put_aligned(I, g->off_dist, 16);
+  c.o_octrot = put_aligned(I, g->oct_rot, 16);
+  c.o_gri = put_aligned(I, g->grp_ritems, 16);
+  c.o_grc = put_aligned(I, g->grp_rcount, 16);
+  c.o_gzi = put_aligned(I, g->grp_zitems, 16);
+  c.o_gzo = put_aligned(I, g->grp_zoff, 16);
+  c.o_fac = put_aligned(D, g->fac, 8);
+  c.o_offph = put_aligned(D, g->off_phase, 8);
+  c.o_octph = put_aligned(D, g->oct_phase, 8);
+  c.o_rot = put_aligned(D, g->rot, 8);
+  c.o_rothalf = put_aligned(D, g->rot_half, 8);
+  c.o_rotoff = put_aligned(L, g->rot_off, 1);
+  c.o_rothalf_off = put_aligned(L, g->rot_half_off, 1);
+  c.gI = I.size(); c.gD = D.size(); c.gL = L.size();
+  void* di = ctx.arena.get("hgeo_i", I.size() * sizeof(int));
+  void* dd = ctx.arena.get("hgeo_d", D.size() * sizeof(double));
+  void* dl = ctx.arena.get("hgeo_l", L.size() * sizeof(long));
+  FMM_HIP(hipMemcpyAsync(di, I.data(), I.size() * sizeof(int), hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipMemcpyAsync(dd, D.data(), D.size() * sizeof(double), hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipMemcpyAsync(dl, L.data(), L.size() * sizeof(long), hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipStreamSynchronize(ctx.stream));
+  c.geo = g;
+}
+
+void helm_upload_gaunt(Context& ctx, HelmCache& c, const std::shared_ptr<const Gaunt>& g) {
+  c.gaunt.reset();
+  void* dg = ctx.arena.get("hgaunt_g", g->g.size() * sizeof(double));
+  void* dof = ctx.arena.get("hgaunt_o", g->off.size() * sizeof(long));
+  FMM_HIP(hipMemcpyAsync(dg, g->g.data(), g->g.size() * sizeof(double), hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipMemcpyAsync(dof, g->off.data(), g->off.size() * sizeof(long), hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipStreamSynchronize(ctx.stream));
+  c.gaunt = g;
+}
+
 HelmCache* helm_tables(Context& ctx, cplx zk, double size, int nlev, double eps, int& ier) {
   ier = 0;
-  auto* c = static_cast<HelmCache*>(ctx.helm_tables.get());
-  const bool hit = c && c->H.zk == zk && c->H.size == size && c->H.nlev == nlev && c->H.eps == eps;
-  if (!hit) {
-    auto nc = std::make_shared<HelmCache>();
-    if (!build_helm_tables(zk, size, nlev, eps, nc->H)) {
-      ier = 16;
-      return nullptr;
-    }
-    const HelmHostTables& H = nc->H;
-    auto& I = nc->I;
-    auto& D = nc->D;
-    auto& Lg = nc->Lg;
-    auto put_i = [&](const std::vector<int>& v) { size_t o = I.size(); I.insert(I.end(), v.begin(), v.end()); while (I.size() % 16) I.push_back(0); return o; };
-    auto put_d = [&](const std::vector<double>& v) { size_t o = D.size(); D.insert(D.end(), v.begin(), v.end()); while (D.size() % 8) D.push_back(0.0); return o; };
-    nc->o_offrot = put_i(H.geo.off_rot);
-    nc->o_offdist = put_i(H.geo.off_dist);
-    nc->o_octrot = put_i(H.geo.oct_rot);
-    nc->o_plev = put_i(H.plev);
-    nc->o_ptrunc = put_i(H.ptrunc);
-    nc->o_fac = put_d(H.geo.fac);
-    nc->o_offph = put_d(H.geo.off_phase);
-    nc->o_octph = put_d(H.geo.oct_phase);
-    nc->o_rot = put_d(H.geo.rot);
-    nc->o_sclev = put_d(H.sclev);
-    nc->o_z = put_d(H.z);
-    nc->o_rotoff = 0;
-    Lg = H.geo.rot_off;
-    nc->o_coax = Lg.size();
-    const int nd = H.geo.ndist;
-    auto put_desc = [&](const CoaxDesc& d) { Lg.push_back(d.base); Lg.push_back(d.pin); Lg.push_back(d.pout); };
-    for (const auto& d : H.m2l) put_desc(d);
-    nc->m2m_base = (nlev + 1) * nd;
-    for (const auto& d : H.m2m) put_desc(d);
-    nc->l2l_base = nc->m2m_base + nlev + 1;
-    for (const auto& d : H.l2l) put_desc(d);
-    // grouped M2L: the geometry tables' rotation tiles and work items (order
-    // pmax), and each M2L table's coaxial blocks as complex 4x4 tiles per
-    // order am: [row block of n - am][column block of l - am], 16 real parts
-    // then 16 imaginary parts of [row][column]
-    {
-      const int P1 = H.pmax + 1;
-      nc->o_gri = put_i(H.geo.grp_ritems);
-      nc->o_grc = put_i(H.geo.grp_rcount);
-      nc->o_gzi = put_i(H.geo.grp_zitems);
-      nc->o_gzo = put_i(H.geo.grp_zoff);
-      nc->o_rothalf = put_d(H.geo.rot_half);
-      const size_t ntab = H.m2l.size();
-      std::vector<long> zt_off(ntab * P1, 0);
-      std::vector<double> zt;
-      bool ok = true;
-      const size_t nzc = H.z.size() / 2;   // complex entries
-      for (size_t t = 0; t < ntab; t++) {
-        // M2L runs from level 2 on; the descriptors of levels 0 and 1 are empty
-        if (t < 2 * (size_t)H.geo.ndist) continue;
-        const CoaxDesc& d = H.m2l[t];
-        if (d.pin != d.pout || d.pout < 0 || d.pout > H.pmax) { ok = false; continue; }
-        const int pz = d.pout;
-        // the table's last block ends inside the coaxial data
-        if ((size_t)(d.base + coax_block(pz, pz, pz) + 1) > nzc) { ok = false; continue; }
-        for (int am = 0; am <= pz; am++) {
-          const int nb4 = (pz - am) / 4 + 1;
-          const size_t b0 = zt.size();
-          zt_off[t * P1 + am] = (long)b0;
-          zt.resize(b0 + 32 * (size_t)nb4 * nb4, 0.0);
-          const long mb = d.base + coax_block(am, d.pin, d.pout);
-          for (int n = am; n <= pz; n++)
-            for (int l = am; l <= pz; l++) {
-              const long ix = mb + (long)(l - am) * (d.pin + 1 - am) + (n - am);
-              const int rr = n - am, cc = l - am;
-              const size_t tile = b0 + 32 * ((size_t)(rr / 4) * nb4 + cc / 4);
-              zt[tile + (rr % 4) * 4 + cc % 4] = H.z[2 * ix];
-              zt[tile + 16 + (rr % 4) * 4 + cc % 4] = H.z[2 * ix + 1];
-            }
-        }
-      }
-      // every list-2 order must lie within its table's tiles
-      const int nd2 = H.geo.ndist;
-      for (int l = 2; l <= nlev && ok; l++)
-        for (int code = 0; code < 343 && ok; code++) {
-          const int pt = H.ptrunc[(size_t)l * 343 + code];
-          if (pt <= 0) continue;
-          const CoaxDesc& d = H.m2l[(size_t)l * nd2 + H.geo.off_dist[code]];
-          ok = d.pin == d.pout && pt <= d.pout;
-        }
-      nc->grouped_m2l = ok;
-      nc->o_zt = put_d(zt);
-      nc->o_rothalf_off = Lg.size();
-      Lg.insert(Lg.end(), H.geo.rot_half_off.begin(), H.geo.rot_half_off.end());
-      nc->o_ztoff = Lg.size();
-      Lg.insert(Lg.end(), zt_off.begin(), zt_off.end());
-    }
-    void* di = ctx.arena.get("htab_i", I.size() * sizeof(int));
-    void* dd = ctx.arena.get("htab_d", D.size() * sizeof(double));
-    void* dl = ctx.arena.get("htab_l", Lg.size() * sizeof(long));
-    FMM_HIP(hipMemcpyAsync(di, I.data(), I.size() * sizeof(int), hipMemcpyHostToDevice, ctx.stream));
-    FMM_HIP(hipMemcpyAsync(dd, D.data(), D.size() * sizeof(double), hipMemcpyHostToDevice, ctx.stream));
-    FMM_HIP(hipMemcpyAsync(dl, Lg.data(), Lg.size() * sizeof(long), hipMemcpyHostToDevice, ctx.stream));
-    FMM_HIP(hipStreamSynchronize(ctx.stream));
-    ctx.helm_tables = nc;
-    c = nc.get();
+  if (!ctx.helm_tables) ctx.helm_tables = std::make_shared<HelmCache>();
+  HelmCache& c = *static_cast<HelmCache*>(ctx.helm_tables.get());
+  if (c.valid && c.H.zk == zk && c.H.size == size && c.H.nlev == nlev && c.H.eps == eps) return &c;
+  c.valid = false;
+  if (!plan_helm_tables(zk, size, nlev, eps, c.H)) {
+    ier = 16;
+    return nullptr;
   }
-  return c;
+  const HelmHostTables& H = c.H;
+  if (c.geo != H.geo) helm_upload_geometry(ctx, c, H.geo);
+  const auto gaunt = gaunt_for(H.pmax);
+  if (c.gaunt != gaunt) helm_upload_gaunt(ctx, c, gaunt);
+  const int nd = H.geo->ndist, P1 = H.pmax + 1;
+  std::vector<int> I;
+  std::vector<double> D;
+  std::vector<long> L;
+  c.o_plev = put_aligned(I, H.plev, 16);
+  c.o_ptrunc = put_aligned(I, H.ptrunc, 16);
+  c.o_sclev = put_aligned(D, H.sclev, 8);
+  const size_t o_series = put_aligned(D, H.series, 8);
+  c.o_coax = 0;
+  auto put_desc = [&](const CoaxDesc& d) { L.push_back(d.base); L.push_back(d.pin); L.push_back(d.pout); };
+  for (const auto& d : H.m2l) put_desc(d);
+  c.m2m_base = (nlev + 1) * nd;
+  for (const auto& d : H.m2m) put_desc(d);
+  c.l2l_base = c.m2m_base + nlev + 1;
+  for (const auto& d : H.l2l) put_desc(d);
+  // grouped M2L: each M2L operator also as complex 4x4 tiles per order am,
+  // [row block of n - am][column block of l - am], 16 real parts then 16
+  // imaginary parts of [row][column]; every list-2 order must lie within its
+  // table's tiles
+  std::vector<long> zt_off(H.m2l.size() * P1, 0);
+  long nt = 0;
+  int mmax = 0;
+  for (const CoaxJob& J : H.jobs) {
+    mmax = std::max(mmax, std::min(J.pin, J.pout));
+    if (J.m2l < 0) continue;
+    for (int am = 0; am <= J.pout; am++) {
+      zt_off[(size_t)J.m2l * P1 + am] = nt;
+      const long nb4 = (J.pout - am) / 4 + 1;
+      nt += 32 * nb4 * nb4;
+    }
+  }
+  bool ok = true;
+  for (int l = 2; l <= nlev && ok; l++)
+    for (int code = 0; code < 343 && ok; code++) {
+      const int pt = H.ptrunc[(size_t)l * 343 + code];
+      if (pt <= 0) continue;
+      const CoaxDesc& d = H.m2l[(size_t)l * nd + H.geo->off_dist[code]];
+      ok = d.pin == d.pout && pt <= d.pout;
+    }
+  c.grouped_m2l = ok;
+  c.o_ztoff = put_aligned(L, zt_off, 1);
+  c.o_zt = (2 * (size_t)H.nz + 7) / 8 * 8;
+  c.cI = I.size(); c.cD = D.size(); c.cL = L.size();
+  c.cZ = c.o_zt + (size_t)nt;
+  // small enough to go through one pinned buffer (the call before this one on
+  // the context has finished with it)
+  const size_t bI = I.size() * sizeof(int), bD = D.size() * sizeof(double), bL = L.size() * sizeof(long),
+               bJ = H.jobs.size() * sizeof(CoaxJob);
+  char* h = (char*)ctx.arena.get_host("htab_h", bD + bL + bJ + bI);
+  std::memcpy(h, D.data(), bD);
+  std::memcpy(h + bD, L.data(), bL);
+  std::memcpy(h + bD + bL, H.jobs.data(), bJ);
+  std::memcpy(h + bD + bL + bJ, I.data(), bI);
+  double* dd = (double*)ctx.arena.get("htab_d", bD);
+  long* dl = (long*)ctx.arena.get("htab_l", bL);
+  CoaxJob* dj = (CoaxJob*)ctx.arena.get("htab_j", bJ);
+  int* di = (int*)ctx.arena.get("htab_i", bI);
+  double* dz = (double*)ctx.arena.get("htab_z", c.cZ * sizeof(double));
+  FMM_HIP(hipMemcpyAsync(dd, h, bD, hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipMemcpyAsync(dl, h + bD, bL, hipMemcpyHostToDevice, ctx.stream));
+  if (bJ) FMM_HIP(hipMemcpyAsync(dj, h + bD + bL, bJ, hipMemcpyHostToDevice, ctx.stream));
+  FMM_HIP(hipMemcpyAsync(di, h + bD + bL + bJ, bI, hipMemcpyHostToDevice, ctx.stream));
+  if (!H.jobs.empty())
+    hipLaunchKernelGGL(k_coax, dim3((unsigned)H.jobs.size(), (unsigned)(mmax + 1)), dim3(256), 0, ctx.stream, dj, dd + o_series,
+                       (const long*)ctx.arena.get("hgaunt_o", c.gaunt->off.size() * sizeof(long)),
+                       (const double*)ctx.arena.get("hgaunt_g", c.gaunt->g.size() * sizeof(double)), c.gaunt->P + 1,
+                       dl + c.o_ztoff, P1, dz, dz + c.o_zt);
+  FMM_HIP(hipGetLastError());
+  c.valid = true;
+  return &c;
 }
 
 template <typename TN, bool CHG, bool DIP, bool FLD>
@@ -254,23 +285,27 @@ int helm_solve(Context& ctx, const LapCall& c) {
   double* dD = (double*)ctx.arena.get("plan_d", FA.D.size() * sizeof(double));
   FMM_HIP(hipMemcpyAsync(dD, hD, FA.D.size() * sizeof(double), hipMemcpyHostToDevice, s));
   DevPlan P = make_devplan(tree, pmax, O, dI, dD);
-  const int* ti = (const int*)ctx.arena.get("htab_i", HC->I.size() * sizeof(int));
-  const double* td = (const double*)ctx.arena.get("htab_d", HC->D.size() * sizeof(double));
-  const long* tl = (const long*)ctx.arena.get("htab_l", HC->Lg.size() * sizeof(long));
+  const int* gi = (const int*)ctx.arena.get("hgeo_i", HC->gI * sizeof(int));
+  const double* gd = (const double*)ctx.arena.get("hgeo_d", HC->gD * sizeof(double));
+  const long* gl = (const long*)ctx.arena.get("hgeo_l", HC->gL * sizeof(long));
+  const int* ti = (const int*)ctx.arena.get("htab_i", HC->cI * sizeof(int));
+  const double* td = (const double*)ctx.arena.get("htab_d", HC->cD * sizeof(double));
+  const long* tl = (const long*)ctx.arena.get("htab_l", HC->cL * sizeof(long));
+  const double* tz = (const double*)ctx.arena.get("htab_z", HC->cZ * sizeof(double));
   DevTables Tb{};
   Tb.p = pmax;
-  Tb.off_rot = ti + HC->o_offrot; Tb.off_dist = ti + HC->o_offdist; Tb.oct_rot = ti + HC->o_octrot;
-  Tb.fac = td + HC->o_fac; Tb.off_phase = td + HC->o_offph; Tb.oct_phase = td + HC->o_octph;
-  Tb.rot = td + HC->o_rot; Tb.rot_off = tl + HC->o_rotoff;
+  Tb.off_rot = gi + HC->o_offrot; Tb.off_dist = gi + HC->o_offdist; Tb.oct_rot = gi + HC->o_octrot;
+  Tb.fac = gd + HC->o_fac; Tb.off_phase = gd + HC->o_offph; Tb.oct_phase = gd + HC->o_octph;
+  Tb.rot = gd + HC->o_rot; Tb.rot_off = gl + HC->o_rotoff;
   HelmDev Hd;
   Hd.kre = zk.real(); Hd.kim = zk.imag();
-  Hd.nd = H.geo.ndist;
+  Hd.nd = H.geo->ndist;
   Hd.plev = ti + HC->o_plev; Hd.sclev = td + HC->o_sclev; Hd.ptrunc = ti + HC->o_ptrunc;
-  Hd.coax = tl + HC->o_coax; Hd.z = td + HC->o_z;
-  Hd.rot_half = td + HC->o_rothalf; Hd.rot_half_off = tl + HC->o_rothalf_off;
-  Hd.grp_ritems = ti + HC->o_gri; Hd.grp_rcount = ti + HC->o_grc;
-  Hd.grp_zitems = ti + HC->o_gzi; Hd.grp_zoff = ti + HC->o_gzo;
-  Hd.zt = td + HC->o_zt; Hd.zt_off = tl + HC->o_ztoff;
+  Hd.coax = tl + HC->o_coax; Hd.z = tz;
+  Hd.rot_half = gd + HC->o_rothalf; Hd.rot_half_off = gl + HC->o_rothalf_off;
+  Hd.grp_ritems = gi + HC->o_gri; Hd.grp_rcount = gi + HC->o_grc;
+  Hd.grp_zitems = gi + HC->o_gzi; Hd.grp_zoff = gi + HC->o_gzo;
+  Hd.zt = tz + HC->o_zt; Hd.zt_off = tl + HC->o_ztoff;
   const size_t nb = tree.nboxes;
   double* spos = (double*)ctx.arena.get("spos", sizeof(double) * 4 * (size_t)ns);
   double* str64 = (double*)ctx.arena.get("str64", sizeof(double) * 8 * (size_t)ns);

@@ -79,27 +79,45 @@ int sph_bessel_scaled(int n, cplx z, double sc, cplx* fj) {
   return 0;
 }
 
-// smallest j >= 2 with |j_j h_j| + |j_{j-1} h_{j-1}| < eps (|j_0 h_0| + |j_1 h_1|), as j+1
-static int h_decay(cplx z1, cplx z2, double sc, double eps) {
-  const int ntmax = 1000;
-  std::vector<cplx> hf(ntmax + 1), jf(ntmax + 1);
-  sph_hankel_scaled(ntmax, z1, sc, hf.data());
-  if (sph_bessel_scaled(ntmax, z2, sc, jf.data()) != 0) return 1;
-  const double x0 = std::abs(jf[0] * hf[0]) + std::abs(jf[1] * hf[1]);
-  for (int j = 2; j <= ntmax; j++) {
-    double x = std::abs(jf[j] * hf[j]) + std::abs(jf[j - 1] * hf[j - 1]);
-    if (x < eps * x0) return j + 1;
+// The decay rule of a box: smallest j >= 2 with |j_j h_j| + |j_{j-1} h_{j-1}| <
+// eps (|j_0 h_0| + |j_1 h_1|), as j+1, the Bessel functions at z2 (once per
+// box size) and the Hankel functions at z1 only as far as the rule looks.
+namespace {
+struct DecayRule {
+  static constexpr int ntmax = 1000;
+  double sc, eps;
+  bool ok;
+  std::vector<cplx> jf;
+  DecayRule(cplx z2, double sc_, double eps_) : sc(sc_), eps(eps_), jf(ntmax + 1) {
+    ok = sph_bessel_scaled(ntmax, z2, sc, jf.data()) == 0;
   }
-  return 1000;
+  int order(cplx z1) const {
+    if (!ok) return 1;
+    if (std::abs(z1) < 1.0e-15) return 1000;
+    // sph_hankel_scaled's recurrence
+    cplx h[2];
+    sph_hankel_scaled(1, z1, sc, h);
+    cplx hm = h[0], hc = h[1];
+    const double sc2 = sc * sc;
+    const cplx zinv = sc / z1;
+    const double x0 = std::abs(jf[0] * hm) + std::abs(jf[1] * hc);
+    double prev = std::abs(jf[1] * hc);
+    for (int j = 2; j <= ntmax; j++) {
+      const cplx hn = zinv * (2.0 * (j - 1) + 1.0) * hc - sc2 * hm;
+      hm = hc;
+      hc = hn;
+      const double cur = std::abs(jf[j] * hc);
+      if (cur + prev < eps * x0) return j + 1;
+      prev = cur;
+    }
+    return 1000;
+  }
+};
+DecayRule box_rule(double size, cplx zk, double eps) {
+  return DecayRule(zk * size * std::sqrt(3.0) / 2.0, std::min(std::abs(zk * size), 1.0), eps);
 }
-
-int helmholtz_nterms(double size, cplx zk, double eps) {
-  const double sc = std::min(std::abs(zk * size), 1.0);
-  return h_decay(zk * size * 1.5, zk * size * std::sqrt(3.0) / 2.0, sc, eps);
-}
-
-std::vector<int> helmholtz_itable(double size, cplx zk, double eps) {
-  const double sc = std::min(std::abs(zk * size), 1.0);
+int rule_nterms(const DecayRule& r, double size, cplx zk) { return r.order(zk * size * 1.5); }
+std::vector<int> rule_itable(const DecayRule& r, double size, cplx zk) {
   int nt[2][4][4];
   for (int ii = 2; ii <= 3; ii++)
     for (int jj = 0; jj <= 3; jj++)
@@ -109,7 +127,7 @@ std::vector<int> helmholtz_itable(double size, cplx zk, double eps) {
         if (dy > 0) dy -= 0.5;
         if (dz > 0) dz -= 0.5;
         double rr = std::sqrt(dx * dx + dy * dy + dz * dz);
-        nt[ii - 2][jj][kk] = h_decay(zk * size * rr, zk * size * std::sqrt(3.0) / 2.0, sc, eps);
+        nt[ii - 2][jj][kk] = r.order(zk * size * rr);
       }
   std::vector<int> t(343, 0);
   for (int i = -3; i <= 3; i++)
@@ -123,17 +141,14 @@ std::vector<int> helmholtz_itable(double size, cplx zk, double eps) {
       }
   return t;
 }
+}  // namespace
+
+int helmholtz_nterms(double size, cplx zk, double eps) { return rule_nterms(box_rule(size, zk, eps), size, zk); }
+std::vector<int> helmholtz_itable(double size, cplx zk, double eps) {
+  return rule_itable(box_rule(size, zk, eps), size, zk);
+}
 
 namespace {
-
-// Gaunt integrals G(n,s,l;m) for 0 <= m <= min(n,l), n,l <= P,
-// s = |n-l|, |n-l|+2, .., n+l, stored compactly; built once per P.
-struct Gaunt {
-  int P = -1;
-  std::vector<long> off;   // [(m*(P+1)+n)*(P+1)+l]
-  std::vector<double> g;
-  long at(int m, int n, int l) const { return off[((size_t)m * (P + 1) + n) * (P + 1) + l]; }
-};
 
 void gauss_legendre(int q, std::vector<double>& x, std::vector<double>& w) {
   x.resize(q);
@@ -175,11 +190,21 @@ void theta_table(int S, double x, double* y) {
     for (int m = 0; m <= n; m++) y[n * N + m] *= std::sqrt((2.0 * n + 1.0) / (4.0 * M_PI));
 }
 
-std::shared_ptr<const Gaunt> gaunt_for(int P) {
+}  // namespace
+
+std::shared_ptr<const Gaunt> gaunt_for(int pmax) {
+  constexpr size_t kKept = 6;
   static std::mutex mu;
-  static std::shared_ptr<const Gaunt> cached;
+  static std::vector<std::shared_ptr<const Gaunt>> kept;  // most recent last
+  const int P = (pmax + 3) / 4 * 4;
   std::lock_guard<std::mutex> lk(mu);
-  if (cached && cached->P >= P) return cached;
+  for (size_t i = 0; i < kept.size(); i++)
+    if (kept[i]->P == P) {
+      auto g = kept[i];
+      kept.erase(kept.begin() + (long)i);
+      kept.push_back(g);
+      return g;
+    }
   auto G = std::make_shared<Gaunt>();
   G->P = P;
   const int P1 = P + 1, S = 2 * P, Q = 2 * P + 2;
@@ -194,75 +219,96 @@ std::shared_ptr<const Gaunt> gaunt_for(int P) {
   G->g.assign(std::max(tot, 1L), 0.0);
   std::vector<double> x, w;
   gauss_legendre(Q, x, w);
+  // Theta at the nodes, the nodes of one (n, m <= P) or (s, 0) contiguous
   const int N = S + 1;
-  std::vector<double> th((size_t)Q * N * N);
-  for (int q = 0; q < Q; q++) theta_table(S, x[q], &th[(size_t)q * N * N]);
+  std::vector<double> one((size_t)N * N), th((size_t)P1 * P1 * Q), th0((size_t)N * Q);
+  for (int q = 0; q < Q; q++) {
+    theta_table(S, x[q], one.data());
+    for (int n = 0; n <= P; n++)
+      for (int m = 0; m <= n; m++) th[((size_t)n * P1 + m) * Q + q] = one[n * N + m];
+    for (int s = 0; s <= S; s++) th0[(size_t)s * Q + q] = one[s * N];
+  }
 #pragma omp parallel for schedule(dynamic, 1)
   for (int m = 0; m <= P; m++) {
     std::vector<double> prod(Q);
     for (int n = m; n <= P; n++)
       for (int l = m; l <= P; l++) {
-        for (int q = 0; q < Q; q++)
-          prod[q] = 2.0 * M_PI * w[q] * th[(size_t)q * N * N + n * N + m] * th[(size_t)q * N * N + l * N + m];
+        const double *tn = &th[((size_t)n * P1 + m) * Q], *tl = &th[((size_t)l * P1 + m) * Q];
+        for (int q = 0; q < Q; q++) prod[q] = 2.0 * M_PI * w[q] * tn[q] * tl[q];
         long o = G->off[((size_t)m * P1 + n) * P1 + l];
         for (int s = std::abs(n - l), k = 0; s <= n + l; s += 2, k++) {
+          const double* ts = &th0[(size_t)s * Q];
           double a = 0.0;
-          for (int q = 0; q < Q; q++) a += prod[q] * th[(size_t)q * N * N + s * N];
+#pragma omp simd reduction(+ : a)
+          for (int q = 0; q < Q; q++) a += prod[q] * ts[q];
           G->g[o + k] = a;
         }
       }
   }
-  cached = G;
-  return cached;
+  if (kept.size() >= kKept) kept.erase(kept.begin());
+  kept.push_back(G);
+  return G;
 }
 
-// mode 0: M2M (R|R), 1: M2L (S|R), 2: L2L (R|R); sigma = direction sign
-void coax(const Gaunt& G, int mode, double sigma, cplx zk, double d, double sc_in, double sc_out,
-          int pin, int pout, std::vector<double>& z, CoaxDesc& desc) {
-  desc.pin = pin;
-  desc.pout = pout;
-  desc.base = (long)(z.size() / 2);
-  const int S = pin + pout;
-  std::vector<cplx> f(S + 2);
-  const double base = (mode == 0) ? sc_out : sc_in;
-  if (mode == 1) sph_hankel_scaled(S, zk * d, base, f.data());
-  else sph_bessel_scaled(S, zk * d, base, f.data());
-  const int mtop = std::min(pin, pout);
-  const long total = coax_block(mtop + 1, pin, pout);
-  // powers used below: base^e for 0 <= e <= S, ratio^e for 0 <= e <= max(pin, pout)
-  std::vector<double> pb(S + 1, 1.0), pr(std::max(pin, pout) + 1, 1.0);
-  const double ratio = (mode == 0) ? sc_in / sc_out : (mode == 2 ? sc_out / sc_in : 1.0);
-  for (int e = 1; e <= S; e++) pb[e] = pb[e - 1] * base;
-  for (int e = 1; e < (int)pr.size(); e++) pr[e] = pr[e - 1] * ratio;
-  const size_t o0 = z.size();
-  z.resize(o0 + 2 * (size_t)total, 0.0);
-  for (int m = 0; m <= mtop; m++) {
-    const long mb = coax_block(m, pin, pout);
-    const int cols = pin + 1 - m;
-    for (int l = m; l <= pout; l++)
-      for (int n = m; n <= pin; n++) {
-        const long go = G.at(m, n, l);
-        cplx acc = 0.0;
-        for (int s = std::abs(n - l), k = 0; s <= n + l; s += 2, k++) {
-          double sg = (((l + s - n) / 2) & 1) ? -1.0 : 1.0;
-          if (sigma < 0 && (s & 1)) sg = -sg;
-          double c = 4.0 * M_PI * sg * std::sqrt((2.0 * s + 1.0) / (4.0 * M_PI)) * G.g[go + k];
-          double pw;
-          if (mode == 1) pw = pb[n + l - s];
-          else if (mode == 0) pw = pb[s - l + n] * pr[n];
-          else pw = pb[s - n + l] * pr[l];
-          acc += c * pw * f[s];
-        }
-        const size_t e = o0 + 2 * (size_t)(mb + (long)(l - m) * cols + (n - m));
-        z[e] = acc.real();
-        z[e + 1] = acc.imag();
+std::shared_ptr<const HostTables> geometry_for(int p) {
+  constexpr size_t kKept = 4;
+  static std::mutex mu;
+  static std::vector<std::shared_ptr<const HostTables>> kept;  // most recent last
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    for (size_t i = 0; i < kept.size(); i++)
+      if (kept[i]->p == p) {
+        auto g = kept[i];
+        kept.erase(kept.begin() + (long)i);
+        kept.push_back(g);
+        return g;
       }
   }
+  auto g = std::make_shared<HostTables>();
+  build_geometry_tables(p, *g);
+  std::lock_guard<std::mutex> lk(mu);
+  if (kept.size() >= kKept) kept.erase(kept.begin());
+  kept.push_back(g);
+  return g;
+}
+
+namespace {
+
+// adds one operator: its layout and its series
+void add_coax(HelmHostTables& H, int mode, int neg, double d, double sc_in, double sc_out, int pin, int pout, int m2l,
+              CoaxDesc& desc) {
+  CoaxJob J;
+  J.base = H.nz;
+  J.series = (long)H.series.size();
+  J.pin = pin;
+  J.pout = pout;
+  J.mode = mode;
+  J.neg = neg;
+  J.m2l = m2l;
+  desc.pin = pin;
+  desc.pout = pout;
+  desc.base = J.base;
+  H.nz += coax_block(std::min(pin, pout) + 1, pin, pout);
+  const int S = pin + pout, E = std::max(pin, pout);
+  const double base = (mode == 0) ? sc_out : sc_in;
+  const double ratio = (mode == 0) ? sc_in / sc_out : (mode == 2 ? sc_out / sc_in : 1.0);
+  std::vector<cplx> f(S + 2);
+  if (mode == 1) sph_hankel_scaled(S, H.zk * d, base, f.data());
+  else sph_bessel_scaled(S, H.zk * d, base, f.data());
+  for (int s = 0; s <= S; s++) {
+    H.series.push_back(f[s].real());
+    H.series.push_back(f[s].imag());
+  }
+  double v = 1.0;
+  for (int e = 0; e <= S; e++, v *= base) H.series.push_back(v);
+  v = 1.0;
+  for (int e = 0; e <= E; e++, v *= ratio) H.series.push_back(v);
+  H.jobs.push_back(J);
 }
 
 }  // namespace
 
-bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H) {
+bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H) {
   H = HelmHostTables();
   H.zk = zk;
   H.size = size;
@@ -271,53 +317,77 @@ bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTable
   H.plev.assign(nlev + 1, 0);
   H.sclev.assign(nlev + 1, 1.0);
   std::vector<double> bsize(nlev + 1);
+  std::vector<DecayRule> rules;  // level l at l - 2
   int pmax = 1;
   for (int l = 0; l <= nlev; l++) {
     bsize[l] = size / std::pow(2.0, l);
     H.sclev[l] = std::min(std::abs(zk * bsize[l]), 1.0);
     if (l >= 2) {
-      H.plev[l] = helmholtz_nterms(bsize[l], zk, eps);
+      rules.push_back(box_rule(bsize[l], zk, eps));
+      H.plev[l] = rule_nterms(rules.back(), bsize[l], zk);
       pmax = std::max(pmax, H.plev[l]);
     }
   }
   H.pmax = pmax;
   if (pmax > kMaxHelmOrder) return false;
-  build_geometry_tables(pmax, H.geo);
-  const int nd = H.geo.ndist;
+  H.geo = geometry_for(pmax);
+  const int nd = H.geo->ndist;
   H.ptrunc.assign((size_t)(nlev + 1) * 343, 0);
   H.m2l.assign((size_t)(nlev + 1) * nd, CoaxDesc());
   H.m2m.assign(nlev + 1, CoaxDesc());
   H.l2l.assign(nlev + 1, CoaxDesc());
-  auto G = gaunt_for(pmax);
   for (int l = 2; l <= nlev; l++) {
-    const std::vector<int> it = helmholtz_itable(bsize[l], zk, eps);
+    const std::vector<int> it = rule_itable(rules[l - 2], bsize[l], zk);
     std::vector<int> need(nd, 0);
     for (int code = 0; code < 343; code++) {
       int i = code / 49 - 3, j = (code / 7) % 7 - 3, k = code % 7 - 3;
       if (std::max(std::abs(i), std::max(std::abs(j), std::abs(k))) < 2) continue;
       int pt = std::min(it[code], H.plev[l]);
       H.ptrunc[(size_t)l * 343 + code] = pt;
-      int dc = H.geo.off_dist[code];
+      int dc = H.geo->off_dist[code];
       need[dc] = std::max(need[dc], pt);
     }
-    std::vector<std::vector<double>> part(nd);
-    std::vector<CoaxDesc> desc(nd);
-#pragma omp parallel for schedule(dynamic, 1)
     for (int dc = 0; dc < nd; dc++)
       if (need[dc] > 0)
-        coax(*G, 1, -1.0, zk, bsize[l] * H.geo.dist_value[dc], H.sclev[l], H.sclev[l], need[dc], need[dc],
-             part[dc], desc[dc]);
-    for (int dc = 0; dc < nd; dc++) {
-      if (need[dc] == 0) continue;
-      desc[dc].base = (long)(H.z.size() / 2);
-      H.z.insert(H.z.end(), part[dc].begin(), part[dc].end());
-      H.m2l[(size_t)l * nd + dc] = desc[dc];
-    }
+        add_coax(H, 1, 1, bsize[l] * H.geo->dist_value[dc], H.sclev[l], H.sclev[l], need[dc], need[dc], l * nd + dc,
+                 H.m2l[(size_t)l * nd + dc]);
   }
   for (int l = 2; l <= nlev - 1; l++) {
     const double d = bsize[l + 1] * std::sqrt(3.0) / 2.0;
-    coax(*G, 0, 1.0, zk, d, H.sclev[l + 1], H.sclev[l], H.plev[l + 1], H.plev[l], H.z, H.m2m[l]);
-    coax(*G, 2, 1.0, zk, d, H.sclev[l], H.sclev[l + 1], H.plev[l], H.plev[l + 1], H.z, H.l2l[l]);
+    add_coax(H, 0, 0, d, H.sclev[l + 1], H.sclev[l], H.plev[l + 1], H.plev[l], -1, H.m2m[l]);
+    add_coax(H, 2, 0, d, H.sclev[l], H.sclev[l + 1], H.plev[l], H.plev[l + 1], -1, H.l2l[l]);
+  }
+  return true;
+}
+
+bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H) {
+  if (!plan_helm_tables(zk, size, nlev, eps, H)) return false;
+  const auto G = gaunt_for(H.pmax);
+  H.z.assign(2 * (size_t)H.nz, 0.0);
+#pragma omp parallel for schedule(dynamic, 1)
+  for (int t = 0; t < (int)H.jobs.size(); t++) {
+    const CoaxJob& J = H.jobs[t];
+    const int S = J.pin + J.pout;
+    const double* f = &H.series[J.series];
+    const double *pb = f + 2 * (S + 1), *pr = pb + S + 1;
+    for (int m = 0; m <= std::min(J.pin, J.pout); m++) {
+      const long mb = J.base + coax_block(m, J.pin, J.pout);
+      for (int l = m; l <= J.pout; l++)
+        for (int n = m; n <= J.pin; n++) {
+          const long go = G->at(m, n, l);
+          cplx acc = 0.0;
+          for (int s = std::abs(n - l), k = 0; s <= n + l; s += 2, k++) {
+            double sg = (((l + s - n) / 2) & 1) ? -1.0 : 1.0;
+            if (J.neg && (s & 1)) sg = -sg;
+            const double c = 4.0 * M_PI * sg * std::sqrt((2.0 * s + 1.0) / (4.0 * M_PI)) * G->g[go + k];
+            const double pw = J.mode == 1 ? pb[n + l - s] : J.mode == 0 ? pb[s - l + n] * pr[n] : pb[s - n + l] * pr[l];
+            acc += c * pw * cplx(f[2 * s], f[2 * s + 1]);
+          }
+          const size_t e = 2 * (size_t)(mb + (long)(l - m) * (J.pin + 1 - m) + (n - m));
+          H.z[e] = acc.real();
+          H.z[e + 1] = acc.imag();
+        }
+    }
   }
   return true;
 }

@@ -2,6 +2,7 @@
 // expansion orders (h3dterms), and the per-level translation tables.
 #pragma once
 #include <complex>
+#include <memory>
 #include <vector>
 
 #include "tables.hpp"
@@ -27,22 +28,55 @@ struct CoaxDesc {
   int pin = 0, pout = 0;
 };
 
+// What one coaxial operator is computed from: its series start at `series` in
+// HelmHostTables::series with S = pin + pout: f_s (complex, s = 0..S), base^e
+// (e = 0..S), ratio^e (e = 0..max(pin, pout)); mode 0: M2M (R|R), 1: M2L (S|R),
+// 2: L2L (R|R); neg: the direction sign is -1.
+struct CoaxJob {
+  long base = 0;     // as CoaxDesc::base
+  long series = 0;   // doubles
+  int pin = 0, pout = 0, mode = 0, neg = 0;
+  int m2l = -1;      // index of the M2L table this is, or -1
+  int pad = 0;
+};
+
+// Gaunt integrals G(n,s,l;m) for 0 <= m <= min(n,l), n,l <= P,
+// s = |n-l|, |n-l|+2, .., n+l, stored compactly
+struct Gaunt {
+  int P = -1;
+  std::vector<long> off;   // [(m*(P+1)+n)*(P+1)+l]
+  std::vector<double> g;
+  long at(int m, int n, int l) const { return off[((size_t)m * (P + 1) + n) * (P + 1) + l]; }
+};
+// those of the next multiple of four from `pmax` on (so that a call's values do
+// not depend on the calls before it), the last few kept for the process
+std::shared_ptr<const Gaunt> gaunt_for(int pmax);
+
 struct HelmHostTables {
   cplx zk;
   double size = 0, eps = 0;
   int nlev = -1, pmax = 0;
-  HostTables geo;                    // factors, rotations, phases at pmax
+  std::shared_ptr<const HostTables> geo;  // factors, rotations, phases at pmax
   std::vector<int> plev;             // expansion order per level (0 below level 2)
   std::vector<double> sclev;         // rscale per level
   std::vector<int> ptrunc;           // (nlev+1) x 343 list-2 orders
   std::vector<CoaxDesc> m2l;         // (nlev+1) x ndist
   std::vector<CoaxDesc> m2m, l2l;    // per parent level
-  std::vector<double> z;             // all coaxial blocks, complex as (re, im)
+  std::vector<CoaxJob> jobs;         // one per operator
+  std::vector<double> series;        // their series
+  long nz = 0;                       // complex entries of all coaxial blocks
+  std::vector<double> z;             // the blocks themselves, complex as (re, im): build_helm_tables only
 };
 
-// Builds every table the Helmholtz FMM needs for a tree of root side `size`
-// and depth `nlev`.  Returns false when an order exceeds what the device
-// kernels support (kMaxHelmOrder).
+// build_geometry_tables(p), the last few orders kept for the process
+std::shared_ptr<const HostTables> geometry_for(int p);
+
+// The orders, list-2 tables, operator layout and series the Helmholtz FMM
+// needs for a tree of root side `size` and depth `nlev`; the blocks are
+// computed from the series on the device (k_coax).  Returns false when an
+// order exceeds what the device kernels support (kMaxHelmOrder).
+bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H);
+// the same with the blocks computed on the host into H.z
 bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H);
 
 constexpr int kMaxHelmOrder = 120;

@@ -338,6 +338,7 @@ void build_geometry_tables(int p, HostTables& H) {
       total += (long)(2 * n + 1) * (2 * n + 1);
     }
   H.rot.assign(total, 0.0);
+#pragma omp parallel for schedule(dynamic, 1)
   for (int c = 0; c < nrot; c++) {
     auto d = wigner_d(p, thetas[c]);
     for (int n = 0; n <= p; n++) {
@@ -405,6 +406,7 @@ void build_geometry_tables(int p, HostTables& H) {
       th += 16L * (2 * n / 4 + 1) * (n / 4 + 1);
     }
   H.rot_half.assign(th, 0.0);
+#pragma omp parallel for schedule(dynamic, 1)
   for (int c = 0; c < nrot; c++)
     for (int n = 0; n <= p; n++) {
       const int dim = 2 * n + 1, nq = n / 4 + 1;
