@@ -37,9 +37,9 @@ struct HelmCache {
   std::shared_ptr<const HostTables> geo;     // the geometry on the device
   std::shared_ptr<const Gaunt> gaunt;        // the integrals on the device
   size_t gI = 0, gD = 0, gL = 0;             // geometry sizes
-  size_t o_offrot = 0, o_offdist = 0, o_octrot = 0, o_gri = 0, o_grc = 0, o_gzi = 0, o_gzo = 0;
-  size_t o_fac = 0, o_offph = 0, o_octph = 0, o_rot = 0, o_rothalf = 0;
-  size_t o_rotoff = 0, o_rothalf_off = 0;
+  size_t o_offrot = 0, o_offdist = 0, o_octrot = 0;
+  size_t o_fac = 0, o_offph = 0, o_octph = 0, o_rot = 0, o_rotsd = 0;
+  size_t o_rotoff = 0;
   size_t cI = 0, cD = 0, cL = 0, cZ = 0;     // per-call sizes
   size_t o_plev = 0, o_ptrunc = 0, o_sclev = 0, o_coax = 0, o_ztoff = 0, o_zt = 0;
   int m2m_base = 0, l2l_base = 0;
@@ -62,17 +62,12 @@ void helm_upload_geometry(Context& ctx, HelmCache& c, const std::shared_ptr<cons
   c.o_offrot = put_aligned(I, g->off_rot, 16);
   c.o_offdist = put_aligned(I, g->off_dist, 16);
   c.o_octrot = put_aligned(I, g->oct_rot, 16);
-  c.o_gri = put_aligned(I, g->grp_ritems, 16);
-  c.o_grc = put_aligned(I, g->grp_rcount, 16);
-  c.o_gzi = put_aligned(I, g->grp_zitems, 16);
-  c.o_gzo = put_aligned(I, g->grp_zoff, 16);
   c.o_fac = put_aligned(D, g->fac, 8);
   c.o_offph = put_aligned(D, g->off_phase, 8);
   c.o_octph = put_aligned(D, g->oct_phase, 8);
   c.o_rot = put_aligned(D, g->rot, 8);
-  c.o_rothalf = put_aligned(D, g->rot_half, 8);
+  c.o_rotsd = put_aligned(D, g->rot_sd, 8);
   c.o_rotoff = put_aligned(L, g->rot_off, 1);
-  c.o_rothalf_off = put_aligned(L, g->rot_half_off, 1);
   c.gI = I.size(); c.gD = D.size(); c.gL = L.size();
   void* di = ctx.arena.get("hgeo_i", I.size() * sizeof(int));
   void* dd = ctx.arena.get("hgeo_d", D.size() * sizeof(double));
@@ -302,9 +297,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
   Hd.nd = H.geo->ndist;
   Hd.plev = ti + HC->o_plev; Hd.sclev = td + HC->o_sclev; Hd.ptrunc = ti + HC->o_ptrunc;
   Hd.coax = tl + HC->o_coax; Hd.z = tz;
-  Hd.rot_half = gd + HC->o_rothalf; Hd.rot_half_off = gl + HC->o_rothalf_off;
-  Hd.grp_ritems = gi + HC->o_gri; Hd.grp_rcount = gi + HC->o_grc;
-  Hd.grp_zitems = gi + HC->o_gzi; Hd.grp_zoff = gi + HC->o_gzo;
+  Hd.rot_sd = gd + HC->o_rotsd;
   Hd.zt = tz + HC->o_zt; Hd.zt_off = tl + HC->o_ztoff;
   const size_t nb = tree.nboxes;
   double* spos = (double*)ctx.arena.get("spos", sizeof(double) * 4 * (size_t)ns);
@@ -454,23 +447,17 @@ int helm_solve(Context& ctx, const LapCall& c) {
   // expansions fit LDS and a stage's work items fit one pass, else pair by
   // pair (k_hm2l)
   if (P.n_m2l) {
-    int nI = 0;
-    for (int n = 0; n <= pmax; n++) nI += n / 4 + 1;
-    auto grp_lds = [&](int g) {
-      return (6 * kM2LChunk + (size_t)grp_kn_ints(pmax)) * sizeof(int) +
-             sizeof(double) * (2 * (size_t)kM2LGroup * (pmax + 1) + 2 * (size_t)K + 8 +
-                               (size_t)g * grp_member_stride<double>(pmax));
-    };
-    int gmax = 0;
-    for (int g = kM2LGroup; g >= 1 && !gmax && HC->grouped_m2l; g--) {
-      const int gs = g > 2 ? 4 : g;
-      if (nI * gs <= 256 && grp_lds(g) <= ldsmax) gmax = g;
-    }
-    // (one work item per thread: with two, four members' expansions take
-    // ~92 KB of LDS at pmax 23 and leave one workgroup per CU)
-    if (gmax > 0)
-      hipLaunchKernelGGL((k_hm2l_grp<256, 1>), dim3(P.n_m2l), dim3(256), grp_lds(gmax), s, P, Tb, Hd, gmax, mp, lo);
-    else if (m2l_lds)
+    GrpShape G;
+    if (HC->grouped_m2l) G = grp_shape<double>(pmax, ldsmax);
+    if (G.threads > 0) {
+      const size_t need = grp_lds_bytes<double>(pmax, G.room, G.teams);
+#define HM2L_GRP(NT_, I_) \
+  hipLaunchKernelGGL((k_hm2l_grp<NT_, I_>), dim3(P.n_m2l), dim3(NT_), need, s, P, Tb, Hd, G.room, G.lts, mp, lo)
+      if (G.threads == 256) HM2L_GRP(256, 1);
+      else if (G.items == 1) HM2L_GRP(512, 1);
+      else HM2L_GRP(512, 2);
+#undef HM2L_GRP
+    } else if (m2l_lds)
       hipLaunchKernelGGL((k_hm2l<true>), dim3(P.n_m2l), dim3(256), sizeof(double) * 6 * (size_t)K, s, P, Tb, Hd, mp, lo);
     else
       hipLaunchKernelGGL((k_hm2l<false>), dim3(P.n_m2l), dim3(256), lds_ps, s, P, Tb, Hd, mp, lo);

@@ -45,8 +45,7 @@ struct LapTabSet {
   std::vector<float> F;
   size_t off[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   size_t off_l = 0, off_re = 0;
-  size_t off_i[4] = {0, 0, 0, 0};  // grouped M2L items: ritems, rcount, zitems, zoff
-  size_t off_g[4] = {0, 0, 0, 0};  // grouped M2L tables: rot_half, z_m2l_t (doubles); their offsets (longs)
+  size_t off_g[2] = {0, 0};        // grouped M2L tables: rot_sd, z_m2l_t
   size_t off_f = 0;
   long zt_size = 0;
   size_t off_m[4] = {0, 0, 0, 0};    // MFMA tables: mf_rot, mf_z (doubles); mf_rot_off, mf_z_off (longs)
@@ -65,20 +64,15 @@ std::shared_ptr<const LapTabSet> lap_host_tables(int p, double eps) {
   HostTables H;
   build_tables(p, eps, H);
   auto T = std::make_shared<LapTabSet>();
-  // ints: off_rot | off_dist | off_ptrunc | oct_rot | grouped items ; doubles:
+  // ints: off_rot | off_dist | off_ptrunc | oct_rot ; doubles:
   // fac | off_phase | oct_phase | rot | z_m2l | z_m2m | z_l2l | delta | rot_e |
-  // rot_half | z_m2l_t ; longs: rot_off | delta_off | rot_half_off | zt_off
+  // rot_sd | z_m2l_t ; longs: rot_off | delta_off
   auto& Ii = T->I;
   auto& Dd = T->D;
   Ii.insert(Ii.end(), H.off_rot.begin(), H.off_rot.end());
   Ii.insert(Ii.end(), H.off_dist.begin(), H.off_dist.end());
   Ii.insert(Ii.end(), H.off_ptrunc.begin(), H.off_ptrunc.end());
   Ii.insert(Ii.end(), H.oct_rot.begin(), H.oct_rot.end());
-  const std::vector<int>* gi[4] = {&H.grp_ritems, &H.grp_rcount, &H.grp_zitems, &H.grp_zoff};
-  for (int q = 0; q < 4; q++) {
-    T->off_i[q] = Ii.size();
-    Ii.insert(Ii.end(), gi[q]->begin(), gi[q]->end());
-  }
   const std::vector<double>* dparts[9] = {&H.fac, &H.off_phase, &H.oct_phase, &H.rot, &H.z_m2l,
                                           &H.z_m2m, &H.z_l2l, &H.delta, &H.rot_e};
   size_t o[9];
@@ -89,17 +83,13 @@ std::shared_ptr<const LapTabSet> lap_host_tables(int p, double eps) {
   // 32-byte aligned starts for the padded tables of the grouped M2L
   while (Dd.size() % 4) Dd.push_back(0.0);
   T->off_g[0] = Dd.size();
-  Dd.insert(Dd.end(), H.rot_half.begin(), H.rot_half.end());
+  Dd.insert(Dd.end(), H.rot_sd.begin(), H.rot_sd.end());
   while (Dd.size() % 4) Dd.push_back(0.0);
   T->off_g[1] = Dd.size();
   Dd.insert(Dd.end(), H.z_m2l_t.begin(), H.z_m2l_t.end());
   T->L = H.rot_off;
   T->off_l = T->L.size();
   T->L.insert(T->L.end(), H.delta_off.begin(), H.delta_off.end());
-  T->off_g[2] = T->L.size();
-  T->L.insert(T->L.end(), H.rot_half_off.begin(), H.rot_half_off.end());
-  T->off_g[3] = T->L.size();
-  T->L.insert(T->L.end(), H.zt_off.begin(), H.zt_off.end());
   T->zt_size = H.zt_size;
   // MFMA-ordered M2L tables (64-value blocks, 512-byte aligned starts)
   while (Dd.size() % 64) Dd.push_back(0.0);
@@ -115,7 +105,7 @@ std::shared_ptr<const LapTabSet> lap_host_tables(int p, double eps) {
   T->mf_rot_back = H.mf_rot_back;
   T->mf_z_size = H.mf_z_size;
   // FP32 copies of the grouped-M2L tables for the FP32 far field
-  T->F.assign(H.rot_half.begin(), H.rot_half.end());
+  T->F.assign(H.rot_sd.begin(), H.rot_sd.end());
   while (T->F.size() % 4) T->F.push_back(0.0f);
   T->off_f = T->F.size();
   T->F.insert(T->F.end(), H.z_m2l_t.begin(), H.z_m2l_t.end());
@@ -162,12 +152,9 @@ DevTables ensure_tables(Context& ctx, int p, double eps) {
   T.delta = dd + H.off[7];
   T.delta_off = dl + H.off_l;
   T.rot_e = dd + H.off_re;
-  T.grp_ritems = di + H.off_i[0]; T.grp_rcount = di + H.off_i[1];
-  T.grp_zitems = di + H.off_i[2]; T.grp_zoff = di + H.off_i[3];
-  T.rot_half = dd + H.off_g[0]; T.z_m2l_t = dd + H.off_g[1];
-  T.rot_half_off = dl + H.off_g[2]; T.zt_off = dl + H.off_g[3];
+  T.rot_sd = dd + H.off_g[0]; T.z_m2l_t = dd + H.off_g[1];
   T.zt_size = H.zt_size;
-  T.rot_half_f = df;
+  T.rot_sd_f = df;
   T.z_m2l_t_f = df + H.off_f;
   T.mf_rot = dd + H.off_m[0]; T.mf_z = dd + H.off_m[1];
   T.mf_rot_f = df + H.off_mf[0]; T.mf_z_f = df + H.off_mf[1];
@@ -582,36 +569,15 @@ int lap_solve(Context& ctx, const LapCall& c) {
     } else {
       const bool lds = sizeof(T) * 6 * (size_t)K <= max_lds_bytes(ctx);
       const size_t sh = lds ? sizeof(T) * 6 * K : lds_ps;
-      // launch shape of k_m2l_grp: (largest group, threads, items per thread);
-      // the work items of one stage must fit, the group's expansions must fit LDS
-      static const int m2l_shape = [] {
-        const char* v = std::getenv("FMM3D_M2L_SHAPE");
-        if (v && std::strcmp(v, "g2t256i1") == 0) return 1;
-        if (v && std::strcmp(v, "g4t512i1") == 0) return 2;
-        return 0;
-      }();
-      const int gcap = m2l_shape == 1 ? 2 : kM2LGroup;
-      const int nt = m2l_shape == 2 ? 512 : 256, items = m2l_shape == 0 ? 2 : 1;
-      int nI = 0;
-      for (int n = 0; n <= p; n++) nI += n / 4 + 1;
-      int gmax = 0;
-      // LDS: six int arrays, the local, a guard of 8 values, g members of (p+4)^2
-      auto m2l_lds = [&](int g) {
-        return (6 * kM2LChunk + (size_t)grp_kn_ints(p)) * sizeof(int) +
-               sizeof(T) * (2 * (size_t)kM2LGroup * (p + 1) + 2 * (size_t)K + 8 + (size_t)g * grp_member_stride<T>(p));
-      };
-      for (int g = gcap; g >= 1 && !gmax; g--) {
-        const int gs = g > 2 ? 4 : g;
-        if (nI * gs <= items * nt && m2l_lds(g) <= max_lds_bytes(ctx)) gmax = g;
-      }
-      if ((m2l_form == 0 || m2l_form == 3) && gmax > 0) {
-        const size_t need = m2l_lds(gmax);
-        if (m2l_shape == 0)
-          hipLaunchKernelGGL((k_m2l_grp<T, 256, 2>), dim3(P.n_m2l), dim3(256), need, s, P, Tb, gmax, mp, lo);
-        else if (m2l_shape == 1)
-          hipLaunchKernelGGL((k_m2l_grp<T, 256, 1>), dim3(P.n_m2l), dim3(256), need, s, P, Tb, gmax, mp, lo);
-        else
-          hipLaunchKernelGGL((k_m2l_grp<T, 512, 1>), dim3(P.n_m2l), dim3(512), need, s, P, Tb, gmax, mp, lo);
+      const GrpShape G = grp_shape<T>(p, max_lds_bytes(ctx));
+      if ((m2l_form == 0 || m2l_form == 3) && G.threads > 0) {
+        const size_t need = grp_lds_bytes<T>(p, G.room, G.teams);
+#define M2L_GRP(NT_, I_) \
+  hipLaunchKernelGGL((k_m2l_grp<T, NT_, I_>), dim3(P.n_m2l), dim3(NT_), need, s, P, Tb, G.room, G.lts, mp, lo)
+        if (G.threads == 256) M2L_GRP(256, 1);
+        else if (G.items == 1) M2L_GRP(512, 1);
+        else M2L_GRP(512, 2);
+#undef M2L_GRP
       } else if (m2l_form != 2) {
         if (lds) hipLaunchKernelGGL((k_m2l<T, true>), dim3(P.n_m2l), dim3(256), sh, s, P, Tb, mp, lo);
         else hipLaunchKernelGGL((k_m2l<T, false>), dim3(P.n_m2l), dim3(256), sh, s, P, Tb, mp, lo);

@@ -790,24 +790,30 @@ __global__ void k_m2l(DevPlan P, DevTables Tb, const T* __restrict__ mp, T* __re
 }
 
 // ---------------------------------------------------------------------------
-// M2L grouped by translation class.  List-2 sources of one target whose
-// offsets share (dx^2 + dy^2, dz) share the rotation block, the z-shift table
-// and the truncation order; only the azimuthal phase differs.  Up to
-// kM2LGroup of them are translated together: the gs lanes of one work item
-// hold the group's members and read the same table entry, so every table
-// entry is fetched once per group, and each lane produces four consecutive
-// orders m' (rotation) or degrees l (z-shift) of one member, so one LDS read
-// of an input coefficient feeds four FMAs per output part.  Stages run in
-// place (results held in registers across a barrier); the back rotation
-// applies each member's phase, sums the members across lanes in a fixed order
-// and adds the sum to the target's local in LDS.
+// M2L grouped by translation class (m2l_grp.hpp).
 // ---------------------------------------------------------------------------
+template <typename T>
+struct LapM2LSrc {
+  const int *ptrunc, *rot, *dst;
+  const T* z;
+  long zsize;
+  int p;
+  __device__ __forceinline__ void geo(int code, int& pt, int& rc, int& dist) const {
+    pt = ptrunc[code];
+    rc = rot[code];
+    dist = dst[code];
+  }
+  __device__ __forceinline__ const T* ztab(int dist, int am, int q, int& stride) const {
+    stride = 16 * ((p - am) / 4 + 1);
+    return z + (size_t)dist * zsize + 16 * (grp_tiles(p + 1) - grp_tiles(p + 1 - am) + q);
+  }
+};
 template <typename T>
 __device__ __forceinline__ const T* grp_rot_tab(const DevTables& Tb);
 template <>
-__device__ __forceinline__ const double* grp_rot_tab<double>(const DevTables& Tb) { return Tb.rot_half; }
+__device__ __forceinline__ const double* grp_rot_tab<double>(const DevTables& Tb) { return Tb.rot_sd; }
 template <>
-__device__ __forceinline__ const float* grp_rot_tab<float>(const DevTables& Tb) { return Tb.rot_half_f; }
+__device__ __forceinline__ const float* grp_rot_tab<float>(const DevTables& Tb) { return Tb.rot_sd_f; }
 template <typename T>
 __device__ __forceinline__ const T* grp_z_tab(const DevTables& Tb);
 template <>
@@ -816,202 +822,12 @@ template <>
 __device__ __forceinline__ const float* grp_z_tab<float>(const DevTables& Tb) { return Tb.z_m2l_t_f; }
 
 template <typename T, int NT, int ITEMS>
-__global__ __launch_bounds__(NT) void k_m2l_grp(DevPlan P, DevTables Tb, int gmax, const T* __restrict__ mp,
-                                                  T* __restrict__ lo) {
-  extern __shared__ unsigned char smem_raw[];
-  int* s_key = reinterpret_cast<int*>(smem_raw);
-  int* s_box = s_key + kM2LChunk;
-  int* s_code = s_box + kM2LChunk;
-  int* t_key = s_code + kM2LChunk;
-  int* t_box = t_key + kM2LChunk;
-  int* t_code = t_box + kM2LChunk;
-  const int tid = threadIdx.x, bs = blockDim.x;
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(ITEMS == 1 ? 4 : 2))) void k_m2l_grp(DevPlan P, DevTables Tb, int room, int lts, const T* __restrict__ mp,
+                                                T* __restrict__ lo) {
   const int b = P.m2l_boxes[xcd_block()];
-  const int p = P.p, P1 = p + 1, K2 = 2 * P.K;
-  // degree of each packed index k < (p+4)^2, and the members' phases
-  // e^{i am phi}, am = 0..p, of the group in hand
-  int* s_kn = t_code + kM2LChunk;
-  T* s_ph = reinterpret_cast<T*>(s_kn + grp_kn_ints(p));
-  T* acc = s_ph + 2 * kM2LGroup * P1;
-  // members: (p+4)^2 complex each (degrees p+1..p+3 stay zero or hold the
-  // zeros written for a truncated member), after a zero guard of 8 values
-  const int MS = grp_member_stride<T>(p);
-  T* A = acc + K2 + 8;
-  const T ih = (T)P.inv_side[P.level[b]];
-  for (int k = tid; k < K2 + 8 + gmax * MS; k += bs) acc[k] = T(0);
-  for (int k = tid; k < (p + 4) * (p + 4); k += bs) {
-    int n = (int)sqrtf((float)k);
-    while (n * n > k) n--;
-    while ((n + 1) * (n + 1) <= k) n++;
-    s_kn[k] = n;
-  }
-  const T* rtab = grp_rot_tab<T>(Tb);
-  const T* ztab = grp_z_tab<T>(Tb);
-  const int off0 = P.l2_off[b], n2 = P.l2_off[b + 1] - off0;
-  const int bi = P.ijk[3 * b], bj = P.ijk[3 * b + 1], bk = P.ijk[3 * b + 2];
-  for (int c0 = 0; c0 < n2; c0 += kM2LChunk) {
-    const int cn = min(kM2LChunk, n2 - c0);
-    __syncthreads();
-    if (tid < cn) {
-      const int j = P.l2_idx[off0 + c0 + tid];
-      const int di = P.ijk[3 * j] - bi, dj = P.ijk[3 * j + 1] - bj, dk = P.ijk[3 * j + 2] - bk;
-      s_box[tid] = j;
-      s_code[tid] = ((di + 3) * 7 + (dj + 3)) * 7 + (dk + 3);
-      s_key[tid] = (di * di + dj * dj) * 7 + (dk + 3);
-    }
-    __syncthreads();
-    if (tid < cn) {  // stable rank by key
-      const int key = s_key[tid];
-      int rank = 0;
-      for (int t = 0; t < cn; t++) {
-        const int kt = s_key[t];
-        rank += (kt < key) || (kt == key && t < tid);
-      }
-      t_key[rank] = key;
-      t_box[rank] = s_box[tid];
-      t_code[rank] = s_code[tid];
-    }
-    __syncthreads();
-    for (int s0 = 0; s0 < cn;) {
-      const int key0 = t_key[s0];
-      int g = 1;
-      while (g < gmax && s0 + g < cn && t_key[s0 + g] == key0) g++;
-      const int gs = g > 2 ? 4 : g;  // lanes per item
-      const int lg = gs == 4 ? 2 : gs - 1;
-      const int code0 = t_code[s0];
-      const int pt = Tb.off_ptrunc[code0];
-      const int rc = Tb.off_rot[code0];
-      const T* Z = ztab + (size_t)Tb.off_dist[code0] * Tb.zt_size;
-      const int Kp = (pt + 1) * (pt + 1), Kz = (pt + 4) * (pt + 4);
-      for (int idx = tid; idx < g * (pt + 1); idx += bs) {
-        const int jj = idx / (pt + 1), am = idx - jj * (pt + 1);
-        const double* ph = Tb.off_phase + (size_t)t_code[s0 + jj] * 2 * P1;
-        s_ph[2 * (jj * P1 + am)] = (T)ph[2 * am];
-        s_ph[2 * (jj * P1 + am) + 1] = (T)ph[2 * am + 1];
-      }
-      __syncthreads();
-      // (a) members times e^{i m phi}; degrees pt+1..pt+3 set to zero
-      for (int jj = 0; jj < g; jj++) {
-        const T* src = mp + (size_t)t_box[s0 + jj] * K2;
-        const T* phj = s_ph + 2 * jj * P1;
-        T* Aj = A + jj * MS;
-        for (int k = tid; k < Kz; k += bs) {
-          T vr = 0, vi = 0;
-          if (k < Kp) {
-            const int n = s_kn[k];
-            const int m = k - n * n - n, am = m < 0 ? -m : m;
-            const T er = phj[2 * am], ei = m < 0 ? -phj[2 * am + 1] : phj[2 * am + 1];
-            const T xr = src[2 * k], xi = src[2 * k + 1];
-            vr = xr * er - xi * ei;
-            vi = xr * ei + xi * er;
-          }
-          Aj[2 * k] = vr;
-          Aj[2 * k + 1] = vi;
-        }
-      }
-      __syncthreads();
-      // Work items of a stage (rotation items by degree, z-shift items by
-      // order; the two counts are equal): member jj of item u0 in the first
-      // round and of item NI-1-u0 in the second, which pairs the cheapest
-      // items with the most expensive ones.
-      const int NI = Tb.grp_rcount[pt], U0 = bs >> lg;
-      const int u0 = tid >> lg, jj = tid & (gs - 1);
-      int uq[ITEMS];
-      uq[0] = u0 < NI ? u0 : -1;
-      if (ITEMS > 1) uq[ITEMS - 1] = NI - 1 - u0 >= U0 ? NI - 1 - u0 : -1;
-      const bool mem = jj < g;
-      T r[ITEMS][16];
-      // (b) rotate to the z axis
-#pragma unroll
-      for (int q = 0; q < ITEMS; q++) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) r[q][e] = T(0);
-        if (uq[q] >= 0 && mem) {
-          const int it = Tb.grp_ritems[uq[q]], n = it >> 8, qc = it & 255;
-          grp_rot_item<T, false>(rtab + Tb.rot_half_off[rc * P1 + n] + 16 * qc, n / 4 + 1, n, qc, A + jj * MS, r[q]);
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < ITEMS; q++)
-        if (uq[q] >= 0 && mem) {
-          const int it = Tb.grp_ritems[uq[q]];
-          grp_rot_store<T>(it >> 8, 4 * (it & 255), r[q], A + jj * MS);
-        }
-      __syncthreads();
-      // (c) shift along z
-      const int zo = Tb.grp_zoff[pt];
-#pragma unroll
-      for (int q = 0; q < ITEMS; q++) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) r[q][e] = T(0);
-        if (uq[q] >= 0 && mem) {
-          const int it = Tb.grp_zitems[zo + uq[q]], am = it >> 8;
-          grp_z_item<T>(Z + Tb.zt_off[am], (p - am) / 4 + 1, am, it & 255, pt, A + jj * MS, r[q]);
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int q = 0; q < ITEMS; q++)
-        if (uq[q] >= 0 && mem) {
-          const int it = Tb.grp_zitems[zo + uq[q]], am = it >> 8;
-          grp_z_store<T>(am, am + 4 * (it & 255), pt, r[q], A + jj * MS);
-        }
-      __syncthreads();
-      // (d) rotate back, apply e^{-i m phi} and the scale, sum the members
-#pragma unroll
-      for (int q = 0; q < ITEMS; q++) {
-#pragma unroll
-        for (int e = 0; e < 16; e++) r[q][e] = T(0);
-        int n = 0, mp0 = 0;
-        if (uq[q] >= 0) {
-          const int it = Tb.grp_ritems[uq[q]];
-          n = it >> 8;
-          mp0 = 4 * (it & 255);
-          if (mem) {
-            grp_rot_item<T, true>(rtab + Tb.rot_half_off[rc * P1 + n] + 4 * mp0, n / 4 + 1, n, mp0 / 4,
-                                  A + jj * MS, r[q]);
-            const T* ph = s_ph + 2 * jj * P1;
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-              const int mq = mp0 + c <= n ? mp0 + c : n;
-              const T er = ph[2 * mq] * ih, ei = ph[2 * mq + 1] * ih;
-              const T pr = r[q][4 * c], pi = r[q][4 * c + 1], qr = r[q][4 * c + 2], qi = r[q][4 * c + 3];
-              r[q][4 * c] = pr * er + pi * ei;       // (pr + i pi) e^{-i m' phi}
-              r[q][4 * c + 1] = pi * er - pr * ei;
-              r[q][4 * c + 2] = qr * er - qi * ei;   // (qr + i qi) e^{+i m' phi}
-              r[q][4 * c + 3] = qi * er + qr * ei;
-            }
-          }
-        }
-#pragma unroll
-        for (int e = 0; e < 16; e++) {
-          T v = r[q][e];
-          if (gs > 1) v += __shfl_xor(v, 1);
-          if (gs > 2) v += __shfl_xor(v, 2);
-          r[q][e] = v;
-        }
-        if (uq[q] >= 0 && jj == 0) {
-#pragma unroll
-          for (int c = 0; c < 4; c++) {
-            const int mq = mp0 + c;
-            if (mq > n) break;
-            acc[2 * eidx(n, mq)] += r[q][4 * c];
-            acc[2 * eidx(n, mq) + 1] += r[q][4 * c + 1];
-            if (mq > 0) {
-              acc[2 * eidx(n, -mq)] += r[q][4 * c + 2];
-              acc[2 * eidx(n, -mq) + 1] += r[q][4 * c + 3];
-            }
-          }
-        }
-      }
-      __syncthreads();
-      s0 += g;
-    }
-  }
-  __syncthreads();
-  T* out = lo + (size_t)b * K2;
-  for (int k = tid; k < K2; k += bs) out[k] += acc[k];
+  const LapM2LSrc<T> S{Tb.off_ptrunc, Tb.off_rot, Tb.off_dist, grp_z_tab<T>(Tb), Tb.zt_size, P.p};
+  m2l_grp_box<T, ITEMS, false>(P, b, room, lts, S, Tb.off_phase, grp_rot_tab<T>(Tb), mp, lo,
+                               (T)P.inv_side[P.level[b]]);
 }
 
 // ---------------------------------------------------------------------------

@@ -54,16 +54,12 @@ struct DevTables {
   const double *delta;      // d^n(pi/2) per degree, row-major (2n+1)^2
   const long *delta_off;    // start of degree n
   const double *rot_e;      // per rotation class: e^{i k theta}, k = 0..p
-  // grouped M2L work items: rotation (n << 8 | q) by degree, count with n <= pt;
-  // z-shift (|m| << 8 | q) per truncation order pt, start of pt's items
-  const int *grp_ritems, *grp_rcount, *grp_zitems, *grp_zoff;
-  // tiled tables of the grouped M2L: half rotation blocks [m][m' >= 0] per
-  // (class, degree) at rot_half_off[c*(p+1)+n]; z-shift [n-m][l-m] per
-  // distance class (zt_size values each), order m at zt_off[m]; both in 4x4
-  // tiles [row block][column block][row][column], in FP64 and in FP32
-  const double *rot_half, *z_m2l_t;
-  const float *rot_half_f, *z_m2l_t_f;
-  const long *rot_half_off, *zt_off;
+  // tiled tables of the grouped M2L: rotation blocks of sums and differences
+  // [m >= 0][m' >= 0] per class and degree; z-shift [n-m][l-m] per distance
+  // class (zt_size values each) and order; both in 4x4 tiles [row block]
+  // [column block][row][column], in FP64 and in FP32
+  const double *rot_sd, *z_m2l_t;
+  const float *rot_sd_f, *z_m2l_t_f;
   long zt_size;
   // MFMA-ordered M2L tables (FP64 and FP32): forward rotation blocks of
   // (class, degree) at mf_rot_off[c*(p+1)+n], back blocks mf_rot_back

@@ -15,6 +15,13 @@
 
 namespace fmm3d {
 
+// sum of (j/4+1)^2 over j < n: the 4x4 tiles of the square blocks of those degrees
+static long sd_tiles(int n) {
+  long t = 0;
+  for (int j = 0; j < n; j++) t += (long)(j / 4 + 1) * (j / 4 + 1);
+  return t;
+}
+
 static std::vector<std::vector<double>> wigner_d(int p, double beta) {
   const double a = std::cos(0.5 * beta), s = std::sin(0.5 * beta);
   std::vector<std::vector<double>> out(p + 1);
@@ -191,17 +198,12 @@ void build_tables(int p, double eps, HostTables& H) {
   }
   // the same coefficients for the grouped M2L in 4x4 tiles per order m:
   // [row block of n - m][column block of l - m][row][column], zero past p
-  H.zt_off.assign(P1 + 1, 0);
-  for (int m = 0; m <= p; m++) {
-    const long nb4 = (p - m) / 4 + 1;
-    H.zt_off[m + 1] = H.zt_off[m] + 16 * nb4 * nb4;
-  }
-  H.zt_size = H.zt_off[P1];
+  H.zt_size = 16L * sd_tiles(P1);
   H.z_m2l_t.assign((size_t)H.zt_size * H.ndist, 0.0);
   for (int dc = 0; dc < H.ndist; dc++)
     for (int m = 0; m <= p; m++) {
       const int nb4 = (p - m) / 4 + 1;
-      double* zb = &H.z_m2l_t[(size_t)H.zt_size * dc + H.zt_off[m]];
+      double* zb = &H.z_m2l_t[(size_t)H.zt_size * dc + 16L * (sd_tiles(P1) - sd_tiles(P1 - m))];
       for (int n = m; n <= p; n++)
         for (int l = m; l <= p; l++) {
           const int rr = n - m, cc = l - m;
@@ -376,45 +378,27 @@ void build_geometry_tables(int p, HostTables& H) {
   }
   H.ndist = (int)dists.size();
   H.dist_value = dists;
-  // work items of the grouped M2L: a rotation item is (degree n, columns
-  // 4q..4q+3), ordered by n so that the items of degrees <= pt are a prefix;
-  // a z-shift item is (order |m|, degrees l = |m|+4q..+3), listed per pt
-  H.grp_ritems.clear();
-  H.grp_rcount.assign(P1, 0);
-  for (int n = 0; n <= p; n++) {
-    for (int q = 0; 4 * q <= n; q++) H.grp_ritems.push_back((n << 8) | q);
-    H.grp_rcount[n] = (int)H.grp_ritems.size();
-  }
-  H.grp_zitems.clear();
-  H.grp_zoff.assign(P1 + 1, 0);
-  for (int pt = 0; pt <= p; pt++) {
-    H.grp_zoff[pt] = (int)H.grp_zitems.size();
-    for (int am = 0; am <= pt; am++)
-      for (int q = 0; am + 4 * q <= pt; q++) H.grp_zitems.push_back((am << 8) | q);
-  }
-  H.grp_zoff[P1] = (int)H.grp_zitems.size();
-  // rotation blocks for the grouped M2L: columns m' >= 0 only (the others
-  // follow from D[-m][-m'] = D[m][m']), cut into 4x4 tiles [row block][column
-  // block][row][column] so that one work item (four columns) reads one
-  // contiguous 128-byte tile per four rows; rows past 2n and columns past n
-  // are zero
-  H.rot_half_off.assign((size_t)nrot * P1, 0);
-  long th = 0;
-  for (int c = 0; c < nrot; c++)
-    for (int n = 0; n <= p; n++) {
-      H.rot_half_off[(size_t)c * P1 + n] = th;
-      th += 16L * (2 * n / 4 + 1) * (n / 4 + 1);
-    }
-  H.rot_half.assign(th, 0.0);
+  // rotation blocks of the grouped M2L on sums and differences of orders m and
+  // -m (D[-m][-m'] = D[m][m']): D[m][m'] + D[-m][m'] for m, m' >= 0, the row
+  // m = 0 doubled for m' > 0 and the column m' = 0 taken once, then
+  // D[m][m'] - D[-m][m'] for m, m' >= 1; both in a square of 4x4 tiles [row
+  // block][column block][row][sum, difference][column], so that one work item
+  // (four columns) reads contiguous values per four rows; the rest is zero
+  const long nt = 32L * sd_tiles(P1);
+  H.rot_sd.assign((size_t)nrot * nt, 0.0);
 #pragma omp parallel for schedule(dynamic, 1)
   for (int c = 0; c < nrot; c++)
     for (int n = 0; n <= p; n++) {
       const int dim = 2 * n + 1, nq = n / 4 + 1;
       const double* D = &H.rot[H.rot_off[(size_t)c * P1 + n]];
-      double* Db = &H.rot_half[H.rot_half_off[(size_t)c * P1 + n]];
-      for (int row = 0; row < dim; row++)
-        for (int mp = 0; mp <= n; mp++)
-          Db[(((size_t)(row / 4) * nq + mp / 4) * 4 + row % 4) * 4 + mp % 4] = D[row * dim + (mp + n)];
+      double* S = &H.rot_sd[(size_t)c * nt + 32L * sd_tiles(n)];
+      for (int m = 0; m <= n; m++)
+        for (int mp = 0; mp <= n; mp++) {
+          const size_t at = (((size_t)(m / 4) * nq + mp / 4) * 4 + m % 4) * 8 + mp % 4;
+          const double d = D[(n + m) * dim + (n + mp)], e = D[(n - m) * dim + (n + mp)];
+          S[at] = mp == 0 ? d : d + e;
+          S[at + 4] = m > 0 && mp > 0 ? d - e : 0.0;
+        }
     }
 }
 

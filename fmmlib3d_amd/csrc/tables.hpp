@@ -21,12 +21,8 @@ struct HostTables {
   std::vector<long> delta_off;                     // p+1
   std::vector<double> rot_e;                       // nrot x (p+1) complex: e^{i k theta_class}
   // grouped M2L work items (see build_geometry_tables)
-  std::vector<int> grp_ritems, grp_rcount;         // (n << 8 | q); count of items with n <= pt
-  std::vector<int> grp_zitems, grp_zoff;           // (|m| << 8 | q) per pt; start of pt's items
-  std::vector<double> rot_half;                    // per class and degree: 4x4 tiles of [m][m' >= 0]
-  std::vector<long> rot_half_off;                  // nrot x (p+1)
+  std::vector<double> rot_sd;                      // per class and degree: 4x4 tiles of D[m][m'] + D[-m][m'], then of the difference
   std::vector<double> z_m2l_t;                     // per distance class and order m: 4x4 tiles of [n-m][l-m]
-  std::vector<long> zt_off;                        // start of order m within a class, p+2 entries
   long zt_size = 0;                                // doubles per distance class
   // M2L on the matrix cores (16x16x4 MFMA operand order, see
   // build_mfma_tables): per rotation class and degree n the forward and back
