@@ -163,19 +163,21 @@ DevTables ensure_tables(Context& ctx, int p, double eps) {
   return T;
 }
 
+// The near field of n work items (both kinds, pot0 / fld0 at sources, pot1 /
+// fld1 at targets).
 template <typename TN>
-void launch_p2p(const DevPlan& P, const int* items, int n, int kind, const double* spos,
-                const TN* str, const double* str64, const double* tpos, int ifcharge, int ifdipole, bool fld,
-                double* pot, double* fo, hipStream_t s) {
+void launch_p2p(const DevPlan& P, const int* items, int n, const double* spos, const TN* str, const double* str64,
+                const double* tpos, int ifcharge, int ifdipole, bool fld, double* pot0, double* fld0, double* pot1,
+                double* fld1, hipStream_t s) {
   if (n == 0) return;
   DevPlan Q = P;
   Q.p2p_items = items;
   Q.n_p2p = n;
-  dim3 g(item_groups(n)), b(kP2PBlock * kItemWaves);
-#define P2P_CASE(C, Dp, F)                                                                        \
-  if (ifcharge == C && ifdipole == Dp && fld == F) {                                             \
-    hipLaunchKernelGGL((k_p2p<TN, C, Dp, F>), g, b, 0, s, Q, spos, str, str64, tpos, kind, pot, fo); \
-    return;                                                                                       \
+#define P2P_CASE(C, Dp, F)                                                                                        \
+  if (ifcharge == C && ifdipole == Dp && fld == F) {                                                              \
+    hipLaunchKernelGGL((k_p2p<TN, C, Dp, F>), dim3((unsigned)n), dim3(64 * kP2PSplit), 0, s, Q, spos, str, str64, \
+                       tpos, pot0, fld0, pot1, fld1);                                                             \
+    return;                                                                                                       \
   }
   P2P_CASE(1, 0, false) P2P_CASE(1, 0, true) P2P_CASE(0, 1, false) P2P_CASE(0, 1, true)
   P2P_CASE(1, 1, false) P2P_CASE(1, 1, true)
@@ -503,10 +505,19 @@ int lap_solve(Context& ctx, const LapCall& c) {
     tri_near(dIB + O.p2p0, O.n_p2p0, 0, pot_sn, f.iffld ? fld_sn : nullptr);
     tri_near(dIB + O.p2p1, O.n_p2p1, 1, pot_tn, f.iffldtarg ? fld_tn : nullptr);
   } else if (f.ifcharge || f.ifdipole) {
-    launch_p2p<TN>(P, dIB + O.p2p0, O.n_p2p0, 0, spos, strn, str64, tpos, f.ifcharge, f.ifdipole,
-                   f.iffld != 0, pot_sn, fld_sn, s2);
-    launch_p2p<TN>(P, dIB + O.p2p1, O.n_p2p1, 1, spos, strn, str64, tpos, f.ifcharge, f.ifdipole,
-                   f.iffldtarg != 0, pot_tn, fld_tn, s2);
+    // sources and targets in one launch where both want the same outputs
+    const int* it = dIB + O.p2p0;
+    const int n0 = O.n_p2p0, n1 = O.n_p2p1;
+    const bool both = n0 == 0 || n1 == 0 || (f.iffld != 0) == (f.iffldtarg != 0);
+    auto near = [&](const int* i0, int n, bool fld) {
+      launch_p2p<TN>(P, i0, n, spos, strn, str64, tpos, f.ifcharge, f.ifdipole, fld, pot_sn, fld_sn, pot_tn, fld_tn, s2);
+    };
+    if (both) {
+      near(it, n0 + n1, n0 ? f.iffld != 0 : f.iffldtarg != 0);
+    } else {
+      near(it, n0, f.iffld != 0);
+      near(it + 3 * (size_t)n0, n1, f.iffldtarg != 0);
+    }
   }
   if (qp) {
     // after the charges' near field on the same stream: both add into the sums

@@ -280,7 +280,7 @@ __device__ __forceinline__ int xcd_block() {
 constexpr int kFold = 32;
 
 template <typename TN>
-__device__ __forceinline__ TN rsqrt_t(TN x);
+__device__ __forceinline__ TN rsqrt_t(TN x, TN c375 = TN(0.375));
 // x^{-1/2} for normal positive x (callers mask x = 0 themselves).  FP64: the
 // hardware estimate y refined by one second-order step of the Householder
 // iteration for x^{-1/2}, e = 1 - x y^2, y <- y (1 + e/2 + 3e^2/8) (the
@@ -288,12 +288,12 @@ __device__ __forceinline__ TN rsqrt_t(TN x);
 // FP32: the hardware instruction alone (about 1 ulp), without the rescaling
 // of subnormal arguments a library rsqrtf adds.
 template <>
-__device__ __forceinline__ double rsqrt_t<double>(double x) {
+__device__ __forceinline__ double rsqrt_t<double>(double x, double c375) {
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
+  return fma(y * e, fma(e, c375, 0.5), y);
 }
 template <>
-__device__ __forceinline__ float rsqrt_t<float>(float x) { return __builtin_amdgcn_rsqf(x); }
+__device__ __forceinline__ float rsqrt_t<float>(float x, float) { return __builtin_amdgcn_rsqf(x); }
 
 }  // namespace fmm3d

@@ -1004,20 +1004,62 @@ __global__ void k_m2l_fact(DevPlan P, DevTables Tb, const T* __restrict__ mp, T*
 
 // ---------------------------------------------------------------------------
 // P2P near field (src/lfmm3dpart.f:1076-1141, lfmm3dpart_direct_self/_targ).
-// One workgroup per (leaf, chunk of evaluation points); one point per thread.
-// The source loop is wave-uniform, so positions and strengths stream through
-// the scalar cache and every lane reuses them from SGPRs.  Offsets and r^2
+// A work item is 64 evaluation points of a leaf, one per lane; the kP2PSplit waves
+// of a workgroup share it and take parts of every source box, their sums added
+// in order at the end.  The source loop is
+// wave-uniform, so positions and strengths stream through the scalar cache and
+// every lane reuses them from SGPRs; the next source is loaded before the
+// current pair is computed (p2p_sources).
+// Bound: VALU issue, 39 instructions per charge-and-dipole pair in FP64 (a
+// 64-lane FP64 one takes 4 cycles, the reciprocal root 16; the clock falls to
+// about 1.8 GHz under them) and 38 in FP32.  1M + 1M uniform, charges and
+// dipoles, near field alone: FP64 22.4 -> 19.0 ms, FP32 14.5 -> 12.6 ms
+// against one wave per item with the loads next to their use (two exposed
+// scalar-load waits per pair).  FP32 asks for 6 waves per SIMD, not 8: its
+// redo path then spills less (13.1 -> 12.6 ms).  Offsets and r^2
 // are formed in FP64 for every precision; with TN = float the rest of the
 // pair is FP32, summed in FP32 over runs of at most kFold sources and folded
 // into FP64 accumulators, except for the closest pairs (r^2 < rc2, r below
 // 1/32 of the leaf side): such a pair dominates the sums at its point, and a
 // dipole's v.d can cancel, which multiplies the FP32 rounding of v and d by
 // |v||d|/|v.d|.  The FP32 loop only keeps the smallest r^2 of the run (one
-// min per pair, no branch, so the unrolled source loads stay batched); a
+// min per pair, no branch, so the loads stay ahead of the arithmetic); a
 // point whose run held a close pair drops that run's FP32 sums and runs it
 // again with the close pairs in FP64 from the FP64 strengths (redo_run),
 // which happens for a few runs only.
 // ---------------------------------------------------------------------------
+
+// Waves per work item.  Neighbouring waves read the same sources at about the
+// same time, and a small problem's few items still fill the chip: with one
+// wave per item 2,000 points took 135 us, 20,000 points 248 us and 250,000
+// (FP32) 2.5 ms, with four 59 us, 74 us and 1.4 ms, with sixteen 38 us, 66 us
+// and 1.5 ms; 1M + 1M FP32 19.8, 13.0 and 13.3 ms.  It is the same for every
+// call: a request's sums must not depend on what else is in its launch.
+constexpr int kP2PSplit = 4;
+
+// One source of the pair loop in scalar registers
+template <typename TN, bool CHG, bool DIP>
+struct SrcRec {
+  double x, y, z;
+  TN q[2], v[6];
+  __device__ __forceinline__ void load(const double* __restrict__ sp, const TN* __restrict__ st) {
+    x = sp[0]; y = sp[1]; z = sp[2];
+    if (CHG) { q[0] = st[0]; q[1] = st[1]; }
+    if (DIP)
+#pragma unroll
+      for (int k = 0; k < 6; k++) v[k] = st[2 + k];
+  }
+};
+
+// The pair loop's constants, kept in vector registers over the loop (as
+// literals FP64 ones are moved into scalar registers again for every pair)
+template <typename TN>
+struct PairConst {
+  TN c3 = TN(3), c375 = TN(0.375);
+  __device__ __forceinline__ PairConst() {
+    if constexpr (sizeof(TN) == sizeof(double)) asm volatile("" : "+v"(c3), "+v"(c375));
+  }
+};
 
 template <typename TN, bool CHG, bool DIP, bool FLD>
 struct PairAcc {
@@ -1025,39 +1067,39 @@ struct PairAcc {
   // pot += q/r + (v.d)/r^3 = (q + (v.d)/r^2)/r;
   // fld += (q + 3 (v.d)/r^2) d/r^3 - v/r^3 = (c d - v)/r^3, d = x_t - x_s
   // returns r^2 in TN
-  __device__ __forceinline__ TN add(double xt, double yt, double zt, const double* __restrict__ sp,
-                                    const TN* __restrict__ st, bool mask) {
-    const double dxd = xt - sp[0], dyd = yt - sp[1], dzd = zt - sp[2];
+  __device__ __forceinline__ TN add(double xt, double yt, double zt, const SrcRec<TN, CHG, DIP>& s, bool mask,
+                                    const PairConst<TN>& pc) {
+    const double dxd = xt - s.x, dyd = yt - s.y, dzd = zt - s.z;
     const double r2d = fma(dxd, dxd, fma(dyd, dyd, dzd * dzd));
     const TN dx = (TN)dxd, dy = (TN)dyd, dz = (TN)dzd, r2 = (TN)r2d;
-    TN ri = rsqrt_t<TN>(r2);
+    TN ri = rsqrt_t<TN>(r2, pc.c375);
     if (mask) ri = TN(0);
     const TN ri2 = ri * ri;
     if (!DIP) {
-      pr = fma(st[0], ri, pr);
-      pi = fma(st[1], ri, pi);
+      pr = fma(s.q[0], ri, pr);
+      pi = fma(s.q[1], ri, pi);
       if (FLD) {
         const TN ri3 = ri * ri2;
-        const TN cr = st[0] * ri3, ci = st[1] * ri3;
+        const TN cr = s.q[0] * ri3, ci = s.q[1] * ri3;
         fxr = fma(cr, dx, fxr); fxi = fma(ci, dx, fxi);
         fyr = fma(cr, dy, fyr); fyi = fma(ci, dy, fyi);
         fzr = fma(cr, dz, fzr); fzi = fma(ci, dz, fzi);
       }
       return r2;
     }
-    const TN dotr = fma(st[2], dx, fma(st[4], dy, st[6] * dz));
-    const TN doti = fma(st[3], dx, fma(st[5], dy, st[7] * dz));
-    const TN ar = CHG ? fma(dotr, ri2, st[0]) : dotr * ri2;
-    const TN ai = CHG ? fma(doti, ri2, st[1]) : doti * ri2;
+    const TN dotr = fma(s.v[0], dx, fma(s.v[2], dy, s.v[4] * dz));
+    const TN doti = fma(s.v[1], dx, fma(s.v[3], dy, s.v[5] * dz));
+    const TN ar = CHG ? fma(dotr, ri2, s.q[0]) : dotr * ri2;
+    const TN ai = CHG ? fma(doti, ri2, s.q[1]) : doti * ri2;
     pr = fma(ar, ri, pr);
     pi = fma(ai, ri, pi);
     if (FLD) {
-      const TN ri3 = ri * ri2, t3 = TN(3) * ri2;
-      const TN cr = CHG ? fma(t3, dotr, st[0]) : t3 * dotr;
-      const TN ci = CHG ? fma(t3, doti, st[1]) : t3 * doti;
-      fxr = fma(ri3, fma(cr, dx, -st[2]), fxr); fxi = fma(ri3, fma(ci, dx, -st[3]), fxi);
-      fyr = fma(ri3, fma(cr, dy, -st[4]), fyr); fyi = fma(ri3, fma(ci, dy, -st[5]), fyi);
-      fzr = fma(ri3, fma(cr, dz, -st[6]), fzr); fzi = fma(ri3, fma(ci, dz, -st[7]), fzi);
+      const TN ri3 = ri * ri2, t3 = pc.c3 * ri2;
+      const TN cr = CHG ? fma(t3, dotr, s.q[0]) : t3 * dotr;
+      const TN ci = CHG ? fma(t3, doti, s.q[1]) : t3 * doti;
+      fxr = fma(ri3, fma(cr, dx, -s.v[0]), fxr); fxi = fma(ri3, fma(ci, dx, -s.v[1]), fxi);
+      fyr = fma(ri3, fma(cr, dy, -s.v[2]), fyr); fyi = fma(ri3, fma(ci, dy, -s.v[3]), fyi);
+      fzr = fma(ri3, fma(cr, dz, -s.v[4]), fzr); fzi = fma(ri3, fma(ci, dz, -s.v[5]), fzi);
     }
     return r2;
   }
@@ -1081,84 +1123,164 @@ __device__ __forceinline__ void redo_run(PairAcc<TN, CHG, DIP, FLD>& acc, double
                                          double* tot) {
   acc = PairAcc<TN, CHG, DIP, FLD>();
   PairAcc<double, CHG, DIP, FLD> c64;
+  const PairConst<double> pc64;
+  const PairConst<TN> pc;
   for (int s = s0; s < s1; s++) {
     const double* sp = spos + 4 * (size_t)s;
     const double dx = xt - sp[0], dy = yt - sp[1], dz = zt - sp[2];
-    if (s != self && fma(dx, dx, fma(dy, dy, dz * dz)) < rc2)
-      c64.add(xt, yt, zt, sp, str64 + 8 * (size_t)s, false);
-    else
-      acc.add(xt, yt, zt, sp, str + 8 * (size_t)s, s == self);
+    if (s != self && fma(dx, dx, fma(dy, dy, dz * dz)) < rc2) {
+      SrcRec<double, CHG, DIP> r;
+      r.load(sp, str64 + 8 * (size_t)s);
+      c64.add(xt, yt, zt, r, false, pc64);
+    } else {
+      SrcRec<TN, CHG, DIP> r;
+      r.load(sp, str + 8 * (size_t)s);
+      acc.add(xt, yt, zt, r, s == self, pc);
+    }
   }
   c64.fold_into(tot);
 }
 
-template <typename TN, bool CHG, bool DIP, bool FLD>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_p2p(DevPlan P, const double* __restrict__ spos,
-                                             const TN* __restrict__ str, const double* __restrict__ str64,
-                                             const double* __restrict__ tpos, int kind, double* __restrict__ pot,
-                                             double* __restrict__ fld) {
-  // one work item (64 points) per wave
-  const int w = __builtin_amdgcn_readfirstlane((int)(xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6)));
-  if (w >= P.n_p2p) return;
-  const int b = P.p2p_items[3 * w], start = P.p2p_items[3 * w + 2];
-  if (b < 0) return;   // padding item
-  const int n0 = kind ? P.itrg[b] : P.isrc[b];
-  const int nn = kind ? P.ntrg[b] : P.nsrc[b];
-  const int i = start + (int)(threadIdx.x & 63);
-  const bool active = i < nn;
-  const int me = n0 + (active ? i : 0);
-  const double* mp = (kind ? tpos : spos) + 4 * (size_t)me;
-  const double x = mp[0], y = mp[1], z = mp[2];
-  double tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-  PairAcc<TN, CHG, DIP, FLD> acc;
+// The pairs of one point with sources s0..s1-1 (s1 > s0; SELF: source `self`
+// is left out).  Two source records are kept: while a pair is computed the
+// next source's scalar loads are in flight.  They return out of order, so the
+// only wait there is waits for all of them: it stands right before the next
+// record's loads are issued, when the one in hand has had a whole pair's
+// arithmetic to arrive.  (FP32 instructions that read a scalar register issue
+// at half the rate of all-vector ones; FP32 strengths staged in LDS and read
+// as vectors were no faster all the same: 12.6 -> 13.4 ms at 1M + 1M.)
+template <typename TN, bool CHG, bool DIP, bool FLD, bool SELF>
+__device__ __forceinline__ void p2p_sources(PairAcc<TN, CHG, DIP, FLD>& acc, const PairConst<TN>& pc, double x, double y,
+                                            double z, const double* __restrict__ spos, const TN* __restrict__ str,
+                                            const double* __restrict__ str64, int s0, int s1, int self, double rc2,
+                                            double* tot) {
   constexpr bool fold = sizeof(TN) < sizeof(double);
-  // FP32 pairs: pairs closer than 1/32 of this leaf's side run in FP64 (on a
-  // uniform 1M cube 0.05 such pairs per point; the near-field error of the
-  // FP32 pairs falls from 1.5e-7 to 8e-8 of the potential, and on a sphere
-  // with a target next to a dipole from 7e-7 to 3e-9)
-  const double hside = 1.0 / P.inv_side[P.level[b]];
-  const double rc2 = fold ? hside * hside * (1.0 / 1024.0) : 0.0;
   const TN rc2n = (TN)rc2, kFar = TN(1e30);
-  // own box first: a source never acts on itself (index test, lfmm3dpart.f:1193)
-  {
-    const int s0 = P.isrc[b], s1 = s0 + P.nsrc[b];
-    const int self = kind ? -1 : me;
-    for (int c = s0; c < s1; c += (fold ? kFold : (1 << 30))) {
-      const int ce = fold ? min(c + kFold, s1) : s1;
-      TN mn = kFar;
-      for (int s = c; s < ce; s++) {
-        const TN r2 = acc.add(x, y, z, spos + 4 * (size_t)s, str + 8 * (size_t)s, s == self);
-        if (fold) mn = fmin(mn, s == self ? kFar : r2);
-      }
-      if (fold) {
-        if (mn < rc2n) redo_run(acc, x, y, z, spos, str, str64, c, ce, self, rc2, tot);
-        acc.fold_into(tot);
+  SrcRec<TN, CHG, DIP> ra, rb;
+  auto arrived = [] {
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto load = [&](SrcRec<TN, CHG, DIP>& r, unsigned s, int k) {  // source s + k
+    r.load(spos + 4 * (size_t)s + 4 * k, str + 8 * (size_t)s + 8 * k);
+  };
+  load(ra, (unsigned)s0, 0);
+  for (int c = s0; c < s1; c += (fold ? kFold : (1 << 30))) {
+    const int ce = fold ? min(c + kFold, s1) : s1;
+    TN mn = kFar;
+    auto pair = [&](const SrcRec<TN, CHG, DIP>& r, int s) {
+      __builtin_amdgcn_sched_barrier(0);
+      const TN r2 = acc.add(x, y, z, r, SELF && s == self, pc);
+      if (fold) mn = fmin(mn, SELF && s == self ? kFar : r2);
+    };
+    // ra holds source s; kFold is even, so it does at every run's start
+    int s = c;
+    const int lim = min(ce, s1 - 2);
+    for (; s < lim; s += 2) {
+      // (the index, not pointers, is what the loop carries: carried pointers
+      // ended up in vector registers, six readfirstlane per pair)
+      const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane(s);
+      arrived();
+      load(rb, u, 1);
+      pair(ra, s);
+      arrived();
+      load(ra, u, 2);
+      pair(rb, s + 1);
+    }
+    if (s < ce) {  // the last one or two of s0..s1-1: nothing past them is read
+      arrived();
+      if (s + 1 < ce) {
+        load(rb, (unsigned)s, 1);
+        pair(ra, s);
+        arrived();
+        pair(rb, s + 1);
+      } else {
+        pair(ra, s);
       }
     }
-  }
-  for (int jj = P.l1_off[b]; jj < P.l1_off[b + 1]; jj++) {
-    const int j = P.l1_idx[jj];
-    const int s0 = P.isrc[j], s1 = s0 + P.nsrc[j];
-    for (int c = s0; c < s1; c += (fold ? kFold : (1 << 30))) {
-      const int ce = fold ? min(c + kFold, s1) : s1;
-      TN mn = kFar;
-#pragma unroll 4
-      for (int s = c; s < ce; s++) {
-        const TN r2 = acc.add(x, y, z, spos + 4 * (size_t)s, str + 8 * (size_t)s, false);
-        if (fold) mn = fmin(mn, r2);
-      }
-      if (fold) {
-        if (mn < rc2n) redo_run(acc, x, y, z, spos, str, str64, c, ce, -1, rc2, tot);
-        acc.fold_into(tot);
-      }
+    if (fold) {
+      if (mn < rc2n) redo_run(acc, x, y, z, spos, str, str64, c, ce, SELF ? self : -1, rc2, tot);
+      acc.fold_into(tot);
     }
   }
-  if (!fold) acc.fold_into(tot);
+}
+
+template <typename TN, bool CHG, bool DIP, bool FLD>
+__global__ __launch_bounds__(64 * kP2PSplit) __attribute__((amdgpu_waves_per_eu(sizeof(TN) == 4 ? 6 : 8))) void k_p2p(DevPlan P, const double* __restrict__ spos,
+                                             const TN* __restrict__ str, const double* __restrict__ str64,
+                                             const double* __restrict__ tpos, double* __restrict__ pot0,
+                                             double* __restrict__ fld0, double* __restrict__ pot1,
+                                             double* __restrict__ fld1) {
+  const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+  const int w = xcd_block();  // one work item per workgroup
+  const int b = P.p2p_items[3 * w], kind = P.p2p_items[3 * w + 1], start = P.p2p_items[3 * w + 2];
+  double tot[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  bool active = false;
+  int me = 0;
+  if (b >= 0) {  // not a padding item
+    const int n0 = kind ? P.itrg[b] : P.isrc[b];
+    const int nn = kind ? P.ntrg[b] : P.nsrc[b];
+    const int i = start + lane;
+    active = i < nn;
+    me = n0 + (active ? i : 0);
+    const double* mp = (kind ? tpos : spos) + 4 * (size_t)me;
+    const double x = mp[0], y = mp[1], z = mp[2];
+    PairAcc<TN, CHG, DIP, FLD> acc;
+    const PairConst<TN> pc;
+    constexpr bool fold = sizeof(TN) < sizeof(double);
+    // FP32 pairs: pairs closer than 1/32 of this leaf's side run in FP64 (on a
+    // uniform 1M cube 0.05 such pairs per point; the near-field error of the
+    // FP32 pairs falls from 1.5e-7 to 8e-8 of the potential, and on a sphere
+    // with a target next to a dipole from 7e-7 to 3e-9)
+    const double hside = 1.0 / P.inv_side[P.level[b]];
+    const double rc2 = fold ? hside * hside * (1.0 / 1024.0) : 0.0;
+    // this wave's part of a box's sources
+    auto cut = [&](int s0, int n, int q) { return s0 + (int)((long)n * q / kP2PSplit); };
+    // own box first: a source never acts on itself (index test, lfmm3dpart.f:1193)
+    if (kind == 0) {
+      const int s0 = P.isrc[b], n = P.nsrc[b];
+      const int a = cut(s0, n, part), e = cut(s0, n, part + 1);
+      if (a < e) p2p_sources<TN, CHG, DIP, FLD, true>(acc, pc, x, y, z, spos, str, str64, a, e, me, rc2, tot);
+    }
+    const int l0 = P.l1_off[b], l1 = P.l1_off[b + 1];
+    for (int jj = kind == 0 ? l0 : l0 - 1; jj < l1; jj++) {  // targets: their own box, then list 1
+      const int j = jj < l0 ? b : P.l1_idx[jj];
+      const int s0 = P.isrc[j], n = P.nsrc[j];
+      const int a = cut(s0, n, part), e = cut(s0, n, part + 1);
+      if (a < e) p2p_sources<TN, CHG, DIP, FLD, false>(acc, pc, x, y, z, spos, str, str64, a, e, -1, rc2, tot);
+    }
+    if (!fold) acc.fold_into(tot);
+  }
+  // the parts' sums, added in order by the item's first wave, two values at a
+  // time: LDS kept small, since far-field workgroups that need much of it run
+  // beside this kernel (with all eight values at once, 16 KB a workgroup, P2M
+  // waited for the whole near field)
+  constexpr int W = FLD ? 8 : 2;
+  __shared__ double sums[kP2PSplit - 1][2][64];
+#pragma unroll
+  for (int k0 = 0; k0 < W; k0 += 2) {
+    if (k0) __syncthreads();
+    if (part > 0) {
+      sums[part - 1][0][lane] = tot[k0];
+      sums[part - 1][1][lane] = tot[k0 + 1];
+    }
+    __syncthreads();
+    if (part == 0)
+      for (int q = 0; q < kP2PSplit - 1; q++) {
+        tot[k0] += sums[q][0][lane];
+        tot[k0 + 1] += sums[q][1][lane];
+      }
+  }
+  if (part > 0) return;
   if (!active) return;
-  pot[2 * (size_t)me] += tot[0];
-  pot[2 * (size_t)me + 1] += tot[1];
-  if (FLD)
-    for (int k = 0; k < 6; k++) fld[6 * (size_t)me + k] += tot[2 + k];
+  double* po = kind ? pot1 : pot0;
+  po[2 * (size_t)me] += tot[0];
+  po[2 * (size_t)me + 1] += tot[1];
+  if (FLD) {
+    double* fo = kind ? fld1 : fld0;
+    for (int k = 0; k < 6; k++) fo[6 * (size_t)me + k] += tot[2 + k];
+  }
 }
 
 // Plain direct sum over all sources (l3dpartdirect, src/lfmm3dpart.f:1391):
@@ -1174,8 +1296,13 @@ __global__ __launch_bounds__(256) void k_direct(int ns, const double* __restrict
   const double* mp = (pts_are_sources ? spos : pts) + 4 * (size_t)me;
   const double x = mp[0], y = mp[1], z = mp[2];
   PairAcc<double, CHG, DIP, true> acc;
+  const PairConst<double> pc;
   const int self = pts_are_sources ? me : -1;
-  for (int s = 0; s < ns; s++) acc.add(x, y, z, spos + 4 * (size_t)s, str + 8 * (size_t)s, s == self);
+  for (int s = 0; s < ns; s++) {
+    SrcRec<double, CHG, DIP> r;
+    r.load(spos + 4 * (size_t)s, str + 8 * (size_t)s);
+    acc.add(x, y, z, r, s == self, pc);
+  }
   if (!active) return;
   double t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   acc.fold_into(t);

@@ -131,8 +131,14 @@ inline void build_plan_near(const Octree& t, const Flags& f, Flat& F, PlanOffset
     if (want_src) push_items(p2p0, b, 0, t.nsrc[b]);
     if (want_trg) push_items(p2p1, b, 1, t.ntrg[b]);
   }
-  O.p2p0 = F.i(p2p0); O.n_p2p0 = (int)p2p0.size() / 3;
-  O.p2p1 = F.i(p2p1); O.n_p2p1 = (int)p2p1.size() / 3;
+  // one list, sources then targets, so that one launch can run both; the
+  // targets start a workgroup of their own
+  while ((p2p0.size() / 3) % kItemWaves != 0) { p2p0.push_back(-1); p2p0.push_back(0); p2p0.push_back(0); }
+  O.n_p2p0 = (int)p2p0.size() / 3;
+  O.n_p2p1 = (int)p2p1.size() / 3;
+  p2p0.insert(p2p0.end(), p2p1.begin(), p2p1.end());
+  O.p2p0 = F.i(p2p0);
+  O.p2p1 = O.p2p0 + 3 * (size_t)O.n_p2p0;
 }
 
 // Part B2: lists 2-4 and the work lists of the far-field steps (needs all lists).
