@@ -1210,24 +1210,29 @@ __global__ __launch_bounds__(256) void k_hp2p(DevPlan P, double kre, double kim,
     for (int k = 0; k < 6; k++) fld[6 * (size_t)me + k] += tot[2 + k];
 }
 
-// h3dpartdirect (src/hfmm3dpart.f:1268): every source on every point
+// h3dpartdirect (src/hfmm3dpart.f:1268): every source on every point, split over
+// waves and slices like the Laplace k_direct
 template <bool CHG, bool DIP>
-__global__ __launch_bounds__(256) void k_hdirect(double kre, double kim, int ns, const double* __restrict__ spos,
-                                                 const double* __restrict__ str, int npts,
-                                                 const double* __restrict__ pts, int pts_are_sources,
-                                                 double* __restrict__ pot, double* __restrict__ fld) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(64 * kDirectWaves) void k_hdirect(double kre, double kim, int ns,
+                                                               const double* __restrict__ spos,
+                                                               const double* __restrict__ str, int npts,
+                                                               const double* __restrict__ pts, int pts_are_sources,
+                                                               double* __restrict__ partial, double* __restrict__ pot,
+                                                               double* __restrict__ fld) {
+  const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
+  const int i = 64 * blockIdx.x + lane;
   const bool active = i < npts;
   const int me = active ? i : 0;
   const double* mp = (pts_are_sources ? spos : pts) + 4 * (size_t)me;
   const double x = mp[0], y = mp[1], z = mp[2];
   HPairAcc<double, CHG, DIP, true> acc;
   const int self = pts_are_sources ? me : -1;
-  for (int s = 0; s < ns; s++) acc.add(kre, kim, x, y, z, spos + 4 * (size_t)s, str + 8 * (size_t)s, s == self);
-  if (!active) return;
-  pot[2 * (size_t)i] = acc.a[0];
-  pot[2 * (size_t)i + 1] = acc.a[1];
-  for (int k = 0; k < 6; k++) fld[6 * (size_t)i + k] = acc.a[2 + k];
+  const int s0 = direct_cut(ns, part), s1 = direct_cut(ns, part + 1);
+  for (int s = s0; s < s1; s++) acc.add(kre, kim, x, y, z, spos + 4 * (size_t)s, str + 8 * (size_t)s, s == self);
+  double t[8];
+  for (int k = 0; k < 8; k++) t[k] = acc.a[k];
+  add_parts<kDirectWaves, 8>(t, part, lane);
+  if (part == 0 && active) direct_store(t, i, npts, partial, pot, fld);
 }
 
 }  // namespace fmm3d

@@ -179,6 +179,65 @@ static __global__ void k_scatter_sum(int n, int w, const int* __restrict__ perm,
     out[(size_t)2 * w * o + k] = far[(size_t)2 * w * i + k] + near[(size_t)2 * w * i + k];
 }
 
+// The sums of a workgroup's NW waves over the same 64 points, added in order by
+// the first wave, two values at a time: LDS kept small, since far-field
+// workgroups that need much of it run beside the near field (with all eight
+// values at once, 16 KB a workgroup, P2M waited for the whole near field)
+template <int NW, int W>
+__device__ __forceinline__ void add_parts(double (&tot)[8], int part, int lane) {
+  __shared__ double sums[NW - 1][2][64];
+#pragma unroll
+  for (int k0 = 0; k0 < W; k0 += 2) {
+    if (k0) __syncthreads();
+    if (part > 0) {
+      sums[part - 1][0][lane] = tot[k0];
+      sums[part - 1][1][lane] = tot[k0 + 1];
+    }
+    __syncthreads();
+    if (part == 0)
+      for (int q = 0; q < NW - 1; q++) {
+        tot[k0] += sums[q][0][lane];
+        tot[k0 + 1] += sums[q][1][lane];
+      }
+  }
+}
+
+// Direct sums: waves per workgroup, each with its part of the workgroup's slice
+// of the sources, and slices so that about 8,192 waves run (eight on each SIMD)
+// where each still has 64 sources.
+constexpr int kDirectWaves = 4;
+static inline int direct_slices(int npts, int ns) {
+  const int items = (npts + 63) / 64, want = (8192 / kDirectWaves + items - 1) / items;
+  const int most = ns / (64 * kDirectWaves);
+  return want < most ? want : most > 1 ? most : 1;
+}
+// first source of part q of this workgroup's slice
+__device__ __forceinline__ int direct_cut(int ns, int q) {
+  return (int)((long)ns * (blockIdx.y * kDirectWaves + q) / (gridDim.y * kDirectWaves));
+}
+// one slice: the result itself; several: to `partial`, eight values per point
+__device__ __forceinline__ void direct_store(const double (&t)[8], int i, int npts, double* __restrict__ partial,
+                                             double* __restrict__ pot, double* __restrict__ fld) {
+  if (gridDim.y > 1) {
+    for (int k = 0; k < 8; k++) partial[8 * ((size_t)blockIdx.y * npts + i) + k] = t[k];
+    return;
+  }
+  pot[2 * (size_t)i] = t[0];
+  pot[2 * (size_t)i + 1] = t[1];
+  for (int k = 0; k < 6; k++) fld[6 * (size_t)i + k] = t[2 + k];
+}
+static __global__ void k_direct_sum(int npts, int nsl, const double* __restrict__ partial, double* __restrict__ pot,
+                                    double* __restrict__ fld) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= npts) return;
+  double t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  for (int q = 0; q < nsl; q++)
+    for (int k = 0; k < 8; k++) t[k] += partial[8 * ((size_t)q * npts + i) + k];
+  pot[2 * (size_t)i] = t[0];
+  pot[2 * (size_t)i + 1] = t[1];
+  for (int k = 0; k < 6; k++) fld[6 * (size_t)i + k] = t[2 + k];
+}
+
 // Sums of the list-3 slices of one evaluation item (box, kind, first point,
 // first slice, number of slices), 8 values per point (pot, d/dz, U, D as
 // complex), added in slice order to the outputs: pot += pot, fld -= grad
