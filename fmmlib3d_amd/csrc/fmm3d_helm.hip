@@ -393,9 +393,12 @@ int helm_solve(Context& ctx, const LapCall& c) {
   form(std::false_type{}, P.n_p2m, mp);
   tm.mark(2);
   // STEP 3: M2M, bottom-up
-  for (size_t g = 0; g < O.m2m_groups.size(); g++)
-    hipLaunchKernelGGL(k_hm2m, dim3(O.m2m_groups[g].second), dim3(256), lds_ps, s, P, Tb, Hd,
-                       O.m2m_groups[g].first, HC->m2m_base + O.m2m_group_level[g], mp);
+  for (size_t g = 0; g < O.m2m_groups.size(); g++) {
+    hipLaunchKernelGGL(k_hm2m, dim3(O.m2m_groups[g].second, 8), dim3(256), lds_ps, s, P, Tb, Hd,
+                       O.m2m_groups[g].first, HC->m2m_base + O.m2m_group_level[g], mp, lo);
+    hipLaunchKernelGGL((k_child_sum<double>), dim3(O.m2m_groups[g].second), dim3(256), 0, s, P,
+                       O.m2m_groups[g].first, mp, lo);
+  }
   tm.mark(3);
   // while the device runs P2M and M2M: list 1 and the P2P plan
   auto t_lists0 = std::chrono::steady_clock::now();
@@ -465,7 +468,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
   tm.mark(6);
   // STEP 5: L2L, top-down
   for (size_t g = 0; g < O.l2l_groups.size(); g++)
-    hipLaunchKernelGGL(k_hl2l, dim3(O.l2l_groups[g].second), dim3(256), lds_ps, s, P, Tb, Hd,
+    hipLaunchKernelGGL(k_hl2l, dim3(O.l2l_groups[g].second, 8), dim3(256), lds_ps, s, P, Tb, Hd,
                        O.l2l_groups[g].first, HC->l2l_base + O.l2l_group_level[g], lo);
   tm.mark(7);
   // STEP 7: L2P and STEP 6: M2P (list 3), from packed expansions

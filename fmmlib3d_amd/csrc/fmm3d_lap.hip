@@ -467,8 +467,10 @@ int lap_solve(Context& ctx, const LapCall& c) {
   mark(2);
   // ---- STEP 3: M2M, bottom-up
   const size_t lds_ps = sizeof(T) * 4 * K;
-  for (auto& g : O.m2m_groups)
-    hipLaunchKernelGGL((k_m2m<T>), dim3(g.second), dim3(256), lds_ps, s, P, Tb, g.first, mp);
+  for (auto& g : O.m2m_groups) {
+    hipLaunchKernelGGL((k_m2m<T>), dim3(g.second, 8), dim3(256), lds_ps, s, P, Tb, g.first, mp, lo);
+    hipLaunchKernelGGL((k_child_sum<T>), dim3(g.second), dim3(256), 0, s, P, g.first, mp, lo);
+  }
   mark(3);
   // ---- while the device runs P2M and M2M: list 1 and the P2P plan (part B1)
   auto t_lists0 = std::chrono::steady_clock::now();
@@ -601,7 +603,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   mark(6);
   // ---- STEP 5: L2L, top-down
   for (auto& g : O.l2l_groups)
-    hipLaunchKernelGGL((k_l2l<T>), dim3(g.second), dim3(256), lds_ps, s, P, Tb, g.first, lo);
+    hipLaunchKernelGGL((k_l2l<T>), dim3(g.second, 8), dim3(256), lds_ps, s, P, Tb, g.first, lo);
   mark(7);
   // ---- STEP 7: L2P (packed local + gradient expansions, wave-uniform reads)
   if (P.n_l2p) {

@@ -921,39 +921,40 @@ __device__ void hpoint_and_shoot(const DevTables& Tb, const HelmDev& Hd, int rc,
   __syncthreads();
 }
 
-// M2M into the parents of one level (src/hfmm3drouts.f:193-266)
-__global__ void k_hm2m(DevPlan P, DevTables Tb, HelmDev Hd, int first, int tab, double* __restrict__ mp) {
+// M2M into the parents of one level (src/hfmm3drouts.f:193-266), one workgroup
+// per child, into the child's local (then k_child_sum), like the Laplace k_m2m
+__global__ void k_hm2m(DevPlan P, DevTables Tb, HelmDev Hd, int first, int tab, const double* __restrict__ mp,
+                       double* __restrict__ lo) {
   extern __shared__ unsigned char smem_raw[];
   double* A = reinterpret_cast<double*>(smem_raw);
   double* B = A + 2 * P.K;
-  const int b = P.m2m_boxes[first + blockIdx.x];
+  const int b = P.m2m_boxes[first + blockIdx.x], c = blockIdx.y;
   const int lev = P.level[b];
   const int pp = Hd.plev[lev], pc = Hd.plev[lev + 1];
-  for (int c = 0; c < P.nchild[b]; c++) {
-    const int ch = P.child[8 * b + c];
-    if (P.nsrc[ch] == 0) continue;
-    const int o = (P.ijk[3 * ch] & 1 ? 0 : 1) | (P.ijk[3 * ch + 1] & 1 ? 0 : 2) | (P.ijk[3 * ch + 2] & 1 ? 0 : 4);
-    const double* ph = Tb.oct_phase + (size_t)(o * 2 + 0) * 2 * (Tb.p + 1);
-    hpoint_and_shoot(Tb, Hd, Tb.oct_rot[o * 2 + 0], ph, tab, pc, pp, mp + 2 * (size_t)ch * P.K,
-                     mp + 2 * (size_t)b * P.K, A, B);
-  }
+  if (c >= P.nchild[b]) return;
+  const int ch = P.child[8 * b + c];
+  if (P.nsrc[ch] == 0) return;
+  const int o = (P.ijk[3 * ch] & 1 ? 0 : 1) | (P.ijk[3 * ch + 1] & 1 ? 0 : 2) | (P.ijk[3 * ch + 2] & 1 ? 0 : 4);
+  const double* ph = Tb.oct_phase + (size_t)(o * 2 + 0) * 2 * (Tb.p + 1);
+  hpoint_and_shoot(Tb, Hd, Tb.oct_rot[o * 2 + 0], ph, tab, pc, pp, mp + 2 * (size_t)ch * P.K,
+                   lo + 2 * (size_t)ch * P.K, A, B);
 }
 
-// L2L from the parents of one level (src/hfmm3drouts.f:483-556)
+// L2L from the parents of one level (src/hfmm3drouts.f:483-556), one workgroup
+// per child
 __global__ void k_hl2l(DevPlan P, DevTables Tb, HelmDev Hd, int first, int tab, double* __restrict__ lo) {
   extern __shared__ unsigned char smem_raw[];
   double* A = reinterpret_cast<double*>(smem_raw);
   double* B = A + 2 * P.K;
-  const int b = P.l2l_boxes[first + blockIdx.x];
+  const int b = P.l2l_boxes[first + blockIdx.x], c = blockIdx.y;
   const int lev = P.level[b];
   const int pp = Hd.plev[lev], pc = Hd.plev[lev + 1];
-  for (int c = 0; c < P.nchild[b]; c++) {
-    const int ch = P.child[8 * b + c];
-    const int o = (P.ijk[3 * ch] & 1 ? 0 : 1) | (P.ijk[3 * ch + 1] & 1 ? 0 : 2) | (P.ijk[3 * ch + 2] & 1 ? 0 : 4);
-    const double* ph = Tb.oct_phase + (size_t)(o * 2 + 1) * 2 * (Tb.p + 1);
-    hpoint_and_shoot(Tb, Hd, Tb.oct_rot[o * 2 + 1], ph, tab, pp, pc, lo + 2 * (size_t)b * P.K,
-                     lo + 2 * (size_t)ch * P.K, A, B);
-  }
+  if (c >= P.nchild[b]) return;
+  const int ch = P.child[8 * b + c];
+  const int o = (P.ijk[3 * ch] & 1 ? 0 : 1) | (P.ijk[3 * ch + 1] & 1 ? 0 : 2) | (P.ijk[3 * ch + 2] & 1 ? 0 : 4);
+  const double* ph = Tb.oct_phase + (size_t)(o * 2 + 1) * 2 * (Tb.p + 1);
+  hpoint_and_shoot(Tb, Hd, Tb.oct_rot[o * 2 + 1], ph, tab, pp, pc, lo + 2 * (size_t)b * P.K,
+                   lo + 2 * (size_t)ch * P.K, A, B);
 }
 
 // M2L over the pruned list 2 of each target box (src/hfmm3drouts.f:330-477);

@@ -179,6 +179,26 @@ static __global__ void k_scatter_sum(int n, int w, const int* __restrict__ perm,
     out[(size_t)2 * w * o + k] = far[(size_t)2 * w * i + k] + near[(size_t)2 * w * i + k];
 }
 
+// The second half of M2M: a parent's multipole gains its children's translated
+// expansions, which lie in the children's locals, in order; the locals are zero
+// again afterwards.
+template <typename T>
+__global__ void k_child_sum(DevPlan P, int first, T* __restrict__ mp, T* __restrict__ lo) {
+  const int b = P.m2m_boxes[first + blockIdx.x], n = P.nchild[b];
+  for (int k = threadIdx.x; k < 2 * P.K; k += blockDim.x) {
+    T v[8], s = mp[2 * (size_t)b * P.K + k];
+#pragma unroll
+    for (int c = 0; c < 8; c++) v[c] = c < n ? lo[2 * (size_t)P.child[8 * b + c] * P.K + k] : T(0);
+#pragma unroll
+    for (int c = 0; c < 8; c++)
+      if (c < n) {
+        s += v[c];
+        lo[2 * (size_t)P.child[8 * b + c] * P.K + k] = T(0);
+      }
+    mp[2 * (size_t)b * P.K + k] = s;
+  }
+}
+
 // The sums of a workgroup's NW waves over the same 64 points, added in order by
 // the first wave, two values at a time: LDS kept small, since far-field
 // workgroups that need much of it run beside the near field (with all eight
