@@ -50,16 +50,16 @@ SEED = 2
 FP64_PEAK_TFLOPS = 78.6        # MI355X FP64 vector (= FP64 matrix) peak
 FP32_PEAK_TFLOPS = 157.3       # MI355X FP32 vector peak (packed)
 FLOPS_PER_PAIR = 65            # charge+dipole, pot+fld, rsqrt counted as 2
-# HBM bytes per k_p2p launch on this workload, from rocprofv3 FETCH_SIZE and
+# HBM bytes of the k_p2p launch on this workload, from rocprofv3 FETCH_SIZE and
 # WRITE_SIZE runs calibrated against a 1 GiB device copy
-# (profiles/fmm_kernels_lap1M_helm500k.md): 2 x FETCH KiB + WRITE KiB.
-P2P_TRAFFIC_BYTES = {"fp64": (2 * 2674172 + 62877) * 1024, "fp32": (2 * 1212368 + 88665) * 1024}
+# (profiles/m2l_p2p_counters_lap1M.md): 2 x FETCH KiB + WRITE KiB.
+P2P_TRAFFIC_BYTES = {"fp64": (2 * 3202000 + 126100) * 1024, "fp32": (2 * 927100 + 343700) * 1024}
 # VALU lane instructions per pair in k_p2p on this workload, from rocprofv3
-# SQ_INSTS_VALU (wave64 instructions x 64 / pairs; profiles/valu_mfma_counters_lap1M.md).
+# SQ_INSTS_VALU (wave64 instructions x 64 / pairs; profiles/m2l_p2p_counters_lap1M.md).
 # A wave64 VALU instruction occupies its SIMD for 4 cycles; the chip has
 # 256 CUs x 4 SIMDs at 2.4 GHz, so the issue-time ceiling of a launch is
 # pairs x this / 64 x 4 / (1024 x 2.4e9) seconds.
-P2P_VALU_INSTR_PER_PAIR = {"fp64": 43.2, "fp32": 44.3}
+P2P_VALU_INSTR_PER_PAIR = {"fp64": 43.4, "fp32": 44.4}
 SIMD_CYCLES_PER_S = 1024 * 2.4e9
 
 
@@ -623,7 +623,7 @@ def main():
                    "inputs": "device-resident (fmm3d_lfmm3dparttarg_dev)"},
         "p50_ms": M["p50_ms"], "p99_ms": M["p99_ms"],
         "rel_err_vs_fp64_direct": {"pottarg": M["err_pottarg"], "fldtarg": M["err_fldtarg"], "sampled_targets": 1000},
-        "roofline": {"kernel": "k_p2p (near field, both launches)", "bound": "valu", "achieved": achieved,
+        "roofline": {"kernel": "k_p2p (near field, one launch for sources and targets)", "bound": "valu", "achieved": achieved,
                      "peak": peak, "unit": "TFLOP/s", "frac": achieved / peak,
                      "achieved_alone": achieved_alone, "frac_alone": achieved_alone / peak,
                      "p2p_ms": M["p2p_ms"], "p2p_ms_alone": p2p_alone_ms,
@@ -631,10 +631,10 @@ def main():
                      "valu_issue_frac": issue_s / (M["p2p_ms"] * 1e-3),
                      "valu_issue_frac_alone": issue_s / (p2p_alone_ms * 1e-3),
                      "note": "P2P is VALU bound (no matrix-core form); peak = the vector peak of the pair "
-                             "arithmetic's type. Both launches run on the second stream beside the far-field "
-                             "kernels and are timed with HIP events on that stream; *_alone: the same launches "
+                             "arithmetic's type. It runs on the second stream beside the far-field "
+                             "kernels and is timed with HIP events on that stream; *_alone: the same launch "
                              "with the near field on the caller's stream (FMM3D_NEAR_STREAM=0), 2 extra steps. "
-                             "algorithmic flops = %d pairs x %d. valu_issue_frac: time the launches' VALU "
+                             "algorithmic flops = %d pairs x %d. valu_issue_frac: time the launch's VALU "
                              "instructions (%.1f per pair, rocprofv3 SQ_INSTS_VALU) need at one wave64 instruction "
                              "per 4 cycles per SIMD, 1024 SIMDs, 2.4 GHz, over the measured time; FP32 peak "
                              "counts packed FP32, which this build does not emit"
