@@ -89,21 +89,18 @@ void helm_upload_gaunt(Context& ctx, HelmCache& c, const std::shared_ptr<const G
   c.gaunt = g;
 }
 
-HelmCache* helm_tables(Context& ctx, cplx zk, double size, int nlev, double eps, int& ier) {
-  ier = 0;
-  if (!ctx.helm_tables) ctx.helm_tables = std::make_shared<HelmCache>();
-  HelmCache& c = *static_cast<HelmCache*>(ctx.helm_tables.get());
-  if (c.valid && c.H.zk == zk && c.H.size == size && c.H.nlev == nlev && c.H.eps == eps) return &c;
+// The tables of the plan H on the device: queues on ctx.stream what this
+// context does not hold yet.  H's orders have been checked against what the
+// kernels take: a call that is refused queues nothing and keeps the tables of
+// the call before it.
+HelmCache& helm_upload_tables(Context& ctx, HelmCache& c, HelmHostTables&& plan) {
   c.valid = false;
-  if (!plan_helm_tables(zk, size, nlev, eps, c.H)) {
-    ier = 16;
-    return nullptr;
-  }
+  c.H = std::move(plan);
   const HelmHostTables& H = c.H;
   if (c.geo != H.geo) helm_upload_geometry(ctx, c, H.geo);
   const auto gaunt = gaunt_for(H.pmax);
   if (c.gaunt != gaunt) helm_upload_gaunt(ctx, c, gaunt);
-  const int nd = H.geo->ndist, P1 = H.pmax + 1;
+  const int nd = H.geo->ndist, P1 = H.pmax + 1, nlev = H.nlev;
   std::vector<int> I;
   std::vector<double> D;
   std::vector<long> L;
@@ -148,7 +145,7 @@ HelmCache* helm_tables(Context& ctx, cplx zk, double size, int nlev, double eps,
   c.cI = I.size(); c.cD = D.size(); c.cL = L.size();
   c.cZ = c.o_zt + (size_t)nt;
   // small enough to go through one pinned buffer (the call before this one on
-  // the context has finished with it)
+  // the context has finished with it, whichever way it ended: QueuedWork)
   const size_t bI = I.size() * sizeof(int), bD = D.size() * sizeof(double), bL = L.size() * sizeof(long),
                bJ = H.jobs.size() * sizeof(CoaxJob);
   char* h = (char*)ctx.arena.get_host("htab_h", bD + bL + bJ + bI);
@@ -172,7 +169,7 @@ HelmCache* helm_tables(Context& ctx, cplx zk, double size, int nlev, double eps,
                        dl + c.o_ztoff, P1, dz, dz + c.o_zt);
   FMM_HIP(hipGetLastError());
   c.valid = true;
-  return &c;
+  return c;
 }
 
 template <typename TN, bool CHG, bool DIP, bool FLD>
@@ -218,6 +215,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
   const int ns = c.ns, nt = c.nt;
   const Flags f{c.ifcharge ? 1 : 0, c.ifdipole ? 1 : 0, c.ifpot ? 1 : 0, c.iffld ? 1 : 0,
                 nt > 0 && c.ifpottarg ? 1 : 0, nt > 0 && c.iffldtarg ? 1 : 0};
+  QueuedWork queued(ctx);
   thread_local Octree tree;  // storage reused across calls
   const int* dsperm = nullptr;
   const int* dtperm = nullptr;
@@ -229,11 +227,14 @@ int helm_solve(Context& ctx, const LapCall& c) {
     return 4;
   }
   auto t_tree = std::chrono::steady_clock::now();
-  int ier = 0;
-  HelmCache* HC = helm_tables(ctx, zk, tree.size, tree.nlev, eps, ier);
-  if (!HC) return ier;
-  const HelmHostTables& H = HC->H;
-  const int pmax = H.pmax, K = (pmax + 1) * (pmax + 1);
+  // the tables this context holds, or a plan of new ones; nothing is queued
+  // for them until the order has been checked
+  if (!ctx.helm_tables) ctx.helm_tables = std::make_shared<HelmCache>();
+  HelmCache* HC = static_cast<HelmCache*>(ctx.helm_tables.get());
+  const bool held = HC->valid && HC->H.zk == zk && HC->H.size == tree.size && HC->H.nlev == tree.nlev && HC->H.eps == eps;
+  HelmHostTables plan;
+  if (!held && !plan_helm_tables(zk, tree.size, tree.nlev, eps, plan)) return 16;
+  const int pmax = held ? HC->H.pmax : plan.pmax, K = (pmax + 1) * (pmax + 1);
   // LDS budgets of the kernels at this order
   const size_t ldsmax = max_lds_bytes(ctx);
   const int Hh = (pmax + 2) * (pmax + 3) / 2, Fn = pmax + 2;
@@ -254,6 +255,10 @@ int helm_solve(Context& ctx, const LapCall& c) {
   const size_t lds_ps = sizeof(double) * 4 * (size_t)K;
   const bool m2l_lds = sizeof(double) * 6 * (size_t)K <= ldsmax;
   if (lds_ps > ldsmax) return 16;
+  auto lds_eval = [](int pd) { return sizeof(double) * 2 * 64 * (size_t)(pd + 2); };  // k_heval3 (L2P) at degree pd
+  if (lds_eval(pmax + 1) > ldsmax) return 16;
+  if (!held) helm_upload_tables(ctx, *HC, std::move(plan));
+  const HelmHostTables& H = HC->H;
   thread_local Flat FA, FB, FC;  // plan parts: boxes, near lists, far lists (storage reused)
   FA.I.clear(); FA.D.clear(); FB.I.clear(); FB.D.clear(); FC.I.clear(); FC.D.clear();
   PlanOffsets O;
@@ -544,13 +549,11 @@ int helm_solve(Context& ctx, const LapCall& c) {
     std::memcpy(hh, hv.data(), hv.size() * sizeof(int));
     int* dh = (int*)ctx.arena.get("heval_i", std::max<size_t>(hv.size(), 1) * sizeof(int));
     FMM_HIP(hipMemcpyAsync(dh, hh, hv.size() * sizeof(int), hipMemcpyHostToDevice, s));
-    const size_t lds3 = sizeof(double) * 2 * 64 * (size_t)(pdmax + 2);
-    if (lds3 > ldsmax) return 16;
     if (!it_l.empty()) {
       double* pack = (double*)ctx.arena.get("hpack_l", sizeof(double) * 16 * (size_t)std::max(tot_l, 1));
       hipLaunchKernelGGL((k_hpack<false>), dim3((unsigned)pk_l.size()), dim3(256), 0, s, P, Hd, fac, lo, dh + o_pl,
                          dh + o_ol, grad, pack);
-      hipLaunchKernelGGL((k_heval3<false>), dim3((unsigned)(it_l.size() / 3)), dim3(64), lds3, s, P, Hd, fac, pack,
+      hipLaunchKernelGGL((k_heval3<false>), dim3((unsigned)(it_l.size() / 3)), dim3(64), lds_eval(pdmax), s, P, Hd, fac, pack,
                          dh + o_sl, dh + o_il, grad, spos, tpos, f.ifpot, f.iffld, f.ifpottarg, f.iffldtarg, pot_s,
                          fld_s, pot_t, fld_t, (double*)nullptr);
     }
@@ -581,7 +584,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
   if (f.iffldtarg) scatter(nt, 3, tperm, fld_t, fld_tn, c.fldtarg_dev);
   tm.mark(10);
   FMM_HIP(hipGetLastError());
-  FMM_HIP(hipStreamSynchronize(s));
+  queued.wait();
   auto& lt = last_timings();
   lt.assign(13, 0.0);
   auto ms = [](auto a, auto b) { return std::chrono::duration<double, std::milli>(b - a).count(); };
@@ -673,6 +676,7 @@ int htri_direct(Context& ctx, const LapCall& c) {
   const int n = c.ns, nt = c.nt;
   const std::vector<double>& sr = tri_sym_rule(c.tri_nqtri);
   if (sr.empty() || sr.size() / 3 > (size_t)kSymRuleMax) return 128;
+  QueuedWork queued(ctx);
   hipStream_t s = ctx.stream;
   double* hr = (double*)ctx.arena.get_host("htri_rule_h", sizeof(double) * 3 * kSymRuleMax);
   std::memcpy(hr, sr.data(), sizeof(double) * sr.size());
@@ -709,7 +713,7 @@ int htri_direct(Context& ctx, const LapCall& c) {
   run(n, c.src_dev, 1, c.ifpot, c.pot_dev, c.iffld, c.fld_dev);
   run(nt, c.trg_dev, 0, c.ifpottarg, c.pottarg_dev, c.iffldtarg, c.fldtarg_dev);
   FMM_HIP(hipGetLastError());
-  FMM_HIP(hipStreamSynchronize(s));
+  queued.wait();
   return 0;
 }
 

@@ -226,6 +226,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   const int ns = c.ns, nt = c.nt;
   const Flags f{c.ifcharge ? 1 : 0, c.ifdipole ? 1 : 0, c.ifpot ? 1 : 0, c.iffld ? 1 : 0,
                 nt > 0 && c.ifpottarg ? 1 : 0, nt > 0 && c.iffldtarg ? 1 : 0};
+  QueuedWork queued(ctx);
   thread_local Octree own_tree;  // storage reused across calls
   Octree& tree = c.tree_in ? const_cast<Octree&>(*c.tree_in) : own_tree;
   const bool prebuilt = c.tree_in != nullptr;
@@ -757,7 +758,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
     FMM_HIP(e2);
   }
   FMM_HIP(hipGetLastError());
-  FMM_HIP(hipStreamSynchronize(s));
+  queued.wait();
   auto& lt = last_timings();
   lt.assign(13, 0.0);
   auto ms = [](auto a, auto b) { return std::chrono::duration<double, std::milli>(b - a).count(); };

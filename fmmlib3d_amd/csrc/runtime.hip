@@ -36,6 +36,18 @@ hipStream_t near_stream(Context& ctx) {
   return aux_stream(ctx);
 }
 
+void QueuedWork::wait() {
+  FMM_HIP(hipStreamSynchronize(ctx_.stream));
+  done_ = true;
+}
+
+QueuedWork::~QueuedWork() {
+  if (done_) return;
+  // (an error here is the error the call already reports)
+  if (hipStreamSynchronize(ctx_.stream) != hipSuccess) (void)hipGetLastError();
+  if (ctx_.aux && hipStreamSynchronize(ctx_.aux) != hipSuccess) (void)hipGetLastError();
+}
+
 void Arena::use_fixed(void* base, size_t cap) {
   release_all();
   fbase_ = (char*)base;

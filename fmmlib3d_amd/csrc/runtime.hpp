@@ -112,6 +112,26 @@ void staged_download(Context& ctx, void* host, const void* dev, size_t bytes);
 // `ctx.stream` when the context keeps it there or FMM3D_NEAR_STREAM=0
 hipStream_t near_stream(Context& ctx);
 
+// The work a call queues on a context's streams.  A call that leaves early (a
+// buffer that cannot be had, a refused order, a HIP error) still has copies in
+// flight from the context's pinned buffers and kernels that write its cached
+// tables, and the next call may come on another stream: unless wait() has been
+// reached, the destructor waits for both streams.
+class QueuedWork {
+ public:
+  explicit QueuedWork(Context& ctx) : ctx_(ctx) {}
+  ~QueuedWork();
+  QueuedWork(const QueuedWork&) = delete;
+  QueuedWork& operator=(const QueuedWork&) = delete;
+  // the end of a call: ctx.stream has finished (the second stream is joined to
+  // it by events before)
+  void wait();
+
+ private:
+  Context& ctx_;
+  bool done_ = false;
+};
+
 Context& default_context();
 
 // last per-stage timings of this thread

@@ -203,6 +203,7 @@ struct Server {
   }
 
   static int solve(Context& ctx, Request& r) {
+    QueuedWork queued(ctx);
     auto up = [&](const char* name, const std::vector<double>& h) -> double* {
       if (h.empty()) return nullptr;
       double* d = (double*)ctx.arena.get(name, h.size() * sizeof(double));
@@ -236,7 +237,7 @@ struct Server {
     down(r.fld, c.fld_dev, 6 * (size_t)r.ns);
     down(r.pt, c.pottarg_dev, 2 * (size_t)r.nt);
     down(r.ft, c.fldtarg_dev, 6 * (size_t)r.nt);
-    FMM_HIP(hipStreamSynchronize(ctx.stream));
+    queued.wait();
     return 0;
   }
 
@@ -244,6 +245,7 @@ struct Server {
   // merged; inputs concatenated and uploaded once; one graph-captured solve;
   // outputs split back.  A tree that cannot be built fails the batch (4).
   static int solve_fused(Context& ctx, std::vector<std::shared_ptr<Request>>& batch) {
+    QueuedWork queued(ctx);
     const Request& r0 = *batch[0];
     double eps;
     int nbox;
@@ -312,7 +314,7 @@ struct Server {
     down(c.fld_dev, 6, &Request::fld, &Request::ns);
     down(c.pottarg_dev, 2, &Request::pt, &Request::nt);
     down(c.fldtarg_dev, 6, &Request::ft, &Request::nt);
-    FMM_HIP(hipStreamSynchronize(ctx.stream));
+    queued.wait();
     return 0;
   }
 };
