@@ -608,10 +608,8 @@ int lap_solve(Context& ctx, const LapCall& c) {
   mark(7);
   // ---- STEP 7: L2P (packed local + gradient expansions, wave-uniform reads)
   if (P.n_l2p) {
-    const size_t E = (size_t)pack_entries(p);
-    // (one entry more than the packs hold: the walk loads one ahead)
-    T* pack = (T*)ctx.arena.get("l2p_pack", sizeof(T) * kPackEntry * (E * (size_t)P.n_l2p + 1));
-    const size_t tot = E * (size_t)P.n_l2p;
+    T* pack = (T*)ctx.arena.get("l2p_pack", sizeof(T) * pack_values(p, P.n_l2p));
+    const size_t tot = (size_t)pack_entries(p) * P.n_l2p;
     hipLaunchKernelGGL((k_l2p_pack<T>), dim3((unsigned)std::min<size_t>(blocks(tot, 256), 65536)), dim3(256), 0, s,
                        P, fac, lo, pack);
     if (P.n_l2pi)
@@ -670,7 +668,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
       const size_t o_pk = nbx, o_off = o_pk + pk.size(), o_it = o_off + off.size(), o_red = o_it + it.size();
       for (auto* v : {&slot, &pk, &off, &it, &red}) hv.insert(hv.end(), v->begin(), v->end());
       const int* dh = upload_ints("m2p_i", hv, s);
-      T* pack = (T*)ctx.arena.get("m2p_pack", sizeof(T) * kPackEntry * ((size_t)tot + 1));
+      T* pack = (T*)ctx.arena.get("m2p_pack", sizeof(T) * pack_values(pd, pk.size()));
       const size_t nit = it.size() / 5;
       double* partial = (double*)ctx.arena.get("m2p_part", sizeof(double) * 8 * 64 * nit);
       const size_t tp = (size_t)pk.size() * Hd;

@@ -361,26 +361,27 @@ __global__ __launch_bounds__(256) void k_form2(DevPlan P, const double* __restri
 // the pack holds, for each X of E, Gz, Gu, Gd and c+- = X(n, +-a) (c- = 0 for
 // a = 0), the four reals that take the harmonic h = H_n^a to c+ h + c- conj(h),
 //   re: (c+ + c-)_re h_re - (c+ - c-)_im h_im,  im: (c+ + c-)_im h_re + (c+ - c-)_re h_im,
-// times the scale of FacLayout's recurrence, then that recurrence's factor for
-// degree n + 1: kPackEntry values.  Entries are in the order of the walk
-// (column a, then n = a..pd), columns padded to an even count by zero entries.
-// The walk reads them with scalar loads, one entry ahead, and pays 16 FMAs and
+// times the scale of FacLayout's recurrence: kPackEntry values.  Entries are in
+// the order of the walk (column a, then n = a..pd); that recurrence's factors
+// for degree n + 1 stand once, in the same order, ahead of the packs (with them
+// in the entries and the columns padded to an even count the packs took 17%
+// more at order 26, 50% at order 2, and a fixed workspace held fewer points).
+// The walk reads both with scalar loads, one entry ahead, and pays 16 FMAs and
 // the recurrence's 5 operations per entry and point (32 and 9 before, the
 // harmonics normalised and c+ h, c- conj(h) taken apart).  VALU bound: 400,000
 // clustered points at order 39, M2P 11.4 -> 8.2 ms; 200,000 + 180,000 at order
 // 26 7.8 -> 5.7 ms; 1M + 1M uniform, L2P 1.59 -> 1.22 ms (FP32 1.22 -> 0.74 ms).
 // ---------------------------------------------------------------------------
-constexpr int kPackEntry = 18;
-__host__ __device__ inline int pack_col(int pd, int a) { return (pd + 2 - a) & ~1; }  // entries of column a
-__host__ __device__ inline int pack_entries(int pd) {
-  int e = 0;
-  for (int a = 0; a <= pd; a++) e += pack_col(pd, a);
-  return e;
-}
+constexpr int kPackEntry = 16;
+__host__ __device__ inline int pack_entries(int pd) { return (pd + 1) * (pd + 2) / 2; }
+// values ahead of the packs: the factors and one read ahead of the last
+__host__ __device__ inline int pack_head(int pd) { return (pack_entries(pd) + 1 + 15) / 16 * 16; }
+// values of n packs, with the entry that the walk reads past the last
+inline size_t pack_values(int pd, size_t n) { return pack_head(pd) + kPackEntry * ((size_t)pack_entries(pd) * n + 1); }
 
 // coefficients c+- of E, Gz, Gu, Gd at (n, a), as (re, im) pairs, to an entry
 template <typename T>
-__device__ __forceinline__ void pack_store(T* __restrict__ o, const T (&v)[16], T g, T beta) {
+__device__ __forceinline__ void pack_store(T* __restrict__ o, const T (&v)[16], T g) {
 #pragma unroll
   for (int x = 0; x < 4; x++) {
     o[4 * x] = g * (v[4 * x] + v[4 * x + 2]);
@@ -388,8 +389,6 @@ __device__ __forceinline__ void pack_store(T* __restrict__ o, const T (&v)[16], 
     o[4 * x + 2] = g * (v[4 * x + 1] + v[4 * x + 3]);
     o[4 * x + 3] = g * (v[4 * x] - v[4 * x + 2]);
   }
-  o[16] = beta;
-  o[17] = T(0);
 }
 
 template <typename T>
@@ -401,18 +400,18 @@ __global__ void k_l2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
   const size_t total = (size_t)P.n_l2p * NE;
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
     const int i = (int)(t / NE);
-    int a = 0, r = (int)(t - (size_t)i * NE);
-    while (r >= pack_col(p, a)) { r -= pack_col(p, a); a++; }
+    const int w = (int)(t - (size_t)i * NE);
+    int a = 0, r = w;
+    while (r >= p + 1 - a) { r -= p + 1 - a; a++; }
     const int n = a + r;
+    if (i == 0) pack[w] = (T)fac[L.BT + hidx(n + 1, a)];
     const T* E = lo + 2 * (size_t)P.l2p_boxes[i] * K;
     T v[16];
 #pragma unroll
     for (int e = 0; e < 16; e++) v[e] = T(0);
-    if (n <= p) {
-      v[0] = E[2 * eidx(n, a)];
-      v[1] = E[2 * eidx(n, a) + 1];
-      if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
-    }
+    v[0] = E[2 * eidx(n, a)];
+    v[1] = E[2 * eidx(n, a) + 1];
+    if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
     if (n + 1 <= p) {
       const int n1 = n + 1;
       for (int sgn = 0; sgn < (a > 0 ? 2 : 1); sgn++) {
@@ -426,27 +425,28 @@ __global__ void k_l2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
         v[13 + 2 * sgn] = fd * E[2 * eidx(n1, m + 1) + 1];
       }
     }
-    pack_store(pack + kPackEntry * t, v, n <= p ? (T)fac[L.GN + hidx(n, a)] : T(0), n <= p ? (T)fac[L.BT + hidx(n + 1, a)] : T(0));
+    pack_store(pack + pack_head(p) + kPackEntry * t, v, (T)fac[L.GN + hidx(n, a)]);
   }
 }
 
-// One pack entry in scalar registers
+// One pack entry and its factor in scalar registers
 template <typename T, bool GRAD>
 struct PackRec {
   T c[GRAD ? 16 : 4], b;
-  __device__ __forceinline__ void load(const T* __restrict__ o) {
+  __device__ __forceinline__ void load(const T* __restrict__ o, const T* __restrict__ beta) {
 #pragma unroll
     for (int e = 0; e < (GRAD ? 16 : 4); e++) c[e] = o[e];
-    b = o[16];
+    b = *beta;
   }
 };
 
 // The walk over one pack at a point: w, zz, rho of the recurrence, h00 its
-// first value; out (pot, d/dz, U, D) is added to.  Reads one entry past the
+// first value, beta its factors; out (pot, d/dz, U, D) is added to.  Two entries
+// at a time, a column of odd length ending on one.  Reads one entry past the
 // pack's last.
 template <typename T, bool GRAD>
-__device__ __forceinline__ void pack_walk(const T* __restrict__ pk, int pd, C2<T> w, T zz, T rho, T h00,
-                                          C2<T> (&out)[4]) {
+__device__ __forceinline__ void pack_walk(const T* __restrict__ pk, const T* __restrict__ beta, int pd, C2<T> w, T zz,
+                                          T rho, T h00, C2<T> (&out)[4]) {
   PackRec<T, GRAD> ra, rb;
   auto arrived = [] {
     __builtin_amdgcn_sched_barrier(0);
@@ -468,21 +468,32 @@ __device__ __forceinline__ void pack_walk(const T* __restrict__ pk, int pd, C2<T
     hp = h;
     h = hn;
   };
-  ra.load(pk);
+  ra.load(pk, beta);
   int e = 0;
   for (int a = 0; a <= pd; a++) {
     if (a > 0) hmm = cmul(w, hmm);
     h = hmm;
     hp = {T(0), T(0)};
-    for (const int end = e + pack_col(pd, a); e < end; e += 2) {
+    const int end = e + pd + 1 - a;
+    for (; e + 1 < end; e += 2) {
       const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane(e);
       const T* __restrict__ o = pk + (size_t)kPackEntry * u;
+      const T* __restrict__ bt = beta + u;
       arrived();
-      rb.load(o + kPackEntry);
+      rb.load(o + kPackEntry, bt + 1);
       step(ra);
       arrived();
-      ra.load(o + 2 * kPackEntry);
+      ra.load(o + 2 * kPackEntry, bt + 2);
       step(rb);
+    }
+    if (e < end) {
+      const unsigned u = (unsigned)__builtin_amdgcn_readfirstlane(e);
+      arrived();
+      rb.load(pk + (size_t)kPackEntry * (u + 1), beta + u + 1);
+      step(ra);
+      arrived();
+      ra = rb;
+      e++;
     }
   }
 }
@@ -502,7 +513,7 @@ __global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const T* __restrict__ p
   const int ib = P.l2p_items[3 * w], kind = P.l2p_items[3 * w + 1], start = P.l2p_items[3 * w + 2];
   if (ib < 0) return;   // padding item
   const int b = P.l2p_boxes[ib];
-  const T* pk = pack + (size_t)ib * pack_entries(p) * kPackEntry;
+  const T* pk = pack + pack_head(p) + (size_t)ib * pack_entries(p) * kPackEntry;
   const T ih = (T)P.inv_side[P.level[b]];
   const double cx = P.center[3 * b], cy = P.center[3 * b + 1], cz = P.center[3 * b + 2];
   const int wp = kind ? wpot1 : wpot0, wf = kind ? wfld1 : wfld0;
@@ -519,9 +530,9 @@ __global__ __launch_bounds__(256) void k_l2p2(DevPlan P, const T* __restrict__ p
   const T r2 = ux * ux + uy * uy + uz * uz;
   C2<T> out[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
   if (wf)
-    pack_walk<T, true>(pk, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
+    pack_walk<T, true>(pk, pack, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
   else
-    pack_walk<T, false>(pk, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
+    pack_walk<T, false>(pk, pack, p, C2<T>{-ux, -uy}, uz, r2, T(1), out);
   if (!active) return;
   const C2<T> pv = out[0], gz = out[1], gu = out[2], gd = out[3];
   const size_t id = (size_t)(n0 + i);
@@ -550,8 +561,9 @@ __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
   for (size_t t = blockIdx.x * (size_t)blockDim.x + threadIdx.x; t < total; t += (size_t)gridDim.x * blockDim.x) {
     const int i = (int)(t / NE), w = (int)(t - (size_t)i * NE);
     int a = 0, r = w;
-    while (r >= pack_col(pd, a)) { r -= pack_col(pd, a); a++; }
+    while (r >= pd + 1 - a) { r -= pd + 1 - a; a++; }
     const int n = a + r;
+    if (i == 0) pack[w] = (T)fac[L.BT + hidx(n + 1, a)];
     const T* E = mp + 2 * (size_t)boxes[i] * K;
     auto ef = [&](int off, int n1, int m1, int e) -> T {  // factor * E(n1, m1), zero outside
       if (n1 < 0 || m1 > n1 || m1 < -n1) return T(0);
@@ -565,7 +577,7 @@ __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
       v[1] = E[2 * eidx(n, a) + 1];
       if (a > 0) { v[2] = E[2 * eidx(n, -a)]; v[3] = E[2 * eidx(n, -a) + 1]; }
     }
-    if (grad && n >= 1 && n <= pd) {
+    if (grad && n >= 1) {
       const int n1 = n - 1;
       for (int sgn = 0; sgn < (a > 0 ? 2 : 1); sgn++) {
         const int m = sgn ? -a : a;
@@ -576,8 +588,7 @@ __global__ void k_m2p_pack(DevPlan P, const double* __restrict__ fac, const T* _
         }
       }
     }
-    pack_store(pack + kPackEntry * ((size_t)offs[i] + w), v, n <= pd ? (T)fac[L.GN + hidx(n, a)] : T(0),
-               n <= pd ? (T)fac[L.BT + hidx(n + 1, a)] : T(0));
+    pack_store(pack + pack_head(pd) + kPackEntry * ((size_t)offs[i] + w), v, (T)fac[L.GN + hidx(n, a)]);
   }
 }
 
@@ -619,11 +630,11 @@ __global__ __launch_bounds__(256) void k_m2p_eval(DevPlan P, const T* __restrict
     const T r2 = ux * ux + uy * uy + uz * uz;
     const T ir2 = T(1) / r2, ir = sqrt(ir2);
     C2<T> out[4] = {{0, 0}, {0, 0}, {0, 0}, {0, 0}};
-    const T* c = pack + kPackEntry * (size_t)slot[j];
+    const T* c = pack + pack_head(pd) + kPackEntry * (size_t)slot[j];
     if (grad)
-      pack_walk<T, true>(c, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
+      pack_walk<T, true>(c, pack, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
     else
-      pack_walk<T, false>(c, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
+      pack_walk<T, false>(c, pack, pd, C2<T>{-ux * ir2, -uy * ir2}, uz * ir2, ir2, ir, out);
     // pot = sum M S(u)/h ; the gradient w.r.t. x adds another 1/h
     const T sg = ih * ih;
 #pragma unroll
