@@ -53,6 +53,21 @@ struct LapTabSet {
   long mf_rot_back = 0, mf_z_size = 0;
 };
 
+// FMM3D_M2L_ROTATION, read once: 0 the default (pairs grouped by translation
+// class, k_m2l_grp), 1 "pairs" (one pair at a time with per-class rotation
+// blocks), 2 "factored" (factored rotations), 3 "mfma" (the grouped kernel on
+// the matrix cores).
+int m2l_form() {
+  static const int form = [] {
+    const char* v = std::getenv("FMM3D_M2L_ROTATION");
+    if (v && std::strcmp(v, "factored") == 0) return 2;
+    if (v && std::strcmp(v, "pairs") == 0) return 1;
+    if (v && std::strcmp(v, "mfma") == 0) return 3;
+    return 0;
+  }();
+  return form;
+}
+
 // The host tables of order p, built once per process (tens to a hundred ms
 // at p = 26..39) and shared by every context.
 std::shared_ptr<const LapTabSet> lap_host_tables(int p, double eps) {
@@ -63,6 +78,8 @@ std::shared_ptr<const LapTabSet> lap_host_tables(int p, double eps) {
   if (it != cache.end()) return it->second;
   HostTables H;
   build_tables(p, eps, H);
+  // half of all tables (26 of 50 MB at order 26): only where they are read
+  if (m2l_form() == 3) build_mfma_tables(p, H);
   auto T = std::make_shared<LapTabSet>();
   // ints: off_rot | off_dist | off_ptrunc | oct_rot ; doubles:
   // fac | off_phase | oct_phase | rot | z_m2l | z_m2m | z_l2l | delta | rot_e |
@@ -551,17 +568,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   mark(5);
   // ---- STEP 4: M2L
   if (P.n_m2l) {
-    // Default: pairs grouped by translation class (k_m2l_grp).
-    // FMM3D_M2L_ROTATION=pairs selects one pair at a time with per-class
-    // rotation blocks, =factored the factored rotations, =mfma the grouped
-    // kernel on the matrix cores.
-    static const int m2l_form = [] {
-      const char* v = std::getenv("FMM3D_M2L_ROTATION");
-      if (v && std::strcmp(v, "factored") == 0) return 2;
-      if (v && std::strcmp(v, "pairs") == 0) return 1;
-      if (v && std::strcmp(v, "mfma") == 0) return 3;
-      return 0;
-    }();
+    const int form_m2l = m2l_form();
     // FMM3D_M2L_ROTATION=mfma: the grouped M2L on the matrix cores
     // (k_m2l_mfma) wherever its LDS fits and p <= 47 (three row tiles);
     // FMM3D_M2L_MFMA_THREADS=512 runs eight waves per workgroup.
@@ -570,7 +577,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
       return (v && std::strcmp(v, "512") == 0) ? 512 : 256;
     }();
     const size_t mf_lds = m2l_mfma_lds<T>(p);
-    if (m2l_form == 3 && p <= 47 && mf_lds <= max_lds_bytes(ctx)) {
+    if (form_m2l == 3 && p <= 47 && mf_lds <= max_lds_bytes(ctx)) {
       const int mrt = p / 16 + 1;
 #define M2L_MFMA(NT_, R_) \
   hipLaunchKernelGGL((k_m2l_mfma<T, NT_, R_>), dim3(P.n_m2l), dim3(NT_), mf_lds, s, P, Tb, mp, lo)
@@ -584,7 +591,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
       const bool lds = sizeof(T) * 6 * (size_t)K <= max_lds_bytes(ctx);
       const size_t sh = lds ? sizeof(T) * 6 * K : lds_ps;
       const GrpShape G = grp_shape<T>(p, max_lds_bytes(ctx));
-      if ((m2l_form == 0 || m2l_form == 3) && G.threads > 0) {
+      if ((form_m2l == 0 || form_m2l == 3) && G.threads > 0) {
         const size_t need = grp_lds_bytes<T>(p, G.room, G.teams);
 #define M2L_GRP(NT_, I_) \
   hipLaunchKernelGGL((k_m2l_grp<T, NT_, I_>), dim3(P.n_m2l), dim3(NT_), need, s, P, Tb, G.room, G.lts, mp, lo)
@@ -592,7 +599,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
         else if (G.items == 1) M2L_GRP(512, 1);
         else M2L_GRP(512, 2);
 #undef M2L_GRP
-      } else if (m2l_form != 2) {
+      } else if (form_m2l != 2) {
         if (lds) hipLaunchKernelGGL((k_m2l<T, true>), dim3(P.n_m2l), dim3(256), sh, s, P, Tb, mp, lo);
         else hipLaunchKernelGGL((k_m2l<T, false>), dim3(P.n_m2l), dim3(256), sh, s, P, Tb, mp, lo);
       } else {

@@ -117,7 +117,7 @@ struct SqrtBinom {
 // applies the same rows to the reversed input).  Back: the transpose,
 // out_m = sum_{m'} F[m'][m] in_{m'}, which has the same symmetry.
 // z-shift of order m: out_l = sum_n Z[m][l][n] in_n for l, n = m..p.
-static void build_mfma_tables(int p, HostTables& H) {
+void build_mfma_tables(int p, HostTables& H) {
   const int P1 = p + 1;
   H.mf_rot_off.assign((size_t)H.nrot * P1, 0);
   long tot = 0;
@@ -211,7 +211,6 @@ void build_tables(int p, double eps, HostTables& H) {
               H.z_m2l[Z * dc + ((size_t)m * P1 + l) * P1 + n];
         }
     }
-  build_mfma_tables(p, H);
   H.z_m2m.assign(Z, 0.0);
   H.z_l2l.assign(Z, 0.0);
   const double r = std::sqrt(3.0) / 4.0;

@@ -50,6 +50,8 @@ int laplace_nterms(double eps);
 // l3dterms_list2 (src/l3dterms.f:136): 7^3 table indexed by offset code
 std::vector<int> laplace_itable(double eps);
 void build_tables(int p, double eps, HostTables& H);
+// adds the tables of the M2L on the matrix cores (mf_*) to those of build_tables
+void build_mfma_tables(int p, HostTables& H);
 // the factor table alone (FacLayout(p): degrees up to p+1), as built for order p
 void build_fac_table(int p, std::vector<double>& fac);
 // the kernel-independent part (factors, rotation classes and blocks, phases,

@@ -212,6 +212,8 @@ int main() {
     const int p = laplace_nterms(e);
     HostTables H;
     build_tables(p, e, H);
+    CHECK(H.mf_rot.empty() && H.mf_z.empty());
+    build_mfma_tables(p, H);
     CHECK(!H.mf_rot.empty() && !H.mf_z.empty());
     CHECK((long)H.mf_rot.size() == 2 * H.mf_rot_back);
     CHECK((long)H.mf_z.size() == H.mf_z_size * H.ndist);

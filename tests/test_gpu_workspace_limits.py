@@ -1,6 +1,6 @@
 """Calls near the size that the fixed workspace of
-fmm3d_lfmm3dparttarg_dev_noalloc holds: what it took it keeps taking (the
-largest multiple of 500 points that fitted before the packed expansions, the
+fmm3d_lfmm3dparttarg_dev_noalloc holds: what it took it keeps taking (sizes
+within 2,000 points of the limit from before the packed expansions, the
 strengths and the tables grew), with the results of fmm3d_lfmm3dparttarg_dev
 bit for bit."""
 import numpy as np
@@ -13,7 +13,8 @@ from hip_arrays import DeviceArrays
 pytestmark = pytest.mark.gpu
 
 # (precision mode, iprec, distribution, sources = targets)
-LIMITS = [(0, 2, "clusters", 65500), (0, 0, "cube", 270000), (0, 2, "plummer", 87000)]
+LIMITS = [(0, 2, "clusters", 65500), (0, 0, "cube", 270000), (0, 2, "plummer", 87000), (0, 1, "clusters", 106500),
+          (0, 3, "cube", 80000), (0, -2, "cube", 458000)]
 
 
 @pytest.mark.parametrize("prec,iprec,dist,n", LIMITS)
