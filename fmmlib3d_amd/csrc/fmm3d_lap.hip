@@ -317,7 +317,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   constexpr bool near32 = sizeof(TN) < sizeof(double);
   double* spos = (double*)ctx.arena.get("spos", sizeof(double) * 4 * (size_t)ns);
   double* str64 = (double*)ctx.arena.get("str64", sizeof(double) * 8 * (size_t)ns);
-  float* str32 = near32 || sizeof(T) == 4 ? (float*)ctx.arena.get("str32", sizeof(float) * 8 * (size_t)ns) : nullptr;
+  float* str32 = near32 ? (float*)ctx.arena.get("str32", sizeof(float) * 8 * (size_t)ns) : nullptr;
   double* tpos = (double*)ctx.arena.get("tpos", sizeof(double) * 4 * (size_t)std::max(nt, 1));
   T* mp = (T*)ctx.arena.get("mp", sizeof(T) * 2 * K * nb, 16);
   T* lo = (T*)ctx.arena.get("lo", sizeof(T) * 2 * K * nb, 16);
@@ -329,6 +329,11 @@ int lap_solve(Context& ctx, const LapCall& c) {
   double* fld_sn = (double*)ctx.arena.get("fld_sn", sizeof(double) * 6 * (size_t)ns);
   double* pot_tn = (double*)ctx.arena.get("pot_tn", sizeof(double) * 2 * (size_t)std::max(nt, 1));
   double* fld_tn = (double*)ctx.arena.get("fld_tn", sizeof(double) * 6 * (size_t)std::max(nt, 1));
+  // an FP32 far field beside an FP64 near field: P2M and P2L alone read the FP32
+  // strengths (32 bytes a source), before anything is added to the far fields
+  // (48): they stand there, and the fields are cleared after P2L
+  constexpr bool str32_in_fld = sizeof(T) == 4 && !near32;
+  if (str32_in_fld) str32 = (float*)(void*)fld_s;
   const TN* strn = near32 ? (const TN*)(const void*)str32 : (const TN*)(const void*)str64;
   const int* sperm = dsperm ? dsperm : dI + O.sperm;
   const int* tperm = dsperm ? dtperm : dI + O.tperm;
@@ -381,7 +386,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   zero(mp, 2 * (size_t)K * nb);
   zero(lo, 2 * (size_t)K * nb);
   zero(pot_s, 2 * (size_t)ns);
-  zero(fld_s, 6 * (size_t)ns);
+  if (!str32_in_fld) zero(fld_s, 6 * (size_t)ns);
   zero(pot_sn, 2 * (size_t)ns);
   zero(fld_sn, 6 * (size_t)ns);
   if (nt > 0) {
@@ -565,6 +570,7 @@ int lap_solve(Context& ctx, const LapCall& c) {
   auto t_lists3 = std::chrono::steady_clock::now();
   form(std::true_type{}, P.n_p2l, lo);
   qp_form(std::true_type{}, P.n_p2l, lo);
+  if (str32_in_fld) zero(fld_s, 6 * (size_t)ns);
   mark(5);
   // ---- STEP 4: M2L
   if (P.n_m2l) {

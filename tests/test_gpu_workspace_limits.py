@@ -14,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 # (precision mode, iprec, distribution, sources = targets)
 LIMITS = [(0, 2, "clusters", 65500), (0, 0, "cube", 270000), (0, 2, "plummer", 87000), (0, 1, "clusters", 106500),
-          (0, 3, "cube", 80000), (0, -2, "cube", 458000)]
+          (0, 3, "cube", 80000), (0, -2, "cube", 458000), (2, 1, "cube", 486000), (2, -2, "cube", 498000),
+          (2, 1, "clusters", 161500)]
 
 
 @pytest.mark.parametrize("prec,iprec,dist,n", LIMITS)
