@@ -811,9 +811,11 @@ int lap_direct(Context& ctx, const LapCall& c) {
     hipLaunchKernelGGL(k_gather_sources, dim3(blocks(ns, 256)), dim3(256), 0, s, ns, dperm, c.src_dev,
                        c.q_dev, c.ds_dev, c.dv_dev, c.ifcharge ? 1 : 0, c.ifdipole ? 1 : 0, spos, str64,
                        (float*)nullptr);
-  // the slices' sums (a caller's fixed scratch is not asked for more: one slice)
-  const size_t nsum = std::max((size_t)ns * direct_slices(std::max(ns, 1), ns), (size_t)nt * direct_slices(std::max(nt, 1), ns));
-  double* partial = ctx.arena.fixed() ? nullptr : (double*)ctx.arena.get("direct_part", sizeof(double) * 8 * std::max<size_t>(nsum, 1));
+  // the slices' sums: at most about 16 MB, and none where the points alone fill
+  // the chip
+  const size_t npart = std::max(c.ifpot || c.iffld ? direct_partial(ns, ns) : 0,
+                                c.ifpottarg || c.iffldtarg ? direct_partial(nt, ns) : 0);
+  double* partial = npart ? (double*)ctx.arena.get("direct_part", sizeof(double) * npart) : nullptr;
   auto run = [&](int npts, const double* pts, int are_src) {
     if (npts <= 0) return;
     if (ns == 0 || (!c.ifcharge && !c.ifdipole)) {
@@ -821,7 +823,7 @@ int lap_direct(Context& ctx, const LapCall& c) {
       hipLaunchKernelGGL((k_fill_zero<double>), dim3(blocks(6 * (size_t)npts, 256)), dim3(256), 0, s, 6 * (size_t)npts, fld);
       return;
     }
-    const int nsl = ctx.arena.fixed() ? 1 : direct_slices(npts, ns);
+    const int nsl = direct_slices(npts, ns);
 #define DCASE(C, D)                                                                                   \
   if ((c.ifcharge ? 1 : 0) == C && (c.ifdipole ? 1 : 0) == D)                                         \
     hipLaunchKernelGGL((k_direct<C, D>), dim3(blocks(npts, 64), nsl), dim3(64 * kDirectWaves), 0, s, ns, \

@@ -231,6 +231,11 @@ static inline int direct_slices(int npts, int ns) {
   const int most = ns / (64 * kDirectWaves);
   return want < most ? want : most > 1 ? most : 1;
 }
+// doubles of the slices' sums of npts points (one slice goes to the results)
+static inline size_t direct_partial(int npts, int ns) {
+  const int nsl = npts > 0 && ns > 0 ? direct_slices(npts, ns) : 1;
+  return nsl > 1 ? 8 * (size_t)npts * nsl : 0;
+}
 // first source of part q of this workgroup's slice
 __device__ __forceinline__ int direct_cut(int ns, int q) {
   return (int)((long)ns * (blockIdx.y * kDirectWaves + q) / (gridDim.y * kDirectWaves));
