@@ -460,7 +460,11 @@ int helm_solve(Context& ctx, const LapCall& c) {
     if (G.threads > 0) {
       const size_t need = grp_lds_bytes<double>(pmax, G.room, G.teams);
 #define HM2L_GRP(NT_, I_) \
-  hipLaunchKernelGGL((k_hm2l_grp<NT_, I_>), dim3(P.n_m2l), dim3(NT_), need, s, P, Tb, Hd, G.room, G.lts, mp, lo)
+  launch_pieces(P.n_m2l, NT_, [&](long first, unsigned count) {                                                     \
+    DevPlan Q = P;                                                                                                  \
+    Q.m2l_boxes += first;                                                                                           \
+    hipLaunchKernelGGL((k_hm2l_grp<NT_, I_>), dim3(count), dim3(NT_), need, s, Q, Tb, Hd, G.room, G.lts, mp, lo);   \
+  })
       if (G.threads == 256) HM2L_GRP(256, 1);
       else if (G.items == 1) HM2L_GRP(512, 1);
       else HM2L_GRP(512, 2);
@@ -646,8 +650,10 @@ int helm_direct(Context& ctx, const LapCall& c) {
     const int nsl = direct_slices(npts, ns);
 #define HDCASE(C, D)                                                                                       \
   if ((c.ifcharge ? 1 : 0) == C && (c.ifdipole ? 1 : 0) == D)                                              \
-    hipLaunchKernelGGL((k_hdirect<C, D>), dim3(blocks(npts, 64), nsl), dim3(64 * kDirectWaves), 0, s, c.zk_re, c.zk_im, ns, \
-                       spos, str64, npts, pts, are_src, partial, pot, fld);
+    launch_pieces(blocks(npts, 64), 64 * kDirectWaves, [&](long first, unsigned count) {                   \
+      hipLaunchKernelGGL((k_hdirect<C, D>), dim3(count, nsl), dim3(64 * kDirectWaves), 0, s, c.zk_re,      \
+                         c.zk_im, ns, spos, str64, npts, (int)(64 * first), pts, are_src, partial, pot, fld); \
+    });
     HDCASE(1, 0) HDCASE(0, 1) HDCASE(1, 1)
 #undef HDCASE
     if (nsl > 1)

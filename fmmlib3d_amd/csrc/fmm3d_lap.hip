@@ -186,14 +186,15 @@ template <typename TN>
 void launch_p2p(const DevPlan& P, const int* items, int n, const double* spos, const TN* str, const double* str64,
                 const double* tpos, int ifcharge, int ifdipole, bool fld, double* pot0, double* fld0, double* pot1,
                 double* fld1, hipStream_t s) {
-  if (n == 0) return;
-  DevPlan Q = P;
-  Q.p2p_items = items;
-  Q.n_p2p = n;
 #define P2P_CASE(C, Dp, F)                                                                                        \
   if (ifcharge == C && ifdipole == Dp && fld == F) {                                                              \
-    hipLaunchKernelGGL((k_p2p<TN, C, Dp, F>), dim3((unsigned)n), dim3(64 * kP2PSplit), 0, s, Q, spos, str, str64, \
-                       tpos, pot0, fld0, pot1, fld1);                                                             \
+    launch_pieces(n, 64 * kP2PSplit, [&](long first, unsigned count) {                                            \
+      DevPlan Q = P;                                                                                              \
+      Q.p2p_items = items + 3 * first;                                                                            \
+      Q.n_p2p = (int)count;                                                                                       \
+      hipLaunchKernelGGL((k_p2p<TN, C, Dp, F>), dim3(count), dim3(64 * kP2PSplit), 0, s, Q, spos, str, str64,     \
+                         tpos, pot0, fld0, pot1, fld1);                                                           \
+    });                                                                                                           \
     return;                                                                                                       \
   }
   P2P_CASE(1, 0, false) P2P_CASE(1, 0, true) P2P_CASE(0, 1, false) P2P_CASE(0, 1, true)
@@ -600,7 +601,11 @@ int lap_solve(Context& ctx, const LapCall& c) {
       if ((form_m2l == 0 || form_m2l == 3) && G.threads > 0) {
         const size_t need = grp_lds_bytes<T>(p, G.room, G.teams);
 #define M2L_GRP(NT_, I_) \
-  hipLaunchKernelGGL((k_m2l_grp<T, NT_, I_>), dim3(P.n_m2l), dim3(NT_), need, s, P, Tb, G.room, G.lts, mp, lo)
+  launch_pieces(P.n_m2l, NT_, [&](long first, unsigned count) {                                                     \
+    DevPlan Q = P;                                                                                                  \
+    Q.m2l_boxes += first;                                                                                           \
+    hipLaunchKernelGGL((k_m2l_grp<T, NT_, I_>), dim3(count), dim3(NT_), need, s, Q, Tb, G.room, G.lts, mp, lo);     \
+  })
         if (G.threads == 256) M2L_GRP(256, 1);
         else if (G.items == 1) M2L_GRP(512, 1);
         else M2L_GRP(512, 2);
@@ -826,8 +831,10 @@ int lap_direct(Context& ctx, const LapCall& c) {
     const int nsl = direct_slices(npts, ns);
 #define DCASE(C, D)                                                                                   \
   if ((c.ifcharge ? 1 : 0) == C && (c.ifdipole ? 1 : 0) == D)                                         \
-    hipLaunchKernelGGL((k_direct<C, D>), dim3(blocks(npts, 64), nsl), dim3(64 * kDirectWaves), 0, s, ns, \
-                       spos, str64, npts, pts, are_src, partial, pot, fld);
+    launch_pieces(blocks(npts, 64), 64 * kDirectWaves, [&](long first, unsigned count) {              \
+      hipLaunchKernelGGL((k_direct<C, D>), dim3(count, nsl), dim3(64 * kDirectWaves), 0, s, ns, spos, \
+                         str64, npts, (int)(64 * first), pts, are_src, partial, pot, fld);            \
+    });
     DCASE(1, 0) DCASE(0, 1) DCASE(1, 1)
 #undef DCASE
     if (nsl > 1)

@@ -1216,12 +1216,12 @@ __global__ __launch_bounds__(256) void k_hp2p(DevPlan P, double kre, double kim,
 template <bool CHG, bool DIP>
 __global__ __launch_bounds__(64 * kDirectWaves) void k_hdirect(double kre, double kim, int ns,
                                                                const double* __restrict__ spos,
-                                                               const double* __restrict__ str, int npts,
+                                                               const double* __restrict__ str, int npts, int first,
                                                                const double* __restrict__ pts, int pts_are_sources,
                                                                double* __restrict__ partial, double* __restrict__ pot,
                                                                double* __restrict__ fld) {
   const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-  const int i = 64 * blockIdx.x + lane;
+  const int i = first + 64 * (int)blockIdx.x + lane;
   const bool active = i < npts;
   const int me = active ? i : 0;
   const double* mp = (pts_are_sources ? spos : pts) + 4 * (size_t)me;

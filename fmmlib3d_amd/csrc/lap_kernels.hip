@@ -1282,20 +1282,21 @@ __global__ __launch_bounds__(64 * kP2PSplit) __attribute__((amdgpu_waves_per_eu(
 
 // Direct sum over all sources (l3dpartdirect, src/lfmm3dpart.f:1391): the pair
 // arithmetic of the near field in FP64 with every source acting on every point.
-// A workgroup takes 64 points and slice blockIdx.y of the sources, each wave a
-// part of the slice (direct_slices); the waves' sums are added in order, the
-// slices' by k_direct_sum.  24,001 sources acting on themselves and on 10,007
+// A workgroup takes 64 points, from `first` on, and slice blockIdx.y of the
+// sources, each wave a part of the slice (direct_slices); the waves' sums are
+// added in order, the slices' by k_direct_sum.  24,001 sources acting on themselves and on 10,007
 // targets: 13.4 -> 1.46 ms (the FP64 instructions alone take about 1 ms); one
 // wave for 64 points and all sources left two thirds of the SIMDs without a wave,
 // and each waited for its own scalar loads.
 template <bool CHG, bool DIP>
 __global__ __launch_bounds__(64 * kDirectWaves) void k_direct(int ns, const double* __restrict__ spos,
-                                                              const double* __restrict__ str, int npts,
+                                                              const double* __restrict__ str, int npts, int first,
                                                               const double* __restrict__ pts, int pts_are_sources,
                                                               double* __restrict__ partial, double* __restrict__ pot,
                                                               double* __restrict__ fld) {
   const int part = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), lane = (int)(threadIdx.x & 63);
-  const int first = 64 * blockIdx.x, i = first + lane;
+  first += 64 * (int)blockIdx.x;
+  const int i = first + lane;
   const bool active = i < npts;
   const int me = active ? i : 0;
   const double* mp = (pts_are_sources ? spos : pts) + 4 * (size_t)me;
@@ -1305,7 +1306,7 @@ __global__ __launch_bounds__(64 * kDirectWaves) void k_direct(int ns, const doub
   const PairConst<double> pc;
   double t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   if (s0 < s1) {
-    if (pts_are_sources && s0 < first + 64 && s1 > first)  // the points' own sources among them
+    if (pts_are_sources && s0 - first < 64 && s1 > first)  // the points' own sources among them
       p2p_sources<double, CHG, DIP, true, true>(acc, pc, x, y, z, spos, str, str, s0, s1, me, 0.0, t);
     else
       p2p_sources<double, CHG, DIP, true, false>(acc, pc, x, y, z, spos, str, str, s0, s1, -1, 0.0, t);

@@ -271,6 +271,17 @@ inline size_t max_lds_bytes(Context& ctx) {
   return v;
 }
 
+// n workgroups of `threads` each as launches f(first, count): a grid counts
+// its threads in 32 bits, which the near field's and the grouped M2L's larger
+// workgroups reach at 16.8 and 8.4 million (pieces are whole rounds of
+// xcd_block)
+constexpr long launch_piece(unsigned threads) { return 0xffffffffL / threads / 512 * 512; }
+template <typename F>
+inline void launch_pieces(long n, unsigned threads, F&& f) {
+  const long most = launch_piece(threads);
+  for (long i = 0; i < n; i += most) f(i, (unsigned)(n - i < most ? n - i : most));
+}
+
 inline unsigned blocks(size_t n, unsigned b) { return (unsigned)((n + b - 1) / b); }
 
 }  // namespace fmm3d

@@ -127,7 +127,23 @@ static void check_plan(const Octree& t) {
   }
 }
 
+// launches of the larger grids: pieces in order, none above 2^32 - 1 threads
+static void check_launch_pieces() {
+  for (unsigned threads : {64u, 256u, 512u})
+    for (long n : {0L, 1L, 511L, 8388096L, 8388097L, 16776704L, 16776705L, 40000000L, 2147483647L}) {
+      long at = 0;
+      launch_pieces(n, threads, [&](long first, unsigned count) {
+        CHECK(first == at && count > 0);
+        CHECK((unsigned long)count * threads <= 0xfffffffful);
+        at = first + count;
+        CHECK(at == n || count % 512 == 0);
+      });
+      CHECK(at == n);
+    }
+}
+
 int main() {
+  check_launch_pieces();
   const int cases[][3] = {  // ns, nt, dist
       {20000, 5000, 0}, {30000, 0, 1}, {25000, 2000, 2}, {12000, 3000, 3}, {3000, 100, 4}, {1, 0, 0}, {50, 50, 1}};
   const int nboxes[] = {40, 80, 160, 400};
