@@ -119,18 +119,10 @@ HelmCache& helm_upload_tables(Context& ctx, HelmCache& c, HelmHostTables&& plan)
   // [row block of n - am][column block of l - am], 16 real parts then 16
   // imaginary parts of [row][column]; every list-2 order must lie within its
   // table's tiles
-  std::vector<long> zt_off(H.m2l.size() * P1, 0);
-  long nt = 0;
+  std::vector<long> zt_off;
+  const long nt = coax_tile_offsets(H, zt_off);
   int mmax = 0;
-  for (const CoaxJob& J : H.jobs) {
-    mmax = std::max(mmax, std::min(J.pin, J.pout));
-    if (J.m2l < 0) continue;
-    for (int am = 0; am <= J.pout; am++) {
-      zt_off[(size_t)J.m2l * P1 + am] = nt;
-      const long nb4 = (J.pout - am) / 4 + 1;
-      nt += 32 * nb4 * nb4;
-    }
-  }
+  for (const CoaxJob& J : H.jobs) mmax = std::max(mmax, std::min(J.pin, J.pout));
   bool ok = true;
   for (int l = 2; l <= nlev && ok; l++)
     for (int code = 0; code < 343 && ok; code++) {

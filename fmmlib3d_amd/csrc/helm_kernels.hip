@@ -797,11 +797,12 @@ __global__ __launch_bounds__(64) void k_heval3(DevPlan P, HelmDev Hd, const doub
 // ---------------------------------------------------------------------------
 // The coaxial operators from their series (CoaxJob): block (m; l, n) is
 //   sum_s 4 pi i^{l+s-n} sigma^s f_s sqrt((2s+1)/4pi) G(n,s,l;m) pw,
-// s = |n-l|, |n-l|+2, .., n+l, pw the scale powers of the mode.  One workgroup
-// per (operator, m), one thread per entry.  M2L operators are also written as
-// the complex 4x4 tiles of the grouped M2L, tile_off[table * P1 + m] on, the
-// tiles' edges zero.  An order-36 tree's 70 operators take 0.1 ms here; computed
-// on the host and sent they cost 10 to 20 ms for every new root box or wavenumber.
+// s = |n-l|, |n-l|+2, .., n+l, pw the scale powers of the mode (coax_entry).
+// One workgroup per (operator, m), one thread per entry.  M2L operators are also
+// written as the complex 4x4 tiles of the grouped M2L, tile_off[table * P1 + m]
+// on, the tiles' edges zero.  An order-36 tree's 70 operators take 0.1 ms here;
+// computed on the host and sent they cost 10 to 20 ms for every new root box or
+// wavenumber.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_coax(const CoaxJob* __restrict__ jobs, const double* __restrict__ series,
                                               const long* __restrict__ goff, const double* __restrict__ gaunt, int GP1,
@@ -810,33 +811,20 @@ __global__ __launch_bounds__(256) void k_coax(const CoaxJob* __restrict__ jobs, 
   const CoaxJob J = jobs[blockIdx.x];
   const int m = blockIdx.y;
   if (m > J.pin || m > J.pout) return;
-  const int S = J.pin + J.pout;
   const double* f = series + J.series;
-  const double *pb = f + 2 * (S + 1), *pr = pb + S + 1;
-  const long A = J.pout + 1, B = J.pin + 1, M = m;
-  const long mb = J.base + M * A * B - (A + B) * M * (M - 1) / 2 + (M - 1) * M * (2 * M - 1) / 6;  // coax_block
-  const int nrow = (J.pin - m) / 4 + 1, ncol = (J.pout - m) / 4 + 1;  // 4x4 tiles of n - m, l - m
+  const int nrow = 4 * coax_tile_rows(J, m), ncol = 4 * coax_tile_cols(J, m);
   double* tb = J.m2l >= 0 ? tiles + tile_off[(size_t)J.m2l * P1 + m] : nullptr;
-  for (int e = threadIdx.x; e < 16 * nrow * ncol; e += blockDim.x) {
-    const int rr = e / (4 * ncol), cc = e - rr * 4 * ncol, n = m + rr, l = m + cc;
+  for (int e = threadIdx.x; e < nrow * ncol; e += blockDim.x) {
+    const int row = e / ncol, col = e - row * ncol, n = m + row, l = m + col;
     double re = 0.0, im = 0.0;
-    const bool in = n <= J.pin && l <= J.pout;
-    if (in) {
-      const double* g = gaunt + goff[((size_t)m * GP1 + n) * GP1 + l];
-      const int s0 = n > l ? n - l : l - n;
-      for (int s = s0; s <= n + l; s += 2) {
-        const bool neg = ((((l + s - n) / 2) & 1) != 0) != (J.neg && (s & 1));
-        const double c = (neg ? -4.0 : 4.0) * M_PI * sqrt((2.0 * s + 1.0) / (4.0 * M_PI)) * g[(s - s0) / 2];
-        const double pw = J.mode == 1 ? pb[n + l - s] : J.mode == 0 ? pb[s - l + n] * pr[n] : pb[s - n + l] * pr[l];
-        re += c * pw * f[2 * s];
-        im += c * pw * f[2 * s + 1];
-      }
-      const size_t o = 2 * (size_t)(mb + (long)(l - m) * (J.pin + 1 - m) + (n - m));
+    if (n <= J.pin && l <= J.pout) {
+      coax_entry(J, n, l, f, gaunt + goff[((size_t)m * GP1 + n) * GP1 + l], re, im);
+      const long o = 2 * coax_at(J, m, n, l);
       z[o] = re;
       z[o + 1] = im;
     }
     if (tb) {
-      double* t = tb + 32 * ((size_t)(rr / 4) * ncol + cc / 4) + (rr % 4) * 4 + cc % 4;
+      double* t = tb + coax_tile_at(J, m, row, col);
       t[0] = re;
       t[16] = im;
     }

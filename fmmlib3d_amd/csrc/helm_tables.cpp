@@ -360,36 +360,18 @@ bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables
   return true;
 }
 
-bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H) {
-  if (!plan_helm_tables(zk, size, nlev, eps, H)) return false;
-  const auto G = gaunt_for(H.pmax);
-  H.z.assign(2 * (size_t)H.nz, 0.0);
-#pragma omp parallel for schedule(dynamic, 1)
-  for (int t = 0; t < (int)H.jobs.size(); t++) {
-    const CoaxJob& J = H.jobs[t];
-    const int S = J.pin + J.pout;
-    const double* f = &H.series[J.series];
-    const double *pb = f + 2 * (S + 1), *pr = pb + S + 1;
-    for (int m = 0; m <= std::min(J.pin, J.pout); m++) {
-      const long mb = J.base + coax_block(m, J.pin, J.pout);
-      for (int l = m; l <= J.pout; l++)
-        for (int n = m; n <= J.pin; n++) {
-          const long go = G->at(m, n, l);
-          cplx acc = 0.0;
-          for (int s = std::abs(n - l), k = 0; s <= n + l; s += 2, k++) {
-            double sg = (((l + s - n) / 2) & 1) ? -1.0 : 1.0;
-            if (J.neg && (s & 1)) sg = -sg;
-            const double c = 4.0 * M_PI * sg * std::sqrt((2.0 * s + 1.0) / (4.0 * M_PI)) * G->g[go + k];
-            const double pw = J.mode == 1 ? pb[n + l - s] : J.mode == 0 ? pb[s - l + n] * pr[n] : pb[s - n + l] * pr[l];
-            acc += c * pw * cplx(f[2 * s], f[2 * s + 1]);
-          }
-          const size_t e = 2 * (size_t)(mb + (long)(l - m) * (J.pin + 1 - m) + (n - m));
-          H.z[e] = acc.real();
-          H.z[e + 1] = acc.imag();
-        }
+long coax_tile_offsets(const HelmHostTables& H, std::vector<long>& off) {
+  const int P1 = H.pmax + 1;
+  off.assign(H.m2l.size() * P1, 0);
+  long n = 0;
+  for (const CoaxJob& J : H.jobs) {
+    if (J.m2l < 0) continue;
+    for (int am = 0; am <= J.pout; am++) {
+      off[(size_t)J.m2l * P1 + am] = n;
+      n += 32L * coax_tile_rows(J, am) * coax_tile_cols(J, am);
     }
   }
-  return true;
+  return n;
 }
 
 }  // namespace fmm3d

@@ -1,6 +1,7 @@
 // Host-side pieces of the Helmholtz FMM: spherical Bessel / Hankel series,
 // expansion orders (h3dterms), and the per-level translation tables.
 #pragma once
+#include <cmath>
 #include <complex>
 #include <memory>
 #include <vector>
@@ -65,7 +66,6 @@ struct HelmHostTables {
   std::vector<CoaxJob> jobs;         // one per operator
   std::vector<double> series;        // their series
   long nz = 0;                       // complex entries of all coaxial blocks
-  std::vector<double> z;             // the blocks themselves, complex as (re, im): build_helm_tables only
 };
 
 // build_geometry_tables(p), the last few orders kept for the process
@@ -76,15 +76,49 @@ std::shared_ptr<const HostTables> geometry_for(int p);
 // computed from the series on the device (k_coax).  Returns false when an
 // order exceeds what the device kernels support (kMaxHelmOrder).
 bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H);
-// the same with the blocks computed on the host into H.z
-bool build_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H);
+// where the 4x4 tiles of order am of M2L table t start (k_coax), off[t * (pmax + 1)
+// + am]; returns their size in doubles
+long coax_tile_offsets(const HelmHostTables& H, std::vector<long>& off);
 
 constexpr int kMaxHelmOrder = 120;
 
+// What k_coax computes and where, also compiled for the host so that the
+// sanitizers see it.
+#if defined(__HIP__)
+#define FMM_HD __host__ __device__
+#else
+#define FMM_HD
+#endif
+
 // offset (complex entries) of the m-block inside a packed coaxial operator
-inline long coax_block(int m, int pin, int pout) {
+FMM_HD inline long coax_block(int m, int pin, int pout) {
   const long A = pout + 1, B = pin + 1, M = m;
   return M * A * B - (A + B) * M * (M - 1) / 2 + (M - 1) * M * (2 * M - 1) / 6;
+}
+// entry (l, n) of that block, from J.base on
+FMM_HD inline long coax_at(const CoaxJob& J, int m, int n, int l) {
+  return J.base + coax_block(m, J.pin, J.pout) + (long)(l - m) * (J.pin + 1 - m) + (n - m);
+}
+// 4x4 tiles of the m-block: rows n - m, columns l - m
+FMM_HD inline int coax_tile_rows(const CoaxJob& J, int m) { return (J.pin - m) / 4 + 1; }
+FMM_HD inline int coax_tile_cols(const CoaxJob& J, int m) { return (J.pout - m) / 4 + 1; }
+// the real part of (n, l) = (m + row, m + col) in those tiles; the imaginary
+// part is 16 further
+FMM_HD inline long coax_tile_at(const CoaxJob& J, int m, int row, int col) {
+  return 32 * ((long)(row / 4) * coax_tile_cols(J, m) + col / 4) + (row % 4) * 4 + col % 4;
+}
+// the entry: f the operator's series, g the integrals G(n, s, l; m) of s = |n-l|, ..
+FMM_HD inline void coax_entry(const CoaxJob& J, int n, int l, const double* f, const double* g, double& re, double& im) {
+  const int S = J.pin + J.pout, s0 = n > l ? n - l : l - n;
+  const double *pb = f + 2 * (S + 1), *pr = pb + S + 1;
+  re = im = 0.0;
+  for (int s = s0; s <= n + l; s += 2) {
+    const bool neg = ((((l + s - n) / 2) & 1) != 0) != (J.neg && (s & 1));
+    const double c = (neg ? -4.0 : 4.0) * M_PI * sqrt((2.0 * s + 1.0) / (4.0 * M_PI)) * g[(s - s0) / 2];
+    const double pw = J.mode == 1 ? pb[n + l - s] : J.mode == 0 ? pb[s - l + n] * pr[n] : pb[s - n + l] * pr[l];
+    re += c * pw * f[2 * s];
+    im += c * pw * f[2 * s + 1];
+  }
 }
 
 }  // namespace fmm3d

@@ -9,6 +9,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstdint>
+#include <algorithm>
 #include <vector>
 
 #include "helm_tables.hpp"
@@ -142,6 +143,47 @@ static void check_launch_pieces() {
     }
 }
 
+// what k_coax does for the operators of H, in arrays of the sizes that the
+// device has: every entry and every tile value written once
+static void check_coax(const HelmHostTables& H) {
+  const auto G = gaunt_for(H.pmax);
+  const int GP1 = G->P + 1, P1 = H.pmax + 1;
+  std::vector<long> off;
+  const long nt = coax_tile_offsets(H, off);
+  std::vector<double> z(2 * (size_t)H.nz, 0.0), tiles((size_t)nt, 0.0);
+  std::vector<char> zn(H.nz, 0), tn((size_t)nt, 0);
+  for (const CoaxJob& J : H.jobs) {
+    const std::vector<double> f(H.series.begin() + J.series, H.series.begin() + J.series + 3 * (J.pin + J.pout + 1) +
+                                                                 std::max(J.pin, J.pout) + 1);
+    for (int m = 0; m <= std::min(J.pin, J.pout); m++)
+      for (int row = 0; row < 4 * coax_tile_rows(J, m); row++)
+        for (int col = 0; col < 4 * coax_tile_cols(J, m); col++) {
+          const int n = m + row, l = m + col;
+          double re = 0.0, im = 0.0;
+          if (n <= J.pin && l <= J.pout) {
+            const long go = G->off.at(((size_t)m * GP1 + n) * GP1 + l);
+            CHECK(go >= 0 && go + std::min(n, l) < (long)G->g.size());
+            coax_entry(J, n, l, f.data(), &G->g[go], re, im);
+            CHECK(std::isfinite(re) && std::isfinite(im));
+            const long o = coax_at(J, m, n, l);
+            CHECK(o >= 0 && o < H.nz);
+            zn.at(o)++;
+            z.at(2 * o) = re;
+            z.at(2 * o + 1) = im;
+          }
+          if (J.m2l >= 0) {
+            const long t = off.at((size_t)J.m2l * P1 + m) + coax_tile_at(J, m, row, col);
+            tn.at(t)++;
+            tn.at(t + 16)++;
+            tiles.at(t) = re;
+            tiles.at(t + 16) = im;
+          }
+        }
+  }
+  for (char c : zn) CHECK(c == 1);
+  for (char c : tn) CHECK(c == 1);
+}
+
 int main() {
   check_launch_pieces();
   const int cases[][3] = {  // ns, nt, dist
@@ -239,11 +281,12 @@ int main() {
   for (auto& z : zks)
     for (double e : {.5e-3, .5e-6, .5e-9}) {
       HelmHostTables H;
-      const bool ok = build_helm_tables(cplx(z[0], z[1]), 1.0, 5, e, H);
+      const bool ok = plan_helm_tables(cplx(z[0], z[1]), 1.0, 5, e, H);
       if (!ok) continue;  // an order beyond kMaxHelmOrder: reported, not built
       CHECK((int)H.plev.size() == 6);
       for (int l = 2; l <= 5; l++) CHECK(H.plev[l] > 0 && H.plev[l] <= H.pmax);
-      for (auto& d : H.m2l) CHECK(d.base >= 0 && 2 * (size_t)d.base <= H.z.size());
+      for (auto& d : H.m2l) CHECK(d.base >= 0 && d.base <= H.nz);
+      check_coax(H);
     }
   std::printf("host_check: %d failed checks\n", fails);
   return fails ? 1 : 0;
