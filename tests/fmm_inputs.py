@@ -128,3 +128,23 @@ def icosphere(level, radius=1.0):
     V = np.array(verts) * radius
     return V[np.array(f)]
 
+
+
+# leaf size of the octree by iprec (src/lfmm3dpart.f:289-300)
+LEAF_SIZE = {-2: 40, -1: 50, 0: 80, 1: 160, 2: 400, 3: 800, 4: 1200, 5: 1400}
+
+
+def tree_work(iprec, source, target=None):
+    """What the tree of a call gives the far field to do, so that a test can say
+    which kernels its inputs reach: levels, leaves with sources at level 2 and
+    below (P2M), pairs of lists 2 to 4 whose source box has sources (M2L, M2P,
+    P2L), and the number of children of each box at level 2 and below that has
+    any (M2M, L2L)."""
+    import fmmlib3d_amd as F
+    ier, box, _, _, lists, nlev, _, _ = F.d3tstrcr(source, target, LEAF_SIZE[iprec])
+    assert ier == 0
+    level, nsrc, kids = box[:, 0], box[:, 14], (box[:, 5:13] > 0).sum(1)
+    deep = level >= 2
+    pairs = [sum(int((nsrc[np.array(l, int) - 1] > 0).sum()) for l in lists[k] if l) for k in (1, 2, 3)]
+    return {"levels": nlev, "p2m": int((deep & (kids == 0) & (nsrc > 0)).sum()), "list2": pairs[0], "list3": pairs[1],
+            "list4": pairs[2], "children": kids[deep & (kids > 0)], "children_level2": kids[(level == 2) & (kids > 0)]}
