@@ -24,8 +24,9 @@ namespace fmm3d {
 // At the end the sums go to LDS, the parts of a block added in order.
 //
 // A step is 5 FP64 operations and 2 products of 19 cycles for 64 (source,
-// column) values, of which 72% are used at order 39 (blocks of 41, 25 and 9
-// steps).  400,000 clustered points, order 39: P2L 28.1 -> 7.4 ms, P2M 2.6 ->
+// column) values; a walk ends at a multiple of four.  At order 39 71% of them are
+// used in P2M (820 entries, blocks of 40, 24 and 8 steps), 64% in P2L (861; 44,
+// 28 and 12).  400,000 clustered points, order 39: P2L 28.1 -> 7.4 ms, P2M 2.6 ->
 // 0.8 ms (with the tables in LDS, k_form2: 12.9 and 1.1 ms).  Dipoles take two
 // operands of weights: with both in one wave (one wave per SIMD) 200,000 +
 // 180,000 points at order 26 took 4.8 ms for P2L but 0.70 for P2M (k_form2: 5.6
