@@ -253,9 +253,8 @@ std::shared_ptr<const Gaunt> gaunt_for(int pmax) {
 std::shared_ptr<const HostTables> geometry_for(int p) {
   constexpr size_t kKept = 4;
   static std::mutex mu;
-  static std::vector<std::shared_ptr<const HostTables>> kept;  // most recent last
-  {
-    std::lock_guard<std::mutex> lk(mu);
+  static std::vector<std::shared_ptr<const HostTables>> kept;  // most recent last, one of each order
+  auto find = [&]() -> std::shared_ptr<const HostTables> {
     for (size_t i = 0; i < kept.size(); i++)
       if (kept[i]->p == p) {
         auto g = kept[i];
@@ -263,10 +262,18 @@ std::shared_ptr<const HostTables> geometry_for(int p) {
         kept.push_back(g);
         return g;
       }
+    return nullptr;
+  };
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    if (auto g = find()) return g;
   }
   auto g = std::make_shared<HostTables>();
   build_geometry_tables(p, *g);
   std::lock_guard<std::mutex> lk(mu);
+  // another thread may have built the same order meanwhile: with two of one
+  // order kept, calls would get them in turn and upload their tables each time
+  if (auto other = find()) return other;
   if (kept.size() >= kKept) kept.erase(kept.begin());
   kept.push_back(g);
   return g;

@@ -10,6 +10,8 @@
 #include <cstdlib>
 #include <cstdint>
 #include <algorithm>
+#include <memory>
+#include <thread>
 #include <vector>
 
 #include "helm_tables.hpp"
@@ -184,8 +186,21 @@ static void check_coax(const HelmHostTables& H) {
   for (char c : tn) CHECK(c == 1);
 }
 
+// tables asked for by several threads at once (the request server's workers)
+// are one object, also afterwards
+static void check_kept_tables() {
+  for (int p : {20, 21}) {
+    std::shared_ptr<const HostTables> got[4];
+    std::vector<std::thread> th;
+    for (int t = 0; t < 4; t++) th.emplace_back([&, t] { got[t] = geometry_for(p); });
+    for (auto& t : th) t.join();
+    for (int k = 0; k < 8; k++) CHECK(geometry_for(p) == got[k % 4]);
+  }
+}
+
 int main() {
   check_launch_pieces();
+  check_kept_tables();
   const int cases[][3] = {  // ns, nt, dist
       {20000, 5000, 0}, {30000, 0, 1}, {25000, 2000, 2}, {12000, 3000, 3}, {3000, 100, 4}, {1, 0, 0}, {50, 50, 1}};
   const int nboxes[] = {40, 80, 160, 400};
