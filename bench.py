@@ -54,12 +54,13 @@ FLOPS_PER_PAIR = 65            # charge+dipole, pot+fld, rsqrt counted as 2
 # WRITE_SIZE runs calibrated against a 1 GiB device copy
 # (profiles/m2l_p2p_counters_lap1M.md): 2 x FETCH KiB + WRITE KiB.
 P2P_TRAFFIC_BYTES = {"fp64": (2 * 3202000 + 126100) * 1024, "fp32": (2 * 927100 + 343700) * 1024}
-# VALU lane instructions per pair in k_p2p on this workload, from rocprofv3
-# SQ_INSTS_VALU (wave64 instructions x 64 / pairs; profiles/m2l_p2p_counters_lap1M.md).
-# A wave64 VALU instruction occupies its SIMD for 4 cycles; the chip has
-# 256 CUs x 4 SIMDs at 2.4 GHz, so the issue-time ceiling of a launch is
-# pairs x this / 64 x 4 / (1024 x 2.4e9) seconds.
-P2P_VALU_INSTR_PER_PAIR = {"fp64": 43.4, "fp32": 44.4}
+# SIMD cycles that the VALU instructions of k_p2p need per 64 pairs at least, on
+# this workload.  The loop has 38 FP64 instructions of 4 cycles and a reciprocal
+# root of 16 per wave of pairs in FP64; with FP32 pair arithmetic 6 FP64 ones, 4
+# conversions (4 cycles), a root (8) and 27.5 FP32 ones (2).  SQ_INSTS_VALU
+# (profiles/m2l_p2p_counters_lap1M.md) counts 43.4 and 44.4 in all; those outside
+# the loop are taken as 2 cycles each.  256 CUs x 4 SIMDs at the nominal 2.4 GHz.
+P2P_ISSUE_CYCLES = {"fp64": 38 * 4 + 16 + 4.4 * 2, "fp32": 10 * 4 + 8 + 27.5 * 2 + 5.9 * 2}
 SIMD_CYCLES_PER_S = 1024 * 2.4e9
 
 
@@ -576,7 +577,8 @@ def main():
         del os.environ["FMM3D_NEAR_STREAM"]
     p2p_alone_ms = float(np.mean([s_["p2p"] for s_ in st_alone]))
     achieved_alone = flops / (p2p_alone_ms * 1e-3) / 1e12
-    issue_s = pairs * P2P_VALU_INSTR_PER_PAIR["fp64" if best == "fp64" else "fp32"] / 64 * 4 / SIMD_CYCLES_PER_S
+    issue_cycles = P2P_ISSUE_CYCLES["fp64" if best == "fp64" else "fp32"]
+    issue_s = pairs / 64 * issue_cycles / SIMD_CYCLES_PER_S
     dropin = dropin_leg(F, prec_of[best], src, q, ds, dv, trg)
     print("# drop-in (host arrays): %.1f ms/call, %.3e targets/s" % (dropin["ms_per_call"], dropin["targets_per_s"]),
           file=sys.stderr, flush=True)
@@ -635,10 +637,10 @@ def main():
                              "kernels and is timed with HIP events on that stream; *_alone: the same launch "
                              "with the near field on the caller's stream (FMM3D_NEAR_STREAM=0), 2 extra steps. "
                              "algorithmic flops = %d pairs x %d. valu_issue_frac: time the launch's VALU "
-                             "instructions (%.1f per pair, rocprofv3 SQ_INSTS_VALU) need at one wave64 instruction "
-                             "per 4 cycles per SIMD, 1024 SIMDs, 2.4 GHz, over the measured time; FP32 peak "
-                             "counts packed FP32, which this build does not emit"
-                             % (pairs, FLOPS_PER_PAIR, P2P_VALU_INSTR_PER_PAIR["fp64" if best == "fp64" else "fp32"])},
+                             "instructions need at their issue rates (%.0f SIMD cycles per 64 pairs, 1024 SIMDs, "
+                             "2.4 GHz), over the measured time; FP32 peak counts packed FP32, which this build "
+                             "does not emit"
+                             % (pairs, FLOPS_PER_PAIR, issue_cycles)},
         "cpu_baseline": cpu,
         "dropin_host_arrays": dropin,
         "modes": {k: {kk: vv for kk, vv in v.items() if kk != "latencies_ms"} for k, v in modes.items()},
