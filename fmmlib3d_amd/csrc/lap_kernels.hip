@@ -365,12 +365,14 @@ __global__ __launch_bounds__(256) void k_form2(DevPlan P, const double* __restri
 // the order of the walk (column a, then n = a..pd); that recurrence's factors
 // for degree n + 1 stand once, in the same order, ahead of the packs (with them
 // in the entries and the columns padded to an even count the packs took 17%
-// more at order 26, 50% at order 2, and a fixed workspace held fewer points).
-// The walk reads both with scalar loads, one entry ahead, and pays 16 FMAs and
-// the recurrence's 5 operations per entry and point (32 and 9 before, the
-// harmonics normalised and c+ h, c- conj(h) taken apart).  VALU bound: 400,000
-// clustered points at order 39, M2P 11.4 -> 8.2 ms; 200,000 + 180,000 at order
-// 26 7.8 -> 5.7 ms; 1M + 1M uniform, L2P 1.59 -> 1.22 ms (FP32 1.22 -> 0.74 ms).
+// more at order 26, 50% at order 2, a fixed workspace held fewer points, and the
+// scalar loads straddled their 64-byte lines).  The walk reads both with scalar
+// loads, one entry ahead, and pays 16 FMAs and the recurrence's 5 operations per
+// entry and point (32 and 9 before, the harmonics normalised and c+ h, c- conj(h)
+// taken apart).  VALU bound: 400,000 clustered points at order 39, M2P 11.4 ms
+// with normalised harmonics, 8.2 with the factors in the entries, 5.8 so;
+// 200,000 + 180,000 at order 26 7.8, 5.7 and 4.1 ms; 1M + 1M uniform, L2P 1.59,
+// 1.22 and 1.06 ms (FP32 1.22, 0.74 and 0.70).
 // ---------------------------------------------------------------------------
 constexpr int kPackEntry = 16;
 __host__ __device__ inline int pack_entries(int pd) { return (pd + 1) * (pd + 2) / 2; }

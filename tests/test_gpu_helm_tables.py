@@ -9,10 +9,10 @@ none.  Bar as for the other comparisons with the oracle's FMM, which truncates
 alike.
 
 By order: the grouped M2L with complex shift tables (k_hm2l_grp) at each launch
-shape, eight, four, two and one group at a time, one and two work items per
-thread, and the order beyond it that runs one pair at a time.  The terms of a
-shift cancel the more the larger the box is in wavelengths; above order 40 (100
-to 180 radians across) ten times the bar."""
+shape, eight, four and one group at a time, one and two work items per thread,
+and the order beyond it that runs one pair at a time.  The terms of a shift
+cancel the more the larger the box is in wavelengths; above order 42 (150 and
+180 radians across) ten times the bar."""
 import ctypes
 
 import numpy as np

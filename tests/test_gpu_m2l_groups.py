@@ -1,9 +1,9 @@
 """The grouped M2L (k_m2l_grp) against the M2L one pair at a time (k_m2l,
 FMM3D_M2L_ROTATION=pairs) at the orders of iprec -2 .. 4 (2, 5, 9, 14, 26, 39
-and 51), hence at every launch shape: eight, four, two and one group at a time,
-one and two work items per thread, four, two and one members per group.  (Order
-64 of iprec 5 has more work items than a workgroup takes and runs one pair at a
-time itself.)  The two sum the same terms in another order: a local coefficient
+and 51), hence at every launch shape they take: eight, four and one group at a
+time, one and two work items per thread, four, two and one members per group.
+(Order 64 of iprec 5 has more work items than a workgroup takes and runs one
+pair at a time itself.)  The two sum the same terms in another order: a local coefficient
 is a sum of at most 189 translations of about p products, so FP64 results agree
 to 1e-12 and FP32 ones to 1e-5 of their norm.  The switch is read once per
 process, so the pairs run in a child."""
