@@ -185,6 +185,37 @@ void launch_hp2p(const DevPlan& P, const int* items, int n, int kind, double kre
 #undef HCASE
 }
 
+// LDS of k_heval3 (L2P) at degree pd
+size_t helm_lds_eval(int pd) { return sizeof(double) * 2 * 64 * (size_t)(pd + 2); }
+
+// LDS of the kernels at expansion order p; whether all of it fits
+struct HelmLds {
+  bool fits = false, form2 = false, m2l = false;
+  size_t form = 0, form2_lds = 0, ps = 0;
+  int ts = 0, region2 = 0;
+};
+HelmLds helm_lds(int p, size_t ldsmax) {
+  HelmLds W;
+  const int K = (p + 1) * (p + 1), Hh = (p + 2) * (p + 3) / 2, Fn = p + 2;
+  const size_t per_src = 2 * (size_t)Hh + 2 * (size_t)Fn + 12;
+  if (sizeof(double) * (4 * (size_t)K + per_src) > ldsmax) return W;
+  const int ts = (int)((ldsmax / sizeof(double) - 4 * (size_t)K) / per_src);
+  W.ts = std::max(1, std::min(32, ts));
+  W.form = sizeof(double) * (4 * (size_t)K + (size_t)W.ts * per_src);
+  // per-thread-sum P2M/P2L: half tables up to degree p+1 held by 256
+  // threads x kHFormItems entries, outputs by 256 x kHFormOut
+  // (LDS: 64 KB, or what holds 4 sources at order p+1; the kernel picks
+  // its tile from what is left after the factor head)
+  W.form2 = Hh <= 256 * kHFormItems && K <= 256 * kHFormOut;
+  W.form2_lds = std::max<size_t>((size_t)64 * 1024,
+                                 hform2_fac_bytes(p) + sizeof(double) * (2 * ((size_t)Hh + Fn) + 8) * 4);
+  W.region2 = (int)((W.form2_lds - hform2_fac_bytes(p)) / sizeof(double));
+  W.ps = sizeof(double) * 4 * (size_t)K;
+  W.m2l = sizeof(double) * 6 * (size_t)K <= ldsmax;
+  W.fits = !(W.form2 && W.form2_lds > ldsmax) && W.ps <= ldsmax && helm_lds_eval(p + 1) <= ldsmax;
+  return W;
+}
+
 }  // namespace
 
 // TN: near-field pair arithmetic (double, or float with FP64 offsets and accumulation)
@@ -224,31 +255,13 @@ int helm_solve(Context& ctx, const LapCall& c) {
   if (!ctx.helm_tables) ctx.helm_tables = std::make_shared<HelmCache>();
   HelmCache* HC = static_cast<HelmCache*>(ctx.helm_tables.get());
   const bool held = HC->valid && HC->H.zk == zk && HC->H.size == tree.size && HC->H.nlev == tree.nlev && HC->H.eps == eps;
-  HelmHostTables plan;
-  if (!held && !plan_helm_tables(zk, tree.size, tree.nlev, eps, plan)) return 16;
-  const int pmax = held ? HC->H.pmax : plan.pmax, K = (pmax + 1) * (pmax + 1);
-  // LDS budgets of the kernels at this order
   const size_t ldsmax = max_lds_bytes(ctx);
-  const int Hh = (pmax + 2) * (pmax + 3) / 2, Fn = pmax + 2;
-  const size_t per_src = 2 * (size_t)Hh + 2 * (size_t)Fn + 12;
-  if (sizeof(double) * (4 * (size_t)K + per_src) > ldsmax) return 16;
-  int ts = (int)((ldsmax / sizeof(double) - 4 * (size_t)K) / per_src);
-  ts = std::max(1, std::min(32, ts));
-  const size_t lds_form = sizeof(double) * (4 * (size_t)K + (size_t)ts * per_src);
-  // per-thread-sum P2M/P2L: half tables up to degree pmax+1 held by 256
-  // threads x kHFormItems entries, outputs by 256 x kHFormOut
-  // (LDS: 64 KB, or what holds 4 sources at order pmax+1; the kernel picks
-  // its tile from what is left after the factor head)
-  const bool form2 = Hh <= 256 * kHFormItems && K <= 256 * kHFormOut;
-  const size_t lds_form2 = std::max<size_t>((size_t)64 * 1024,
-                                            hform2_fac_bytes(pmax) + sizeof(double) * (2 * ((size_t)Hh + Fn) + 8) * 4);
-  const int region2 = (int)((lds_form2 - hform2_fac_bytes(pmax)) / sizeof(double));
-  if (form2 && lds_form2 > ldsmax) return 16;
-  const size_t lds_ps = sizeof(double) * 4 * (size_t)K;
-  const bool m2l_lds = sizeof(double) * 6 * (size_t)K <= ldsmax;
-  if (lds_ps > ldsmax) return 16;
-  auto lds_eval = [](int pd) { return sizeof(double) * 2 * 64 * (size_t)(pd + 2); };  // k_heval3 (L2P) at degree pd
-  if (lds_eval(pmax + 1) > ldsmax) return 16;
+  int most = kMaxHelmOrder;
+  while (most > 0 && !helm_lds(most, ldsmax).fits) most--;
+  HelmHostTables plan;
+  if (!held && !plan_helm_tables(zk, tree.size, tree.nlev, eps, plan, most)) return 16;
+  const int pmax = held ? HC->H.pmax : plan.pmax, K = (pmax + 1) * (pmax + 1);
+  const HelmLds W = helm_lds(pmax, ldsmax);
   if (!held) helm_upload_tables(ctx, *HC, std::move(plan));
   const HelmHostTables& H = HC->H;
   thread_local Flat FA, FB, FC;  // plan parts: boxes, near lists, far lists (storage reused)
@@ -375,15 +388,15 @@ int helm_solve(Context& ctx, const LapCall& c) {
       PF.isrc = tri_rng;
       PF.nsrc = tri_rng + nb;
     }
-    if (!form2) {
-      hipLaunchKernelGGL((k_hform<IR>), dim3(nbx), dim3(256), lds_form, s, PF, Hd, fac, fpos, fstr,
-                         f.ifcharge, f.ifdipole, ts, out);
+    if (!W.form2) {
+      hipLaunchKernelGGL((k_hform<IR>), dim3(nbx), dim3(256), W.form, s, PF, Hd, fac, fpos, fstr,
+                         f.ifcharge, f.ifdipole, W.ts, out);
     } else if (f.ifcharge && f.ifdipole) {
-      hipLaunchKernelGGL((k_hform2<IR, true, true>), dim3(nbx), dim3(256), lds_form2, s, PF, Hd, fac, fpos, fstr, region2, out);
+      hipLaunchKernelGGL((k_hform2<IR, true, true>), dim3(nbx), dim3(256), W.form2_lds, s, PF, Hd, fac, fpos, fstr, W.region2, out);
     } else if (f.ifcharge) {
-      hipLaunchKernelGGL((k_hform2<IR, true, false>), dim3(nbx), dim3(256), lds_form2, s, PF, Hd, fac, fpos, fstr, region2, out);
+      hipLaunchKernelGGL((k_hform2<IR, true, false>), dim3(nbx), dim3(256), W.form2_lds, s, PF, Hd, fac, fpos, fstr, W.region2, out);
     } else if (f.ifdipole) {
-      hipLaunchKernelGGL((k_hform2<IR, false, true>), dim3(nbx), dim3(256), lds_form2, s, PF, Hd, fac, fpos, fstr, region2, out);
+      hipLaunchKernelGGL((k_hform2<IR, false, true>), dim3(nbx), dim3(256), W.form2_lds, s, PF, Hd, fac, fpos, fstr, W.region2, out);
     }
   };
   // STEP 1: P2M (hfmm3dpart.f:681-757)
@@ -391,7 +404,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
   tm.mark(2);
   // STEP 3: M2M, bottom-up
   for (size_t g = 0; g < O.m2m_groups.size(); g++) {
-    hipLaunchKernelGGL(k_hm2m, dim3(O.m2m_groups[g].second, 8), dim3(256), lds_ps, s, P, Tb, Hd,
+    hipLaunchKernelGGL(k_hm2m, dim3(O.m2m_groups[g].second, 8), dim3(256), W.ps, s, P, Tb, Hd,
                        O.m2m_groups[g].first, HC->m2m_base + O.m2m_group_level[g], mp, lo);
     hipLaunchKernelGGL((k_child_sum<double>), dim3(O.m2m_groups[g].second), dim3(256), 0, s, P,
                        O.m2m_groups[g].first, mp, lo);
@@ -461,15 +474,15 @@ int helm_solve(Context& ctx, const LapCall& c) {
       else if (G.items == 1) HM2L_GRP(512, 1);
       else HM2L_GRP(512, 2);
 #undef HM2L_GRP
-    } else if (m2l_lds)
+    } else if (W.m2l)
       hipLaunchKernelGGL((k_hm2l<true>), dim3(P.n_m2l), dim3(256), sizeof(double) * 6 * (size_t)K, s, P, Tb, Hd, mp, lo);
     else
-      hipLaunchKernelGGL((k_hm2l<false>), dim3(P.n_m2l), dim3(256), lds_ps, s, P, Tb, Hd, mp, lo);
+      hipLaunchKernelGGL((k_hm2l<false>), dim3(P.n_m2l), dim3(256), W.ps, s, P, Tb, Hd, mp, lo);
   }
   tm.mark(6);
   // STEP 5: L2L, top-down
   for (size_t g = 0; g < O.l2l_groups.size(); g++)
-    hipLaunchKernelGGL(k_hl2l, dim3(O.l2l_groups[g].second, 8), dim3(256), lds_ps, s, P, Tb, Hd,
+    hipLaunchKernelGGL(k_hl2l, dim3(O.l2l_groups[g].second, 8), dim3(256), W.ps, s, P, Tb, Hd,
                        O.l2l_groups[g].first, HC->l2l_base + O.l2l_group_level[g], lo);
   tm.mark(7);
   // STEP 7: L2P and STEP 6: M2P (list 3), from packed expansions
@@ -549,7 +562,7 @@ int helm_solve(Context& ctx, const LapCall& c) {
       double* pack = (double*)ctx.arena.get("hpack_l", sizeof(double) * 16 * (size_t)std::max(tot_l, 1));
       hipLaunchKernelGGL((k_hpack<false>), dim3((unsigned)pk_l.size()), dim3(256), 0, s, P, Hd, fac, lo, dh + o_pl,
                          dh + o_ol, grad, pack);
-      hipLaunchKernelGGL((k_heval3<false>), dim3((unsigned)(it_l.size() / 3)), dim3(64), lds_eval(pdmax), s, P, Hd, fac, pack,
+      hipLaunchKernelGGL((k_heval3<false>), dim3((unsigned)(it_l.size() / 3)), dim3(64), helm_lds_eval(pdmax), s, P, Hd, fac, pack,
                          dh + o_sl, dh + o_il, grad, spos, tpos, f.ifpot, f.iffld, f.ifpottarg, f.iffldtarg, pot_s,
                          fld_s, pot_t, fld_t, (double*)nullptr);
     }

@@ -315,7 +315,7 @@ void add_coax(HelmHostTables& H, int mode, int neg, double d, double sc_in, doub
 
 }  // namespace
 
-bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H) {
+bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H, int most) {
   H = HelmHostTables();
   H.zk = zk;
   H.size = size;
@@ -336,7 +336,7 @@ bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables
     }
   }
   H.pmax = pmax;
-  if (pmax > kMaxHelmOrder) return false;
+  if (pmax > most) return false;
   H.geo = geometry_for(pmax);
   const int nd = H.geo->ndist;
   H.ptrunc.assign((size_t)(nlev + 1) * 343, 0);

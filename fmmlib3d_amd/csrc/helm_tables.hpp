@@ -73,14 +73,13 @@ std::shared_ptr<const HostTables> geometry_for(int p);
 
 // The orders, list-2 tables, operator layout and series the Helmholtz FMM
 // needs for a tree of root side `size` and depth `nlev`; the blocks are
-// computed from the series on the device (k_coax).  Returns false when an
-// order exceeds what the device kernels support (kMaxHelmOrder).
-bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H);
+// computed from the series on the device (k_coax).  Returns false, with nothing
+// built, when an order exceeds `most` (what the device's LDS holds).
+constexpr int kMaxHelmOrder = 120;
+bool plan_helm_tables(cplx zk, double size, int nlev, double eps, HelmHostTables& H, int most = kMaxHelmOrder);
 // where the 4x4 tiles of order am of M2L table t start (k_coax), off[t * (pmax + 1)
 // + am]; returns their size in doubles
 long coax_tile_offsets(const HelmHostTables& H, std::vector<long>& off);
-
-constexpr int kMaxHelmOrder = 120;
 
 // What k_coax computes and where, also compiled for the host so that the
 // sanitizers see it.

@@ -298,6 +298,10 @@ int main() {
       HelmHostTables H;
       const bool ok = plan_helm_tables(cplx(z[0], z[1]), 1.0, 5, e, H);
       if (!ok) continue;  // an order beyond kMaxHelmOrder: reported, not built
+      HelmHostTables R;
+      CHECK(!plan_helm_tables(cplx(z[0], z[1]), 1.0, 5, e, R, H.pmax - 1));
+      CHECK(!R.geo && R.jobs.empty() && R.pmax == H.pmax);
+      CHECK(plan_helm_tables(cplx(z[0], z[1]), 1.0, 5, e, R, H.pmax));
       CHECK((int)H.plev.size() == 6);
       for (int l = 2; l <= 5; l++) CHECK(H.plev[l] > 0 && H.plev[l] <= H.pmax);
       for (auto& d : H.m2l) CHECK(d.base >= 0 && d.base <= H.nz);
