@@ -110,7 +110,8 @@ inline void build_plan_boxes(const Octree& t, const Flags& f, Flat& F, PlanOffse
 // box's items go into one workgroup (kItemWaves items) when they fit, so
 // its waves share the source data in cache: the list is padded with null
 // items (box -1, skipped by the kernels) up to the next workgroup when the
-// box's items would straddle one.
+// box's items would straddle one.  (The Laplace k_p2p takes one item per
+// workgroup; a null item's ends at once.)
 inline void push_items(std::vector<int>& it, int b, int kind, int npts) {
   const int c = (npts + kP2PBlock - 1) / kP2PBlock;
   if (c == 0) return;
